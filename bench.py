@@ -387,6 +387,12 @@ def profile_run(fa, prob, forest, q0, aux, dt, tiles, time_sync, dt_scale=None):
     print("calibration copies: 3 x %d bytes" % COPY_BYTES, flush=True)
 
 
+def is_step(kernel):
+    """Whether a kernel name is the patch update (strips, or tiles for solvers
+    with many wave components)."""
+    return "step_strips" in kernel or "step_tiles" in kernel
+
+
 def _profiled_rows(rows):
     """The dispatches of the profiled steps: those that start after the last
     regrid of the run that grew the forest (all of them for the t = 0 forest)."""
@@ -443,7 +449,7 @@ def pmc_summary(fetch_dir, write_dir, cells):
     lines = ["calibration: 3 copies of %d bytes; FETCH_SIZE factor %.3f, WRITE_SIZE factor %.3f"
              % (COPY_BYTES, f_fetch, f_write)]
     for k in sorted(fetch):
-        if not any(n in k for n in ("step_tiles", "ghost_", "physbc", "time_sync")):
+        if not is_step(k) and not any(n in k for n in ("ghost_", "physbc", "time_sync")):
             continue
         fk = sum(fetch[k]) / len(fetch[k])
         wk = sum(write.get(k, [0.0])) / max(len(write.get(k, [])), 1)
@@ -472,7 +478,7 @@ def valu_summary(pmc_dir, cells):
     span = {}
     for r in _profiled_rows(_csv_rows(pmc_dir, "counter_collection.csv")):
         k = r["Kernel_Name"]
-        if "step_tiles" not in k:
+        if not is_step(k):
             continue
         per.setdefault(k, {}).setdefault(r["Counter_Name"], []).append(float(r["Counter_Value"]))
         span.setdefault(k, {})[r["Dispatch_Id"]] = int(r["End_Timestamp"]) - int(r["Start_Timestamp"])
@@ -502,7 +508,7 @@ def counter_summary(pmc_dir, cells):
     per = {}
     for r in _profiled_rows(_csv_rows(pmc_dir, "counter_collection.csv")):
         k = r["Kernel_Name"]
-        if "step_tiles" in k:
+        if is_step(k):
             per.setdefault(k, {}).setdefault(r["Counter_Name"], []).append(float(r["Counter_Value"]))
     lines = []
     for k in sorted(per):
@@ -552,7 +558,7 @@ def committed_traffic(workload, kernel_tag, cells):
     """HBM bytes per launch of the step kernel: the measured bytes per cell
     update of the committed counter summary of this workload, times the cells
     of this launch (None if there is no summary for this kernel)."""
-    path = os.path.join(ROOT, "profiles", "step_tiles_%s_pmc.txt" % workload)
+    path = os.path.join(ROOT, "profiles", "step_strips_%s_pmc.txt" % workload)
     if not os.path.exists(path):
         return None
     for line in open(path):
@@ -764,11 +770,11 @@ def main():
 
     def roofline(r, rtype):
         achieved = B * cells / (r["kernel_ms"] * 1e-3) / 1e9
-        traffic = committed_traffic(workload, "%s, %d," % (rtype, r["tile"]), cells)
+        traffic = committed_traffic(workload, ">, %s," % rtype, cells)
         return {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": None if traffic is None else round(traffic),
-                "kernel": "step_tiles", "kernel_avg_ms": round(r["kernel_ms"], 5),
+                "kernel": "step_strips", "kernel_avg_ms": round(r["kernel_ms"], 5),
                 "bytes_per_cell_update": round(B, 4), "cell_updates_per_launch": cells,
                 "copy_peak": round(copy_peak, 1), "frac_of_copy_peak": round(achieved / copy_peak, 4)}
 

@@ -1,8 +1,8 @@
 // C ABI of the batched patch-update backend (declared in include/hipclaw.h).
 //
 // Device memory model: one allocation per slab, sized once for max_patches.
-// q lives in two slabs (ping-pong) unless a single tile covers a patch, in
-// which case the step is done in place.  All launches go to one
+// q lives in two slabs (ping-pong); where a single tile covers a patch and
+// memory is short, in one, and the step is done in place.  All launches go to one
 // non-blocking stream of default priority owned by the state.
 #include <hip/hip_runtime.h>
 
@@ -78,10 +78,22 @@ struct SyncProgram {
     bool set = false;         // installed since the last regrid
 };
 
+constexpr size_t CFL_BYTES = sizeof(unsigned long long) * hipclaw::CFL_WORDS * hipclaw::CFL_STRIDE;
+
+// The Courant number in the CFL words of a step (StepArgs::cfl), on the host.
+static double largest_cfl(const unsigned long long* words) {
+    unsigned long long bits = 0;
+    for (int k = 0; k < hipclaw::CFL_WORDS; k++) bits = std::max(bits, words[k * hipclaw::CFL_STRIDE]);
+    double v;
+    std::memcpy(&v, &bits, sizeof(v));
+    return v;
+}
+
 struct hipclaw_state {
     hipclaw_config_t cfg;
     int tile = 16, ntx = 1, nty = 1;
-    bool inplace = false;
+    bool covers = false;         // one tile covers a patch
+    bool inplace = false;        // one slab (covers, and no memory for the second)
     bool conservative = false;   // the solver has the FP32-bulk flux form
     int max_patches = 0, npatch = 0;
     long long pstride = 0, astride = 0;
@@ -180,7 +192,7 @@ struct hipclaw_state {
 // process; its device address is looked up once per device (scratch_ptr) and
 // only that address is passed to kernels, copies and fills.
 namespace {
-constexpr size_t NOALLOC_CFL_BYTES = 256;
+constexpr size_t NOALLOC_CFL_BYTES = CFL_BYTES;
 constexpr size_t NOALLOC_SCRATCH_BYTES =
     NOALLOC_CFL_BYTES + sizeof(int) * (size_t) HIPCLAW_NOALLOC_MAX_SLOTS;
 constexpr int NOALLOC_MAX_DEVICES = 64;
@@ -422,11 +434,9 @@ static bool solver_tile_ok(int solver, int precision, int tile) {
 }
 
 static int solver_default_waves(int solver, int precision, int tile) {
-    if (solver >= 0 && solver <= 2)
-        return precision == HIPCLAW_FP64 ? hipclaw::default_waves_fp64(solver, tile)
-                                         : hipclaw::default_waves_fp32(solver, tile);
-    return tile != 16 ? 0 : precision == HIPCLAW_FP64 ? hipclaw::default_waves_t16<double>()
-                                                      : hipclaw::default_waves_t16<float>();
+    SolverShape sh;
+    if (!solver_shape(solver, &sh)) return 0;
+    return hipclaw::default_waves(sh.meqn * sh.mwaves <= 16, precision == HIPCLAW_FP64, tile);
 }
 
 static int launch_solver_step(int solver, int precision, int tile, int waves,
@@ -501,6 +511,23 @@ static int check_config(const hipclaw_config_t* cfg, int* tile_out) {
     return HIPCLAW_OK;
 }
 
+// The second slab of a state whose tile covers a patch.  Its steps could run in
+// place; with two slabs its patches may be cut into strips of any height, and
+// the update reads same-size ghost strips from the neighbours instead of having
+// them copied first.  Without memory to spare (as much again stays free) the
+// state keeps one slab.
+static void second_slab(hipclaw_state_t* s) {
+    const size_t bytes = sizeof(double) * (size_t) s->pstride * (size_t) s->max_patches;
+    size_t free_bytes = 0, total = 0;
+    s->inplace = true;
+    if (hipMemGetInfo(&free_bytes, &total) == hipSuccess && free_bytes / 2 >= bytes &&
+        hipMalloc((void**) &s->q[1], bytes) == hipSuccess)
+        s->inplace = false;
+    else
+        (void) hipGetLastError();
+    if (s->inplace) s->q[1] = nullptr;
+}
+
 int hipclaw_create(const hipclaw_config_t* cfg, int max_patches, hipclaw_state_t** out) {
     if (!cfg || !out || max_patches <= 0) return fail(HIPCLAW_EINVAL, "hipclaw_create: bad arguments%s");
     *out = nullptr;
@@ -517,7 +544,7 @@ int hipclaw_create(const hipclaw_config_t* cfg, int max_patches, hipclaw_state_t
     }
     s->ntx = tiles_along(cfg->mx, tile);
     s->nty = tiles_along(cfg->my, tile);
-    s->inplace = (s->ntx == 1 && s->nty == 1);
+    s->covers = s->ntx == 1 && s->nty == 1;
     s->max_patches = max_patches;
     // measured on MI355X: per-destination groups pay off once a patch's ghost
     // strips are long (mx >= 32); shorter ones keep one launch per phase
@@ -535,13 +562,13 @@ int hipclaw_create(const hipclaw_config_t* cfg, int max_patches, hipclaw_state_t
     if (hipStreamCreateWithFlags(&s->st, hipStreamNonBlocking) != hipSuccess)
         return cleanup(fail(HIPCLAW_EDEVICE, "hipStreamCreate failed%s"));
     ALLOC(s->q[0], sizeof(double) * s->pstride * max_patches);
-    if (!s->inplace) ALLOC(s->q[1], sizeof(double) * s->pstride * max_patches);
+    if (!s->covers) ALLOC(s->q[1], sizeof(double) * s->pstride * max_patches);
     if (cfg->maux > 0) ALLOC(s->aux, sizeof(double) * s->astride * max_patches);
     ALLOC(s->dxs, sizeof(double) * max_patches);
     ALLOC(s->dys, sizeof(double) * max_patches);
     ALLOC(s->all_slots, sizeof(int) * max_patches);
     ALLOC(s->batch_slots, sizeof(int) * max_patches);
-    ALLOC(s->cfl, sizeof(unsigned long long));
+    ALLOC(s->cfl, CFL_BYTES);
     ALLOC(s->mass_buf, sizeof(double) * 2 * cfg->meqn * (size_t) max_patches);
     if (cfg->subcycle) {
         ALLOC(s->qlast, sizeof(double) * s->pstride * max_patches);
@@ -558,6 +585,7 @@ int hipclaw_create(const hipclaw_config_t* cfg, int max_patches, hipclaw_state_t
             return cleanup(fail(HIPCLAW_EDEVICE, "initial device copies failed%s"));
     }
 #undef ALLOC
+    if (s->covers) second_slab(s);
     std::vector<int> iota(max_patches);
     for (int p = 0; p < max_patches; p++) iota[p] = p;
     if (hipMemcpy(s->all_slots, iota.data(), sizeof(int) * max_patches, hipMemcpyHostToDevice) != hipSuccess ||
@@ -1490,15 +1518,16 @@ static bool tile_allowed(const hipclaw_state_t* s, int t) {
 
 static int set_tile(hipclaw_state_t* s, int t) {
     const int ntx = tiles_along(s->cfg.mx, t), nty = tiles_along(s->cfg.my, t);
-    const bool inplace = ntx == 1 && nty == 1;
-    if (!inplace && !s->q[1]) {   // a ping-pong tile needs the second slab
+    const bool covers = ntx == 1 && nty == 1;
+    if (!covers && !s->q[1]) {   // a ping-pong tile needs the second slab
         if (hipMalloc((void**) &s->q[1], sizeof(double) * s->pstride * (size_t) s->max_patches) != hipSuccess)
             return fail(HIPCLAW_ENOMEM, "hipMalloc of the second slab failed%s");
     }
     s->tile = t;
     s->ntx = ntx;
     s->nty = nty;
-    s->inplace = inplace;
+    s->covers = covers;
+    s->inplace = !s->q[1];
     // a captured graph holds launches of the old tile
     if (s->gexec) { hipGraphExecDestroy(s->gexec); s->gexec = nullptr; }
     if (s->graph) { hipGraphDestroy(s->graph); s->graph = nullptr; }
@@ -1701,19 +1730,17 @@ static int launch_step(hipclaw_state_t* s, const hipclaw::StepArgs& a, hipEvent_
                        hipEvent_t ev1 = nullptr) {
     const hipclaw::StepLaunch L(s->st, ev0, ev1);
     int e = launch_solver_step(s->cfg.solver, s->cfg.precision, s->tile, s->waves, a, L);
-    if (e) return hipfail((hipError_t) e, "step_tiles launch");
+    if (e) return hipfail((hipError_t) e, "step launch");
     return HIPCLAW_OK;
 }
 
 static double read_cfl(hipclaw_state_t* s, int* rc) {
-    unsigned long long bits = 0;
-    hipError_t e = hipMemcpyAsync(&bits, s->cfl, sizeof(bits), hipMemcpyDeviceToHost, s->st);
+    unsigned long long words[CFL_BYTES / sizeof(unsigned long long)];
+    hipError_t e = hipMemcpyAsync(words, s->cfl, CFL_BYTES, hipMemcpyDeviceToHost, s->st);
     if (e == hipSuccess) e = hipStreamSynchronize(s->st);
     if (e != hipSuccess) { *rc = hipfail(e, "reading the CFL number"); return 0.0; }
-    double v;
-    std::memcpy(&v, &bits, sizeof(v));
     *rc = HIPCLAW_OK;
-    return v;
+    return largest_cfl(words);
 }
 
 int hipclaw_step_batch(hipclaw_state_t* s, const int* slots, int nslots, double t, double dt,
@@ -1727,16 +1754,16 @@ int hipclaw_step_batch(hipclaw_state_t* s, const int* slots, int nslots, double 
     if (maxcfl) *maxcfl = 0.0;
     if (nslots == 0) return HIPCLAW_OK;
     HIP_TRY(hipMemcpyAsync(s->batch_slots, slots, sizeof(int) * nslots, hipMemcpyHostToDevice, s->st));
-    if (int e = hipclaw::launch_reset_scalar(s->cfl, s->st)) return hipfail((hipError_t) e, "reset");
+    if (int e = hipclaw::launch_reset_cfl(s->cfl, s->st)) return hipfail((hipError_t) e, "reset");
     if (s->qlast) {  // fclaw2d_clawpatch_save_current_step before every update
         int e = hipclaw::launch_copy_patches(s->q[s->cur], s->qlast, s->batch_slots, nslots,
                                              s->pstride, s->st);
         if (e) return hipfail((hipError_t) e, "copy_patches launch");
     }
     double* src = s->q[s->cur];
-    double* dst = s->inplace ? src : s->q[1 - s->cur];
+    double* dst = s->covers ? src : s->q[1 - s->cur];
     if (int rc = launch_step(s, step_args(s, src, dst, s->batch_slots, nslots, dt))) return rc;
-    if (!s->inplace) {
+    if (!s->covers) {
         int e = hipclaw::launch_copy_interior(dst, src, s->batch_slots, nslots, s->pstride,
                                               s->cfg.mx, s->cfg.my, s->cfg.mbc, s->cfg.meqn, s->st);
         if (e) return hipfail((hipError_t) e, "copy_interior launch");
@@ -1777,7 +1804,7 @@ int hipclaw_step_batch_noalloc(const hipclaw_config_t* cfg, int npatch, const do
     int* dslots = reinterpret_cast<int*>(base + NOALLOC_CFL_BYTES);
     hipStream_t st = static_cast<hipStream_t>(stream);
     HIP_TRY(hipMemcpyAsync(dslots, slots, sizeof(int) * (size_t) nslots, hipMemcpyHostToDevice, st));
-    if (int e = hipclaw::launch_reset_scalar(dcfl, st)) return hipfail((hipError_t) e, "reset");
+    if (int e = hipclaw::launch_reset_cfl(dcfl, st)) return hipfail((hipError_t) e, "reset");
     hipclaw::StepArgs a;
     a.qsrc = q_in;
     a.qdst = q_out;
@@ -1800,13 +1827,11 @@ int hipclaw_step_batch_noalloc(const hipclaw_config_t* cfg, int npatch, const do
     a.dtscale = nullptr;
     const hipclaw::StepLaunch L(st);
     int e = launch_solver_step(cfg->solver, cfg->precision, tile, 0, a, L);
-    if (e) return hipfail((hipError_t) e, "step_tiles launch");
-    unsigned long long bits = 0;
-    HIP_TRY(hipMemcpyAsync(&bits, dcfl, sizeof(bits), hipMemcpyDeviceToHost, st));
+    if (e) return hipfail((hipError_t) e, "step launch");
+    unsigned long long words[CFL_BYTES / sizeof(unsigned long long)];
+    HIP_TRY(hipMemcpyAsync(words, dcfl, CFL_BYTES, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
-    double v;
-    std::memcpy(&v, &bits, sizeof(v));
-    if (maxcfl) *maxcfl = v;
+    if (maxcfl) *maxcfl = largest_cfl(words);
     return HIPCLAW_OK;
 }
 
@@ -1819,7 +1844,7 @@ static int advance_launches(hipclaw_state_t* s, double dt, int nsteps, bool time
             s->kev.push_back(e);
         }
     }
-    if (int e = hipclaw::launch_reset_scalar(s->cfl, s->st)) return hipfail((hipError_t) e, "reset");
+    if (int e = hipclaw::launch_reset_cfl(s->cfl, s->st)) return hipfail((hipError_t) e, "reset");
     if (s->ghost_layout == 2 && s->fused_ok && !s->reg_accumulate) {
         // two launches per step: the update (staging the corrected edge cells of
         // the last synchronisation) and the fused ghost fill + time sync; the
@@ -1927,7 +1952,7 @@ static int subcycle_level(hipclaw_state_t* s, int level, int curr_fine_step, Lev
 
 static int subcycle_launches(hipclaw_state_t* s, double dt, int ncoarse) {
     const int lmin = s->lmin, lmax = s->lmax, nl = lmax - lmin + 1;
-    if (int e = hipclaw::launch_reset_scalar(s->cfl, s->st)) return hipfail((hipError_t) e, "reset");
+    if (int e = hipclaw::launch_reset_cfl(s->cfl, s->st)) return hipfail((hipError_t) e, "reset");
     for (int c = 0; c < ncoarse; c++) {
         LevelCounter tc[HIPCLAW_MAX_PROGRAMS];
         for (int l = 0; l < nl; l++) {   // initialize_timestep_counters (:54-110)
@@ -2070,7 +2095,7 @@ int hipclaw_advance(hipclaw_state_t* s, double dt, int nsteps, double* maxcfl) {
 
 int hipclaw_capture_graph(hipclaw_state_t* s, double dt, int nsteps) {
     if (!s || nsteps <= 0 || !(dt > 0.0)) return fail(HIPCLAW_EINVAL, "hipclaw_capture_graph: bad arguments%s");
-    if (!s->inplace && (nsteps % 2) != 0)
+    if (!s->covers && (nsteps % 2) != 0)
         return fail(HIPCLAW_EINVAL, "ping-pong states need an even number of captured steps%s");
     if (s->gexec) { hipGraphExecDestroy(s->gexec); s->gexec = nullptr; }
     if (s->graph) { hipGraphDestroy(s->graph); s->graph = nullptr; }
@@ -2082,6 +2107,10 @@ int hipclaw_capture_graph(hipclaw_state_t* s, double dt, int nsteps) {
     s->graph_cur = cur0;
     HIP_TRY(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
     int rc = advance_launches(s, dt, nsteps, false);
+    if (!rc && s->cur != cur0) {   // an odd number of steps: the result back into the slab the next replay starts from
+        if (int c = hipclaw::launch_copy_patches(s->q[s->cur], s->q[cur0], s->all_slots, s->npatch, s->pstride, s->st))
+            rc = hipfail((hipError_t) c, "copy_patches launch");
+    }
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(s->st, &g);
     s->cur = cur0;  // capture only recorded the launches
@@ -2095,10 +2124,16 @@ int hipclaw_capture_graph(hipclaw_state_t* s, double dt, int nsteps) {
 
 int hipclaw_replay_graph(hipclaw_state_t* s) {
     if (!s || !s->gexec) return fail(HIPCLAW_EINVAL, "no captured graph%s");
-    if (s->cur != s->graph_cur)
+    if (s->cur != s->graph_cur && !s->covers)
         return fail(HIPCLAW_EINVAL, "the captured graph starts from the other slab (an odd number of "
                                     "steps or a restored step since the capture)%s");
     if (int rc = guard_save(s)) return rc;
+    if (s->cur != s->graph_cur) {   // (any number of steps where a tile covers a patch)
+        if (int e = hipclaw::launch_copy_patches(s->q[s->cur], s->q[s->graph_cur], s->all_slots, s->npatch,
+                                                 s->pstride, s->st))
+            return hipfail((hipError_t) e, "copy_patches launch");
+        s->cur = s->graph_cur;
+    }
     HIP_TRY(hipEventRecord(s->region[0], s->st));
     HIP_TRY(hipGraphLaunch(s->gexec, s->st));
     HIP_TRY(hipEventRecord(s->region[1], s->st));
@@ -2282,9 +2317,16 @@ int hipclaw_regrid(hipclaw_state_t* s, int npatch_new, const int* kind, const in
         s->q[0] = qnew;
         s->q[1] = nullptr;
         s->cur = 0;
-        if (!s->inplace) {
-            if (hipMalloc((void**) &s->q[1], sizeof(double) * s->pstride * (size_t) cap) != hipSuccess)
-                return fail(HIPCLAW_ENOMEM, "hipclaw_regrid: device allocation failed%s");
+        if (s->covers) {
+            const int old = s->max_patches;
+            s->max_patches = cap;
+            second_slab(s);
+            s->max_patches = old;
+        } else if (hipMalloc((void**) &s->q[1], sizeof(double) * s->pstride * (size_t) cap) != hipSuccess) {
+            s->q[1] = nullptr;
+            return fail(HIPCLAW_ENOMEM, "hipclaw_regrid: device allocation failed%s");
+        }
+        if (s->q[1]) {
             HIP_TRY(hipMemset(s->q[1], 0, sizeof(double) * s->pstride * (size_t) cap));
         }
     }

@@ -125,10 +125,8 @@ int launch_apply_qcorr(double* q, const double* qcorr, const int* cmask, const i
                        hipStream_t st);
 int launch_step_fp64(int solver, int tile, int waves, const StepArgs& a, const StepLaunch& st);
 int launch_step_fp32(int solver, int tile, int waves, const StepArgs& a, const StepLaunch& st);
-// The default waves per workgroup of a tile (0 where there is no choice).
-int default_waves_fp64(int solver, int tile);
-int default_waves_fp32(int solver, int tile);
-int launch_reset_scalar(unsigned long long* p, hipStream_t st);
+// The CFL words (StepArgs::cfl) to zero.
+int launch_reset_cfl(unsigned long long* p, hipStream_t st);
 // Whole patch slabs src[slot] -> dst[slot].
 int launch_copy_patches(const double* src, double* dst, const int* slots, int n, long long pstride,
                         hipStream_t st);

@@ -572,7 +572,7 @@ int launch_apply_qcorr(double* q, const double* qcorr, const int* cmask, const i
     return (int) hipGetLastError();
 }
 
-__global__ void reset_scalar(unsigned long long* p) { *p = 0ull; }
+__global__ void reset_cfl(unsigned long long* p) { p[threadIdx.x * CFL_STRIDE] = 0ull; }
 
 // ---------------------------------------------------------------- regrid
 // Gradient criterion of the reference's tag4refinement / tag4coarsening
@@ -923,8 +923,8 @@ int launch_regrid_remap(const double* qold, double* qnew, const int* ops, int no
     return (int) hipGetLastError();
 }
 
-int launch_reset_scalar(unsigned long long* p, hipStream_t st) {
-    hipLaunchKernelGGL(reset_scalar, dim3(1), dim3(1), 0, st, p);
+int launch_reset_cfl(unsigned long long* p, hipStream_t st) {
+    hipLaunchKernelGGL(reset_cfl, dim3(1), dim3(CFL_WORDS), 0, st, p);
     return (int) hipGetLastError();
 }
 
@@ -1103,12 +1103,10 @@ int launch_time_sync(const SyncArgs& a, hipStream_t st) {
 int launch_step_fp64(int solver, int tile, int waves, const StepArgs& a, const StepLaunch& st) {
     switch (solver) {
     case 0: return launch_step_tile<RPAdvection<double>, double, true>(tile, waves, a, st);
-    case 1: return launch_step_tile<RPShallow<double>, double, true, true>(tile, waves, a, st);
+    case 1: return launch_step_tile<RPShallow<double>, double, true>(tile, waves, a, st);
     case 2: return launch_step_tile<RPEuler<double>, double, true>(tile, waves, a, st);
     default: return (int) hipErrorInvalidValue;
     }
 }
-
-int default_waves_fp64(int /*solver*/, int tile) { return tile == 16 ? default_waves_t16<double>() : 0; }
 
 }  // namespace hipclaw

@@ -1,6 +1,7 @@
-// Launch dispatch of the step kernel for one Riemann functor: tile size,
-// waves per workgroup, time-sync registers and the compile-time MC limiter
-// pick one instantiation of step_tiles.  Shared by the built-in solvers' two
+// Launch dispatch of the step kernel for one Riemann functor: the strip kernel
+// (step_strips), or for solvers with more wave components than a lane can keep
+// the LDS tile kernel (step_tiles); time-sync registers and the compile-time
+// method pick the instantiation.  Shared by the built-in solvers' two
 // translation units (FP64 compiled without FMA contraction, FP32-bulk with it)
 // and by solvers an application compiles itself (hipclaw_user_solver.h); the
 // instantiations take the contraction mode of the unit that includes this.
@@ -12,7 +13,7 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
-#include "hipclaw_step.h"
+#include "hipclaw_strips.h"
 
 namespace hipclaw {
 
@@ -108,33 +109,94 @@ inline int launch_step_shape(const StepArgs& a, const StepLaunch& st) {
     }
 }
 
-// Waves per 16 x 16 tile by default: four for FP64, two for the FP32-bulk
-// form (hipclaw_set_waves and the autotuner choose between 2 and 4).  A sweep
-// covers T + 2 = 18 rows, three per wave (19 interfaces each), so two waves
-// take three row groups each where four take two, two, one and one and wait
-// at the barrier, and the smaller workgroups pack more densely on a CU; FP64
-// tiles need the latency hiding of four.  Measured on MI355X (autotuner
-// trials, ms per step): shallow water FP32 on the benchmark forest 0.133 with
-// two waves against 0.150 with four, the Euler shock-bubble 0.076 against
-// 0.094, the 64-run ensemble 0.476 against 0.494.
-template <typename R>
-constexpr int default_waves_t16() { return sizeof(R) == 8 ? 4 : 2; }
+// Strips keep one interface's waves of three rows in registers, 16 wave
+// components (Euler's 4 x 4) at most; a solver with more of them runs on tiles.
+// Below that strips are faster wherever a launch has a few hundred waves'
+// work, and no slower than 1.2 times the tiles where it has less (kernel times
+// with tiles and with strips, us: shallow water FP64 16 x 16, 16 patches 12.4 /
+// 13.7, 256 15.7 / 18.0, 2800 77 / 65; 32 x 32, 6000 patches FP64 534 / 371,
+// FP32-bulk 194 / 144; Euler FP64 899 / 630; advection FP64 142 / 67).
+template <class RP>
+constexpr bool uses_strips() { return RP::MEQN * RP::MWAVES <= 16; }
 
-// waves = 0: the default for 16 x 16 tiles; 2, 3 or 4 select the variant.
-// T = 32 only where WITH32 (its LDS budget is checked per solver).
-template <class RP, typename R, bool WITH_REGS, bool WITH32 = false>
-inline int launch_step_tile(int tile, int waves, const StepArgs& a, const StepLaunch& st) {
-    if (tile == 16 && waves == 0) waves = default_waves_t16<R>();
-    switch (tile) {
-    case 8: return launch_step_shape<RP, R, 8, 2, WITH_REGS>(a, st);
-    case 16:
-        return waves == 2 ? launch_step_shape<RP, R, 16, 2, WITH_REGS>(a, st)
-             : waves == 3 ? launch_step_shape<RP, R, 16, 3, WITH_REGS>(a, st)
-                          : launch_step_shape<RP, R, 16, 4, WITH_REGS>(a, st);
-    case 32:
-        if constexpr (WITH32) return launch_step_shape<RP, R, 32, 16, WITH_REGS>(a, st);
+inline int device_simds() {
+    static std::atomic<int> simds{0};
+    int n = simds.load(std::memory_order_relaxed);
+    if (n <= 0) {
+        int dev = 0, cus = 0;
+        if (hipGetDevice(&dev) == hipSuccess &&
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
+            n = 4 * cus;
+        simds.store(n, std::memory_order_relaxed);
+    }
+    return n;
+}
+
+// pairs: two waves of the kernel fit a SIMD.  nw: waves per workgroup.  The
+// waves share nothing; one per workgroup lets the dispatcher place each by itself.
+template <typename K>
+inline int launch_strips(K kernel, bool pairs, int nw, const StepArgs& a, const StepLaunch& L) {
+    if (a.nwork <= 0) return 0;
+    const bool inplace = a.qsrc == a.qdst;
+    const int simds = device_simds();
+    StripShape sh;
+    if (simds <= 0 || !strip_pattern(a.mx, inplace, sh)) return (int) hipErrorInvalidValue;
+    strip_rows(a.my, a.nwork, simds, pairs, inplace, sh);
+    const long long waves = ((long long) a.nwork + sh.patches - 1) / sh.patches * sh.waves * sh.nsy;
+    const long long blocks = ((waves + nw - 1) / nw + 7) / 8 * 8;   // a multiple of the 8 XCDs
+    if (waves * 64 > 0x7fffffffLL) return (int) hipErrorInvalidConfiguration;
+    if (L.start || L.stop)
+        hipExtLaunchKernelGGL(kernel, dim3((unsigned) blocks), dim3(64 * nw), 0, L.st, L.start, L.stop, 0, a, sh);
+    else
+        hipLaunchKernelGGL(kernel, dim3((unsigned) blocks), dim3(64 * nw), 0, L.st, a, sh);
+    return (int) hipGetLastError();
+}
+
+// The strip kernel of one precision: with and without time-sync registers
+// (overwritten, or added to when subcycling), and with order (2, 2) and the MC
+// limiter on every wave family fixed at compile time.
+template <class RP, typename R, bool WITH_REGS>
+inline int launch_step_strips(int nw, const StepArgs& a, const StepLaunch& st) {
+    constexpr bool FF = sizeof(R) == 4 && RP::CONSERVATIVE, pairs = strip_waves_per_eu<RP, R>() > 1;
+    const bool std = all_mc_limiter<RP>(a) && a.order2 && a.transverse == 2;
+    if (a.reg) {
+        if constexpr (WITH_REGS) {
+            if (a.reg_accumulate)
+                return std ? launch_strips(step_strips<RP, R, FF, 2, true>, pairs, nw, a, st)
+                           : launch_strips(step_strips<RP, R, FF, 2, false>, pairs, nw, a, st);
+            return std ? launch_strips(step_strips<RP, R, FF, 1, true>, pairs, nw, a, st)
+                       : launch_strips(step_strips<RP, R, FF, 1, false>, pairs, nw, a, st);
+        }
         return (int) hipErrorInvalidValue;
-    default: return (int) hipErrorInvalidValue;
+    }
+    return std ? launch_strips(step_strips<RP, R, FF, 0, true>, pairs, nw, a, st)
+               : launch_strips(step_strips<RP, R, FF, 0, false>, pairs, nw, a, st);
+}
+
+// Waves per workgroup by default.  Strips: one.  16 x 16 tiles: four for FP64,
+// two for the FP32-bulk form (a sweep's 18 rows, three per wave, are three
+// groups for each of two waves, where four take two, two, one and one and wait
+// at the barrier; FP64 tiles need the latency hiding of four).
+// hipclaw_set_waves and the autotuner choose 2, 3 or 4.
+inline int default_waves(bool strips, bool fp64, int tile) {
+    return tile != 16 ? 0 : strips ? 1 : fp64 ? 4 : 2;   // (0: one choice)
+}
+
+// waves = 0: the default; 2, 3 or 4 select the variant.
+template <class RP, typename R, bool WITH_REGS>
+inline int launch_step_tile(int tile, int waves, const StepArgs& a, const StepLaunch& st) {
+    if constexpr (uses_strips<RP>()) {
+        return launch_step_strips<RP, R, WITH_REGS>(waves > 0 ? waves : 1, a, st);
+    } else {
+        if (waves == 0) waves = default_waves(false, sizeof(R) == 8, tile);
+        switch (tile) {
+        case 8: return launch_step_shape<RP, R, 8, 2, WITH_REGS>(a, st);
+        case 16:
+            return waves == 2 ? launch_step_shape<RP, R, 16, 2, WITH_REGS>(a, st)
+                 : waves == 3 ? launch_step_shape<RP, R, 16, 3, WITH_REGS>(a, st)
+                              : launch_step_shape<RP, R, 16, 4, WITH_REGS>(a, st);
+        default: return (int) hipErrorInvalidValue;
+        }
     }
 }
 

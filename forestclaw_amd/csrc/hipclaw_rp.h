@@ -52,6 +52,15 @@ __device__ __forceinline__ R zadd(R x) { return sizeof(R) == 4 ? x : R(0) + x; }
 template <typename R>
 __device__ __forceinline__ R zsub(R x) { return sizeof(R) == 4 ? -x : R(0) - x; }
 
+// a b + c.  FP64 rounds twice, as the reference does; FP32 is one fused
+// operation, written out instead of left to the compiler's contraction, so that
+// every copy of the code gives the same bits.
+__device__ __forceinline__ double mad(double a, double b, double c) {
+#pragma clang fp contract(off)
+    return a * b + c;
+}
+__device__ __forceinline__ float mad(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
 // Division and square root.  FP64 keeps IEEE-correct operations (the parity
 // form); the FP32-bulk form uses the hardware reciprocal and square root
 // (v_rcp_f32, v_sqrt_f32, 1 ulp), whose error is far below the form's
@@ -85,6 +94,20 @@ struct rpt2_linear : std::false_type {};
 template <class RP>
 struct rpt2_linear<RP, std::enable_if_t<RP::RPT2_LINEAR>> : std::true_type {};
 
+// A solver whose wave speeds follow from what rpn2 hands to rpt2
+// (RP::speeds(roe, s), the same operations): they need not be kept beside it.
+template <class RP, class = void>
+struct roe_speeds : std::false_type {};
+template <class RP>
+struct roe_speeds<RP, std::void_t<decltype(&RP::speeds)>> : std::true_type {};
+
+// A solver whose FP32 arithmetic names its fused operations (RP::EXPLICIT_FMA):
+// every inlined copy of it gives the same bits.
+template <class RP, class = void>
+struct explicit_fma : std::false_type {};
+template <class RP>
+struct explicit_fma<RP, std::enable_if_t<RP::EXPLICIT_FMA>> : std::true_type {};
+
 // ----------------------------------------------------------------- shallow water
 // Wave components that are zero by construction.  A sum over the waves that
 // starts at +0 may skip those terms without changing its bits (in
@@ -104,8 +127,13 @@ struct RPShallow {
     static constexpr int MEQN = 3, MWAVES = 3, MAUX = 0;
     static constexpr bool CONSERVATIVE = true;  // amdq + apdq = f(qR) - f(qL)
     static constexpr bool RPT2_LINEAR = true;   // bm, bp linear in asdq
+    static constexpr bool EXPLICIT_FMA = true;  // no contraction left to the compiler (mad)
     // u, v, a (and in FP32 1 / (2 a), which rpt2 then takes from the normal solve)
     static constexpr int NROE = sizeof(R) == 4 ? 4 : 3;
+
+    __device__ __forceinline__ static void speeds(const R roe[NROE], R s[MWAVES]) {
+        s[0] = roe[0] - roe[2]; s[1] = roe[0]; s[2] = roe[0] + roe[2];
+    }
 
     // the shear wave carries no depth and no normal momentum
     template <int IXY>
@@ -152,13 +180,7 @@ struct RPShallow {
     // intermediate state h, hu_n of the entropy fix
     template <int SIGN>
     __device__ __forceinline__ static R char_speed(R hu, R h, const PhysParams& pp) {
-        if constexpr (sizeof(R) == 4) {
-            const float rs = __builtin_amdgcn_rsqf(h);
-            const float hs = h * rs;
-            return SIGN < 0 ? hu * rs * rs - sqrt_grav(pp) * hs : hu * rs * rs + sqrt_grav(pp) * hs;
-        } else {
-            return SIGN < 0 ? dv(hu, h) - sq((R) pp.grav * h) : dv(hu, h) + sq((R) pp.grav * h);
-        }
+        return SIGN < 0 ? dv(hu, h) - sq((R) pp.grav * h) : dv(hu, h) + sq((R) pp.grav * h);
     }
 
     template <int IXY>
@@ -179,32 +201,66 @@ struct RPShallow {
                                                  const R* /*auxR*/, const PhysParams& pp,
                                                  R wave[MWAVES][MEQN], R s[MWAVES], R amdq[MEQN],
                                                  R apdq[MEQN], R roe[NROE]) {
+        if constexpr (sizeof(R) == 4) rpn2c_fp32<IXY>(qL, qR, cL, cR, pp, wave, s, amdq, apdq, roe);
+        else rpn2c_fp64<IXY>(qL, qR, cL, cR, pp, wave, s, amdq, apdq, roe);
+    }
+
+    // FP32: one reciprocal and one reciprocal square root for the Roe averages
+    // (1 / (2 a) = rsq(g h) / 2), and the entropy fix without branches: the
+    // states left and right of the shear wave have the same depth and normal
+    // momentum, so one intermediate state serves both, and at most one of the
+    // two outer waves is transonic there.
+    template <int IXY>
+    __device__ __forceinline__ static void rpn2c_fp32(const R* qL, const R* qR, const R* cL, const R* cR,
+                                                      const PhysParams& pp, R wave[MWAVES][MEQN],
+                                                      R s[MWAVES], R amdq[MEQN], R apdq[MEQN], R roe[NROE]) {
+#pragma clang fp contract(off)
+        constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
+        const float gh = (0.5f * (float) pp.grav) * (qL[0] + qR[0]);
+        const float ra = __builtin_amdgcn_rsqf(gh), rh = __builtin_amdgcn_rcpf(cL[0] + cR[0]);
+        const float u = (cL[1] + cR[1]) * rh, v = (cL[2] + cR[2]) * rh;
+        const float a = gh * ra, inv2a = 0.5f * ra;
+        roe[0] = u; roe[1] = v; roe[2] = a; roe[NROE - 1] = inv2a;
+        const float d0 = qR[0] - qL[0], d1 = qR[mu] - qL[mu], d2 = qR[mv] - qL[mv];
+        const float s0 = u - a, s2 = u + a;
+        const float a1 = mad(s2, d0, -d1) * inv2a, a3 = mad(-s0, d0, d1) * inv2a, a2 = mad(-v, d0, d2);
+        wave[0][0] = a1;   wave[0][mu] = a1 * s0; wave[0][mv] = a1 * v; s[0] = s0;
+        wave[1][0] = 0.0f; wave[1][mu] = 0.0f;    wave[1][mv] = a2;     s[1] = u;
+        wave[2][0] = a3;   wave[2][mu] = a3 * s2; wave[2][mv] = a3 * v; s[2] = s2;
+        // characteristic speeds of the left, intermediate and right states
+        const float hm = qL[0] + a1, hum = qL[mu] + wave[0][mu];
+        const float rm = __builtin_amdgcn_rsqf(hm), um = hum * rm * rm, cm = sqrt_grav(pp) * (hm * rm);
+        const float lL = cL[3] - cL[4], lR = cR[3] + cR[4], l1 = um - cm, l3 = um + cm;
+        const bool t1 = lL < 0.0f && l1 > 0.0f, t3 = l3 < 0.0f && lR > 0.0f;
+        const float r = __builtin_amdgcn_rcpf(t3 ? lR - l3 : l1 - lL);
+        const float f1 = t1 ? lL * ((l1 - s0) * r) : rmin(s0, 0.0f);
+        float f3 = t3 ? l3 * ((lR - s2) * r) : rmin(s2, 0.0f);
+        f3 = u > 0.0f ? 0.0f : f3;
+        const float f2 = rmin(u, 0.0f), g1 = s0 - f1, g2 = rmax(u, 0.0f), g3 = s2 - f3;
+        amdq[0] = mad(f3, a3, f1 * a1);
+        amdq[mu] = mad(f3, wave[2][mu], f1 * wave[0][mu]);
+        amdq[mv] = mad(f2, a2, mad(f3, wave[2][mv], f1 * wave[0][mv]));
+        apdq[0] = mad(g3, a3, g1 * a1);
+        apdq[mu] = mad(g3, wave[2][mu], g1 * wave[0][mu]);
+        apdq[mv] = mad(g2, a2, mad(g3, wave[2][mv], g1 * wave[0][mv]));
+    }
+
+    template <int IXY>
+    __device__ __forceinline__ static void rpn2c_fp64(const R* qL, const R* qR, const R* cL, const R* cR,
+                                                      const PhysParams& pp, R wave[MWAVES][MEQN],
+                                                      R s[MWAVES], R amdq[MEQN], R apdq[MEQN], R roe[NROE]) {
         constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
         const R grav = (R) pp.grav;
         const R h = dv(qL[0] + qR[0], R(2));
         const R hsqrtl = cL[0];
         const R hsqrtr = cR[0];
         const R hsq2 = hsqrtl + hsqrtr;
-        R u, v, a, a1, a3;
         const R d0 = qR[0] - qL[0], d1 = qR[mu] - qL[mu], d2 = qR[mv] - qL[mv];
-        if constexpr (sizeof(R) == 4) {
-            // one reciprocal and one reciprocal square root: 1 / (2 a) = rsq(g h) / 2
-            const float rh = __builtin_amdgcn_rcpf(hsq2);
-            u = (cL[1] + cR[1]) * rh;
-            v = (cL[2] + cR[2]) * rh;
-            const float gh = grav * h, ra = __builtin_amdgcn_rsqf(gh);
-            a = gh * ra;
-            const float inv2a = 0.5f * ra;
-            roe[3] = inv2a;
-            a1 = ((u + a) * d0 - d1) * inv2a;
-            a3 = (-((u - a) * d0) + d1) * inv2a;
-        } else {
-            u = dv(cL[1] + cR[1], hsq2);
-            v = dv(cL[2] + cR[2], hsq2);
-            a = sq(grav * h);
-            a1 = dv((u + a) * d0 - d1, R(2) * a);
-            a3 = dv(-((u - a) * d0) + d1, R(2) * a);
-        }
+        const R u = dv(cL[1] + cR[1], hsq2);
+        const R v = dv(cL[2] + cR[2], hsq2);
+        const R a = sq(grav * h);
+        const R a1 = dv((u + a) * d0 - d1, R(2) * a);
+        const R a3 = dv(-((u - a) * d0) + d1, R(2) * a);
         roe[0] = u; roe[1] = v; roe[2] = a;
         const R a2 = -(v * d0) + d2;
 
@@ -261,14 +317,25 @@ struct RPShallow {
                                                 R bp[MEQN]) {
         constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
         const R u = roe[0], v = roe[1], a = roe[2];
-        R a1, a3;
         if constexpr (sizeof(R) == 4) {
-            a1 = ((v + a) * asdq[0] - asdq[mv]) * roe[3];
-            a3 = (-((v - a) * asdq[0]) + asdq[mv]) * roe[3];
-        } else {
-            a1 = dv((v + a) * asdq[0] - asdq[mv], R(2) * a);
-            a3 = dv(-((v - a) * asdq[0]) + asdq[mv], R(2) * a);
+#pragma clang fp contract(off)
+            // waves a1 (1, u, v - a), a2 (0, 1, 0), a3 (1, u, v + a), summed by
+            // their common factors
+            const float r2 = roe[NROE - 1];
+            const float a1 = mad(v + a, asdq[0], -asdq[mv]) * r2, a3 = mad(a - v, asdq[0], asdq[mv]) * r2;
+            const float a2 = mad(-u, asdq[0], asdq[mu]);
+            const float m1 = rmin(v - a, 0.0f) * a1, m3 = rmin(v + a, 0.0f) * a3;
+            const float p1 = rmax(v - a, 0.0f) * a1, p3 = rmax(v + a, 0.0f) * a3;
+            bm[0] = m1 + m3;
+            bm[mu] = mad(u, bm[0], rmin(v, 0.0f) * a2);
+            bm[mv] = mad(v, bm[0], a * (m3 - m1));
+            bp[0] = p1 + p3;
+            bp[mu] = mad(u, bp[0], rmax(v, 0.0f) * a2);
+            bp[mv] = mad(v, bp[0], a * (p3 - p1));
+            return;
         }
+        const R a1 = dv((v + a) * asdq[0] - asdq[mv], R(2) * a);
+        const R a3 = dv(-((v - a) * asdq[0]) + asdq[mv], R(2) * a);
         const R a2 = asdq[mu] - u * asdq[0];
         R wb[3][3], sb[3];
         wb[0][0] = a1;   wb[0][mu] = a1 * u; wb[0][mv] = a1 * (v - a); sb[0] = v - a;
@@ -331,9 +398,14 @@ struct RPEuler {
     static constexpr int MEQN = 4, MWAVES = 4, MAUX = 0;
     static constexpr bool CONSERVATIVE = true;
     static constexpr bool RPT2_LINEAR = true;   // bm, bp linear in asdq
+    static constexpr bool EXPLICIT_FMA = true;  // no contraction left to the compiler (mad)
     // u, v, a, enth, u2v2, g1a2, euv (and in FP32 1 / (2 a), which rpt2 then
     // takes from the normal solve)
     static constexpr int NROE = sizeof(R) == 4 ? 8 : 7;
+
+    __device__ __forceinline__ static void speeds(const R roe[NROE], R s[MWAVES]) {
+        s[0] = roe[0] - roe[2]; s[1] = s[2] = roe[0]; s[3] = roe[0] + roe[2];
+    }
 
     // the shear wave carries no density and no normal momentum
     template <int IXY>
@@ -355,9 +427,10 @@ struct RPEuler {
         const R gamma = (R) pp.gamma;
         const R gamma1 = (R) (pp.gamma - 1.0);
         if constexpr (sizeof(R) == 4) {
-            const float r = __builtin_amdgcn_rsqf(q[0]), rr = r * r;
+#pragma clang fp contract(off)
+            const float r = __builtin_amdgcn_rsqf(q[0]);
             // one pressure (the two summation orders differ only in rounding)
-            const float p = gamma1 * (q[3] - 0.5f * (q[1] * q[1] + q[2] * q[2]) * rr);
+            const float u = q[1] * r, v = q[2] * r, p = gamma1 * mad(-0.5f, mad(u, u, v * v), q[3]);
             c[0] = q[0] * r;
             c[1] = q[mu] * r;
             c[2] = q[mv] * r;
@@ -395,6 +468,7 @@ struct RPEuler {
                                                  const R* /*auxR*/, const PhysParams& pp,
                                                  R wave[MWAVES][MEQN], R s[MWAVES], R amdq[MEQN],
                                                  R apdq[MEQN], R roe[NROE]) {
+#pragma clang fp contract(off)
         constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
         const R gamma = (R) pp.gamma;
         const R gamma1 = (R) (pp.gamma - 1.0);
@@ -414,8 +488,8 @@ struct RPEuler {
             v = dv(cL[2] + cR[2], rhsq2);
             enth = dv(cL[3] + cR[3], rhsq2);
         }
-        const R u2v2 = u * u + v * v;
-        const R a2s = gamma1 * (enth - R(.5) * u2v2);
+        const R u2v2 = mad(v, v, u * u);
+        const R a2s = gamma1 * mad(R(-.5), u2v2, enth);
         if constexpr (sizeof(R) == 4) {
             const float ra = __builtin_amdgcn_rsqf(a2s);
             a = a2s * ra;
@@ -430,21 +504,22 @@ struct RPEuler {
         roe[0] = u; roe[1] = v; roe[2] = a; roe[3] = enth; roe[4] = u2v2; roe[5] = g1a2; roe[6] = euv;
 
         const R d0 = qR[0] - qL[0], d1 = qR[mu] - qL[mu], d2 = qR[mv] - qL[mv], d3 = qR[3] - qL[3];
-        const R a3 = g1a2 * (euv * d0 + u * d1 + v * d2 - d3);
-        const R a2 = d2 - v * d0;
+        const R a3 = g1a2 * (mad(v, d2, mad(u, d1, euv * d0)) - d3);
+        const R a2 = mad(-v, d0, d2);
+        const R t4 = mad(-a, a3, mad(a - u, d0, d1));
         R a4;
-        if constexpr (sizeof(R) == 4) a4 = (d1 + (a - u) * d0 - a * a3) * inv2a;
-        else a4 = dv(d1 + (a - u) * d0 - a * a3, R(2) * a);
+        if constexpr (sizeof(R) == 4) a4 = t4 * inv2a;
+        else a4 = dv(t4, R(2) * a);
         const R a1 = d0 - a3 - a4;
 
         wave[0][0] = a1; wave[0][mu] = a1 * (u - a); wave[0][mv] = a1 * v;
-        wave[0][3] = a1 * (enth - u * a); s[0] = u - a;
+        wave[0][3] = a1 * mad(-u, a, enth); s[0] = u - a;
         wave[1][0] = R(0); wave[1][mu] = R(0); wave[1][mv] = a2;
         wave[1][3] = a2 * v; s[1] = u;
         wave[2][0] = a3; wave[2][mu] = a3 * u; wave[2][mv] = a3 * v;
         wave[2][3] = a3 * R(0.5) * u2v2; s[2] = u;
         wave[3][0] = a4; wave[3][mu] = a4 * (u + a); wave[3][mv] = a4 * v;
-        wave[3][3] = a4 * (enth + u * a); s[3] = u + a;
+        wave[3][3] = a4 * mad(u, a, enth); s[3] = u + a;
 
         // entropy fix
         const R s0 = cL[4] - cL[5];   // u_n - c of the left cell
@@ -456,7 +531,7 @@ struct RPEuler {
             const R rhou1 = qL[mu] + wave[0][mu];
             const R rhov1 = qL[mv] + wave[0][mv];
             const R en1 = qL[3] + wave[0][3];
-            const R p1 = gamma1 * (en1 - dv(R(0.5) * (rhou1 * rhou1 + rhov1 * rhov1), rho1));
+            const R p1 = gamma1 * (en1 - dv(R(0.5) * mad(rhov1, rhov1, rhou1 * rhou1), rho1));
             const R c1 = sq(dv(gamma * p1, rho1));
             const R s1 = dv(rhou1, rho1) - c1;
             R sfract;
@@ -468,15 +543,15 @@ struct RPEuler {
             if (!(s[1] >= R(0))) {
 #pragma unroll
                 for (int m = 0; m < 4; m++) {
-                    amdq[m] = amdq[m] + s[1] * wave[1][m];
-                    amdq[m] = amdq[m] + s[2] * wave[2][m];
+                    amdq[m] = mad(s[1], wave[1][m], amdq[m]);
+                    amdq[m] = mad(s[2], wave[2][m], amdq[m]);
                 }
                 const R s3 = cR[4] + cR[5];   // u_n + c of the right cell
                 const R rho2 = qR[0] - wave[3][0];
                 const R rhou2 = qR[mu] - wave[3][mu];
                 const R rhov2 = qR[mv] - wave[3][mv];
                 const R en2 = qR[3] - wave[3][3];
-                const R p2 = gamma1 * (en2 - dv(R(0.5) * (rhou2 * rhou2 + rhov2 * rhov2), rho2));
+                const R p2 = gamma1 * (en2 - dv(R(0.5) * mad(rhov2, rhov2, rhou2 * rhou2), rho2));
                 const R c2 = sq(dv(gamma * p2, rho2));
                 const R s2 = dv(rhou2, rho2) + c2;
                 bool add = true;
@@ -485,7 +560,7 @@ struct RPEuler {
                 else add = false;
                 if (add) {
 #pragma unroll
-                    for (int m = 0; m < 4; m++) amdq[m] = amdq[m] + sfract * wave[3][m];
+                    for (int m = 0; m < 4; m++) amdq[m] = mad(sfract, wave[3][m], amdq[m]);
                 }
             }
         }
@@ -494,7 +569,7 @@ struct RPEuler {
             R df = R(0);
 #pragma unroll
             for (int mw = 0; mw < 4; mw++)
-                if (!wave_zero<IXY>(mw, m)) df = df + s[mw] * wave[mw][m];
+                if (!wave_zero<IXY>(mw, m)) df = mad(s[mw], wave[mw][m], df);
             apdq[m] = df - amdq[m];
         }
     }
@@ -504,14 +579,32 @@ struct RPEuler {
                                                 const R* /*aux1*/, const R* /*aux2*/,
                                                 const R* /*aux3*/, const PhysParams&, R bm[MEQN],
                                                 R bp[MEQN]) {
+#pragma clang fp contract(off)
         constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
         const R u = roe[0], v = roe[1], a = roe[2], enth = roe[3], u2v2 = roe[4];
         const R g1a2 = roe[5], euv = roe[6];
-        const R a3 = g1a2 * (euv * asdq[0] + u * asdq[mu] + v * asdq[mv] - asdq[3]);
-        const R a2 = asdq[mu] - u * asdq[0];
-        R a4;
-        if constexpr (sizeof(R) == 4) a4 = (asdq[mv] + (a - v) * asdq[0] - a * a3) * roe[7];
-        else a4 = dv(asdq[mv] + (a - v) * asdq[0] - a * a3, R(2) * a);
+        const R a3 = g1a2 * (mad(v, asdq[mv], mad(u, asdq[mu], euv * asdq[0])) - asdq[3]);
+        const R a2 = mad(-u, asdq[0], asdq[mu]);
+        const R t4 = mad(-a, a3, mad(a - v, asdq[0], asdq[mv]));
+        if constexpr (sizeof(R) == 4) {
+            // waves a1 (1, u, v - a, H - v a), a3 (1, u, v, (u^2 + v^2) / 2) +
+            // a2 (0, 1, 0, u), a4 (1, u, v + a, H + v a), summed by their common
+            // factors
+            const float a4 = t4 * roe[7], a1 = asdq[0] - a3 - a4;
+            auto split = [&](float w1, float w2, float w4, float* b) {
+#pragma clang fp contract(off)
+                const float x1 = w1 * a1, x4 = w4 * a4, y3 = w2 * a3, y2 = w2 * a2;
+                const float t = x1 + x4, d = a * (x4 - x1);
+                b[0] = t + y3;
+                b[mu] = mad(u, b[0], y2);
+                b[mv] = mad(v, b[0], d);
+                b[3] = mad(enth, t, mad(v, d, mad(0.5f * u2v2, y3, u * y2)));
+            };
+            split(rmin(v - a, 0.0f), rmin(v, 0.0f), rmin(v + a, 0.0f), bm);
+            split(rmax(v - a, 0.0f), rmax(v, 0.0f), rmax(v + a, 0.0f), bp);
+            return;
+        }
+        const R a4 = dv(t4, R(2) * a);
         const R a1 = asdq[0] - a3 - a4;
         R wb[3][4], sb[3];
         wb[0][0] = a1; wb[0][mu] = a1 * u; wb[0][mv] = a1 * (v - a);
@@ -583,6 +676,7 @@ struct RPAdvection {
     // difference unless the velocity is uniform, so no flux form exists
     static constexpr bool CONSERVATIVE = false;
     static constexpr bool RPT2_LINEAR = true;   // bm, bp linear in asdq
+    static constexpr bool EXPLICIT_FMA = true;  // no contraction left to the compiler (mad)
     static constexpr int NROE = 1;
 
     template <int IXY>

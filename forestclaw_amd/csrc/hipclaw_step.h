@@ -1,4 +1,5 @@
-// Batched patch-update kernel.  A persistent workgroup loops over the T x T
+// What a step reads and writes (StepArgs), the arithmetic shared by both step
+// kernels, and the tile kernel.  A persistent workgroup loops over the T x T
 // tiles of every patch in a work list (all levels of the forest in one
 // launch) and updates each tile's interior cells.
 //
@@ -35,6 +36,8 @@
 
 namespace hipclaw {
 
+constexpr int CFL_WORDS = 16, CFL_STRIDE = 32;   // (256 bytes apart)
+
 struct StepArgs {
     const double* qsrc;        // [slot][meqn][my+2mbc][mx+2mbc]
     double* qdst;              // may equal qsrc when one tile covers a patch
@@ -42,7 +45,10 @@ struct StepArgs {
     const int* work;           // patch slots to update
     const double* dxs;         // [slot]
     const double* dys;         // [slot]
-    unsigned long long* cfl;   // FP64 bits, atomic max (non-negative doubles order as integers)
+    // Courant number: FP64 bits, atomic max (non-negative doubles order as
+    // integers).  CFL_WORDS words CFL_STRIDE apart, the result being the largest
+    // of them: atomics on one word are served one after another, ~11 ns each.
+    unsigned long long* cfl;
     long long pstride;         // doubles per patch in q
     long long astride;         // doubles per patch in aux
     int nwork;
@@ -208,9 +214,9 @@ __device__ __forceinline__ void riemann(const R* qL, const R* qR, const R* auxL,
     }
 }
 
-// Waves per SIMD the register allocation aims for: 4, except FP64 16 x 16
-// tiles, which need more than the 128 VGPRs of 4 waves and are held to the 168
-// of 3 (without the target the allocator let them grow to 2 waves).
+// The tile kernel serves the solvers with more wave components per interface
+// (meqn x mwaves > 16) than the strip kernel's lanes can keep; the allocator
+// sizes it without a target for the waves per SIMD.
 //
 // LIM = 0 reads each wave family's limiter from a.mthlim at run time; LIM > 0
 // is that limiter for every family, fixed at compile time.  The run-time
@@ -218,21 +224,8 @@ __device__ __forceinline__ void riemann(const R* qL, const R* qR, const R* auxL,
 // sweeps and, with the kernel's other uniform values, spills scalar
 // registers into vector lanes; the fixed form has neither (about 40 % fewer
 // vector instructions in each sweep for the MC limiter).
-//
-// A solver with many equations and waves (more than 16 wave components per
-// interface) cannot keep them in the registers of 4 waves; it gets no target
-// and the allocator sizes the kernel itself.
-template <class RP, typename R, int T>
-constexpr int step_waves_per_eu() {
-    if (RP::MEQN * RP::MWAVES > 16) return 1;
-#ifdef HIPCLAW_WPE_F32_T16
-    if (sizeof(R) == 4 && T == 16) return HIPCLAW_WPE_F32_T16;
-#endif
-    return (sizeof(R) == 8 && T == 16) ? 3 : 4;
-}
-
 template <class RP, typename R, int T, int NW, bool FLUXFORM, bool REGS, int LIM = 0>
-__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(step_waves_per_eu<RP, R, T>())))
+__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1)))
 step_tiles(StepArgs a) {
     constexpr int MEQN = RP::MEQN, MW = RP::MWAVES, MAUX = RP::MAUX, NROE = RP::NROE;
     // wave components zero by construction, skipped in the sums over waves

@@ -1,0 +1,93 @@
+// How a launch of the strip kernel (hipclaw_strips.h) lays the patches of its
+// work list on waves of 64 lanes.  Host code, without HIP.
+#pragma once
+
+namespace hipclaw {
+
+// `waves` waves hold `patches` patches side by side, and the pattern repeats;
+// segment k of wave w of the pattern is a strip of one patch (strip_segment),
+// 0 past the last segment.  A strip of w columns takes w + 4 lanes, its halo
+// among them.  Patches of more columns than a pattern holds take `waves` waves
+// of 60 columns each (the last one fewer), computed instead of listed.  In y a
+// patch is cut into nsy strips of H rows, the last one moved back to end at the
+// patch edge: it overlaps the one before it, and both write the same bits.
+struct StripShape {
+    static constexpr int WAVES = 8, SEGS = 6, LANES = 64, HALO = 4, PATCHES = 15;
+    int H, nsy;
+    int waves, patches;
+    unsigned seg[WAVES][SEGS];
+};
+
+// first lane | columns << 6 | patch of the pattern << 12 | first column (0-based) << 16
+constexpr unsigned strip_segment(int lane, int n, int patch, int col) {
+    return (unsigned) lane | (unsigned) n << 6 | (unsigned) patch << 12 | (unsigned) col << 16;
+}
+
+// Packs patches of mx columns.  A patch that does not fit into what is left of
+// a wave is cut and goes on in the next one (11 % more columns per wave at
+// mx = 32, 37 % at mx = 40, than whole strips of equal width), unless `whole`:
+// an update in place needs the patch in one wave, which then reads every cell
+// before it writes it.  Of the patterns of at most WAVES waves, the one with the
+// most columns per wave; false if `whole` patches have no room.
+inline bool strip_pattern(int mx, bool whole, StripShape& sh) {
+    constexpr int MOST = StripShape::LANES - StripShape::HALO;
+    if (whole && mx > MOST) return false;
+    StripShape t{};
+    int col = 0, patch = 0;      // the next column to lay out
+    double best = 0.0;
+    sh = t;
+    for (int w = 0; w < StripShape::WAVES; w++) {
+        int lane = 0;
+        for (int k = 0; k < StripShape::SEGS; k++) {
+            const int room = MOST - lane, left = mx - col;
+            if (room < 1 || (whole && left > room) || patch >= StripShape::PATCHES) break;
+            const int n = left < room ? left : room;
+            t.seg[w][k] = strip_segment(lane, n, patch, col);
+            lane += n + StripShape::HALO;
+            col += n;
+            if (col == mx) { col = 0; patch++; }
+        }
+        // the pattern that ends with this wave, less the patch only begun
+        const double cols = (double) patch * mx / (w + 1);
+        if (patch > 0 && cols > best * 1.0001) {
+            best = cols;
+            sh = t;
+            sh.waves = w + 1;
+            sh.patches = patch;
+            for (int v = 0; v <= w; v++)
+                for (int k = 0; k < StripShape::SEGS; k++)
+                    if ((int) ((sh.seg[v][k] >> 12) & 15) >= patch) sh.seg[v][k] = 0;
+        }
+    }
+    if (best == 0.0) {           // wider than WAVES waves
+        sh.waves = (mx + MOST - 1) / MOST;
+        sh.patches = 1;
+    }
+    return true;
+}
+
+// Rows per strip.  One wave keeps a SIMD's issue slots nearly full, so a launch
+// takes as long as the SIMD with the most waves: ceil(waves / SIMDs) strips of
+// H + 3 row steps each (three rows lead in).  Alone on its SIMD a wave waits for
+// its own results a sixth of the time, which a second one would use (`pairs`:
+// the kernel's registers leave room for it).  Kernel times, us: shallow water
+// FP64, 700 patches of 32 x 32 (420 waves of columns), H = 4, 8, 16, 32: 72, 61,
+// 63, 111; 256 of 16 x 16 (86), H = 1, 2, 4, 8, 16: 22, 18, 24, 35, 59; Euler
+// FP32-bulk, 2800 of 16 x 16 (934), H = 4, 8, 16: 54, 42, 44; Euler FP64 (one
+// wave per SIMD) 131, 105, 91.
+inline void strip_rows(int my, int nwork, int simds, bool pairs, bool whole, StripShape& sh) {
+    const double cols = (double) nwork * sh.waves / sh.patches;
+    double best = 0.0;
+    sh.nsy = 1;
+    for (int nsy = 1; nsy <= (whole ? 1 : my); nsy++) {
+        const int H = (my + nsy - 1) / nsy;
+        if ((my + H - 1) / H != nsy) continue;   // (the same H as fewer strips)
+        const double load = cols * nsy / simds;
+        const long long rounds = load > 1.0 ? (long long) (load + 0.999) : 1;
+        const double cost = (double) rounds * (H + 3) * (pairs && rounds == 1 ? 1.2 : 1.0);
+        if (nsy == 1 || cost < best) { best = cost; sh.nsy = nsy; }
+    }
+    sh.H = (my + sh.nsy - 1) / sh.nsy;
+}
+
+}  // namespace hipclaw

@@ -1,0 +1,639 @@
+// Batched patch update, one wave per group of column strips.
+//
+// The same step as step_tiles (hipclaw_step.h), organised without LDS and
+// without barriers: a wave holds S strips of W interior columns, one staged
+// column (W + 4 of them, with the halo) per lane, and marches up the rows.
+// Rows and the y-interfaces between them live in registers; the x-direction
+// goes across lanes with DPP shifts.  With row n loaded the wave
+//
+//   * sweeps row n - 1 in x (normal and transverse solves);
+//   * solves the y-interface between rows n - 1 and n;
+//   * limits, corrects and splits the y-interface between rows n - 2 and
+//     n - 1, whose limiter needed the one above it;
+//   * updates and stores row n - 2.
+//
+// Every sum is taken in the order step_tiles takes it, so the FP64 form gives
+// the same bits.
+#pragma once
+
+#include <type_traits>
+
+#include "hipclaw_step.h"
+#include "hipclaw_strip_shape.h"
+
+namespace hipclaw {
+
+// Limiter and second-order correction of one interface (clawpack46_inlinelimiter.f,
+// clawpack46_flux2.f:139-153).  dotl, dotr: the waves' products with those of
+// the interface before and after.  FP64 limits the waves and sums them in the
+// reference's order; FP32 puts the limiter into the sum's coefficients, and a
+// wave whose norm is below the smallest normal number has the limiter of a
+// slightly larger one (its terms are below 1e-19 either way).
+template <class RP, typename R, int IXY, bool STD>
+__device__ __forceinline__ void limited_correction(const StepArgs& a, const R wave[RP::MWAVES][RP::MEQN],
+                                                   const R s[RP::MWAVES], const R dotl[RP::MWAVES],
+                                                   const R dotr[RP::MWAVES], R dtd, R cqxx[RP::MEQN]) {
+#pragma clang fp contract(off)
+    constexpr int MEQN = RP::MEQN, MW = RP::MWAVES;
+    using WZ = wave_zeros<RP, IXY>;
+    R phi[MW];
+#pragma unroll
+    for (int mw = 0; mw < MW; mw++) {
+        phi[mw] = R(1);
+        const int mth = STD ? 4 : a.mthlim[mw];
+        if (mth == 0) continue;
+        R wn = R(0);
+#pragma unroll
+        for (int m = 0; m < MEQN; m++)
+            if (!WZ::at(mw, m)) wn = mad(wave[mw][m], wave[mw][m], wn);
+        const R d = s[mw] > R(0) ? +dotl[mw] : +dotr[mw];
+        if constexpr (sizeof(R) == 4) {
+            const float r = d * __builtin_amdgcn_rcpf(rmax(wn, 1.17549435e-38f));
+            phi[mw] = STD ? rmax(0.0f, rmin(rmin(mad(0.5f, r, 0.5f), 2.0f), 2.0f * r)) : philim<float>(mth, r);
+        } else {
+            const R rr = dv(d, wn);
+            phi[mw] = wave_nonzero(wn) ? philim<R>(mth, rr) : R(1);
+        }
+    }
+    R c[MW];
+#pragma unroll
+    for (int mw = 0; mw < MW; mw++) {
+        const R as = fabs(s[mw]);
+        if constexpr (sizeof(R) == 4) c[mw] = mad(-(as * dtd), as, as) * phi[mw];
+        else c[mw] = as * (R(1) - as * dtd);
+    }
+#pragma unroll
+    for (int m = 0; m < MEQN; m++) {
+        R sum = R(0);
+#pragma unroll
+        for (int mw = 0; mw < MW; mw++) {
+            if (WZ::at(mw, m)) continue;
+            if constexpr (sizeof(R) == 4) sum = mad(c[mw], wave[mw][m], sum);
+            else sum = sum + c[mw] * (phi[mw] * wave[mw][m]);
+        }
+        cqxx[m] = sum;
+    }
+}
+
+// Any value: what a skipped stage leaves behind is not read, and must not keep
+// the registers it stands in alive.
+template <typename V, int N>
+__device__ __forceinline__ void unset(V (&v)[N]) {
+#pragma unroll
+    for (int k = 0; k < N; k++) v[k] = __builtin_nondeterministic_value(v[k]);
+}
+
+// Register update (reg_add of the tile kernel).  Each register has one writer
+// per launch, so that adding to it (ACC, subcycling) needs no old value back: an
+// add done in the L2, with the same rounding, that nothing waits for.
+template <int ACC>
+__device__ __forceinline__ void reg_put(double* r, double v) {
+    if constexpr (ACC) unsafeAtomicAdd(r, v);
+    else *r = 0.0 + v;
+}
+
+// a b + c in one rounding: the FP32-bulk form's FP64 state update
+__device__ __forceinline__ double fmad64(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// x, computed where it stands: an address used in a rare branch of the row loop
+// must not be hoisted out of it into registers that live through every row.
+__device__ __forceinline__ int opaque(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
+// Waves per SIMD the register allocation aims for.  The FP64 Euler form keeps
+// more than the 256 registers of two waves and gets all 512; the others run
+// with two waves and nothing in scratch (three waves of 168 registers spill,
+// and a reload waits for the stores in flight: shallow water FP32 on 11,296
+// patches of 32 x 32 0.412 ms with 3 waves and 6 spills against 0.331 with 2).
+template <class RP, typename R>
+constexpr int strip_waves_per_eu() {
+    return RP::MEQN * RP::MWAVES == 1 ? 3 : (sizeof(R) == 8 && RP::MEQN * RP::MWAVES > 9) ? 1 : 2;
+}
+
+template <class RP, typename R, bool FLUXFORM, int KEEP, bool STD>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(strip_waves_per_eu<RP, R>())))
+step_strips(StepArgs a, StripShape sh) {
+#pragma clang fp contract(off)
+    constexpr int MEQN = RP::MEQN, MW = RP::MWAVES, MAUX = RP::MAUX, NROE = RP::NROE;
+    constexpr int NC = cell_values<RP>::N, NCD = NC > 0 ? NC : 1;
+    constexpr int MAD = MAUX > 0 ? MAUX : 1;
+    constexpr bool REGS = KEEP > 0;
+    constexpr int ACC = KEEP == 2;        // registers add up over substeps
+    // Steps per round of the row loop: two copies of the step change their
+    // results over by name instead of by register moves, but only where both
+    // give the same bits.
+    constexpr int U = sizeof(R) == 4 && explicit_fma<RP>::value ? 2 : 1;
+    // FP32 with a linear rpt2: the factor dt / (2 dx) goes on asdq
+    constexpr bool PRE = sizeof(R) == 4 && rpt2_linear<RP>::value;
+    using WZ1 = wave_zeros<RP, 1>;
+    using WZ2 = wave_zeros<RP, 2>;
+
+    const int mx = a.mx, my = a.my, mbc = a.mbc;
+    const int nxp = mx + 2 * mbc;
+    const long long plane = (long long) nxp * (my + 2 * mbc);
+    const int H = sh.H;
+    const int lane = threadIdx.x & 63;
+
+    // Workgroups are dispatched round-robin over the 8 XCDs: each XCD takes one
+    // contiguous run of waves, so that neighbouring strips find the cells they
+    // share in the same L2.  (The grid is a multiple of 8.)
+    const int blk = (int) (blockIdx.x & 7) * (int) (gridDim.x >> 3) + (int) (blockIdx.x >> 3);
+    const int wid = blk * (int) (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int pw = wid / sh.nsy, ty = wid - pw * sh.nsy;
+    const int round = pw / sh.waves, wk = pw - round * sh.waves;
+    const int patch0 = round * sh.patches;
+    if (patch0 >= a.nwork) return;        // (the whole wave)
+    // the lane's segment, staged column kp in it and patch; lanes without a
+    // column repeat another one and write nothing
+    unsigned sg = 0;
+    if (sh.waves > StripShape::WAVES) {
+        const int most = StripShape::LANES - StripShape::HALO;
+        sg = strip_segment(0, min(most, mx - wk * most), 0, wk * most);
+    } else {
+#pragma unroll
+        for (int k = 0; k < StripShape::SEGS; k++) {
+            unsigned w = 0;
+#pragma unroll
+            for (int v = 0; v < StripShape::WAVES; v++) w = wk == v ? sh.seg[v][k] : w;
+            if (k == 0 || (w && lane >= (int) (w & 63))) sg = w;
+        }
+    }
+    const int W = (sg >> 6) & 63;
+    int kp = lane - (int) (sg & 63);
+    int pi = patch0 + (int) ((sg >> 12) & 15);
+    const bool act = kp < W + 4 && pi < a.nwork;
+    kp = min(kp, W + 3);
+    pi = min(pi, a.nwork - 1);
+    const int slot = a.work[pi];
+    const int i0 = 1 + (int) (sg >> 16), j0 = 1 + min(ty * H, my - H);
+    const int i = i0 - 2 + kp;                       // the lane's patch column (1-based)
+    const bool incol = act && kp >= 2 && kp <= W + 1;   // an interior column of the strip
+    const bool ifx = act && kp >= 2 && kp <= W + 2;     // x-interfaces (left of the lane's cell) of the strip
+    const bool ify = act && kp >= 1 && kp <= W + 2;     // columns whose y-interfaces count for the Courant number
+
+    const double dt = a.dtscale ? a.dt * a.dtscale[slot] : a.dt;
+    const double dxs = a.dxs[slot], dys = a.dys[slot];
+    const double dtdx64 = dt / dxs, dtdy64 = dt / dys;
+    const R dtdx = (R) dtdx64, dtdy = (R) dtdy64;
+
+    // offsets of the lane's column to a same-size neighbour's cells, for rows
+    // below, in and above the patch (StepArgs::pull)
+    int dlo = 0, dmid = 0, dhi = 0;
+    if (a.pull) {
+        const int* __restrict__ pt = a.pull + 8 * (long long) slot;
+        const bool gx = i < 1 || i > mx;
+        const int hx = i > mx ? 1 : 0;
+        dmid = gx ? pt[hx] : 0;
+        dlo = gx ? pt[4 + hx] : pt[2];
+        dhi = gx ? pt[6 + hx] : pt[3];
+    }
+    // deferred fix-up: whether the lane's column lies on a corrected x-face, and
+    // that face's increments (of row j at qx[m my + j])
+    bool fix = false;
+    const double* qx = nullptr;
+    if (a.qcorr && (i == 1 || i == mx)) {
+        const int face = i == 1 ? 0 : 1;
+        fix = (a.cmask[slot] >> face) & 1;
+        qx = a.qcorr + (long long) slot * a.cstride + face * MEQN * my - 1;
+    }
+    const double* qp = a.qsrc + (long long) slot * a.pstride + (long long) (j0 + mbc - 3) * nxp + (i + mbc - 1);
+    const double* ap = MAUX > 0 ? a.aux + (long long) slot * a.astride + (long long) (j0 + mbc - 3) * nxp + (i + mbc - 1)
+                                : nullptr;
+    double* qo = a.qdst + (long long) slot * a.pstride + (long long) (j0 + mbc - 1) * nxp + (i + mbc - 1);
+
+    // time-sync registers: whether the lane's x-interface lies on a patch face,
+    // whether its cell is the first interior or first ghost cell of one, and that
+    // face's registers from the strip's first row on; rows of an overlapping last
+    // strip that the strip before it owns are left to it.  What only the patch's
+    // first and last rows need is looked up there.
+    const int own_y = ty * H + 1 - j0;
+    const bool bottom = j0 == 1, top = j0 + H - 1 == my;
+    const bool onface = act && ((kp == 2 && i == 1) || (kp == W + 2 && i == mx + 1));
+    const bool byface = onface || (act && ((kp == 1 && i == 0) || (kp == W + 1 && i == mx)));
+    const double dtdy_el = dt * dys;
+    double* rx = nullptr;
+    if constexpr (REGS) rx = a.reg + (long long) slot * a.rstride + (i <= 1 ? 0 : 4 * MEQN * mx) + j0 - 1;
+    // the registers of y-face `face`, kind 0, at the lane's column; length of the face times dt
+    auto yreg = [&](int face, double* el) __attribute__((always_inline)) {
+        const int sl = opaque(slot);
+        *el = (a.dtscale ? a.dt * a.dtscale[sl] : a.dt) * a.dxs[sl];
+        return a.reg + (long long) sl * a.rstride + face * 4 * MEQN * mx + i - 1;
+    };
+
+    double pq[MEQN], pv[MEQN];            // the row in flight, and the pending fix-up of its x-face cells
+    R pa[MAD];
+    double qr[4][MEQN];                   // rows A (n - 2), B (n - 1), C (n) and N (n + 1), in turn
+    R ar[4][MAD];
+    int j = j0 - 2;                       // patch row of the row in flight
+
+    // What one step leaves to the next, in two copies that steps of even and
+    // odd n write in turn: per-cell values of the Riemann solver for row C
+    // (x and y); the y-interface between rows B and C as solved, with its waves'
+    // products with those of the interface below; the transverse parts of row B
+    // at its upper face and its normal x-flux parts; of the y-interface between
+    // rows A and B the transverse parts it sends up and its flux.
+    R cx[2][NCD], cy[2][NCD];
+    R wv[2][MW][MEQN], sv[2][MW], am[2][MEQN], apq[2][MEQN], ro[2][NROE], dl[2][MW];
+    R tu[2][MEQN], fxm[2][MEQN], fxp[2][MEQN];
+    R gPd[2][MEQN], gPu[2][MEQN], gpl[2][MEQN];
+    double G[2][MEQN];
+    R smaxx = R(0), smaxy = R(0);         // largest |s| of every interface the lane solves
+    const R halfx = R(0.5) * dtdx, halfy = R(0.5) * dtdy;
+
+
+    // Step n: row C is row n.  Every stage is entered as the rows it needs are
+    // there, from the same code in every row, so that a flux at the seam of two
+    // strips has the same bits in both.  Two steps per round: what they leave to
+    // each other changes places by name instead of by moves.
+#pragma unroll 1
+    for (int n0 = -1; n0 <= H + 3; n0 += U) {
+#pragma unroll
+        for (int e = 0; e < U; e++) {
+            const int n = n0 + e;
+            const int P = e, O = 1 - e, A = e, B = e + 1, C = e + 2, N = (e + 3) & 3;
+            if (U > 1 && n > H + 3) break;
+            // ---- row n + 1 under way ----
+            if (n < H + 3) {
+                const double* p = qp + (j < 1 ? dlo : j > my ? dhi : dmid);
+#pragma unroll
+                for (int m = 0; m < MEQN; m++) pq[m] = p[m * plane];
+                if (fix && j >= 1 && j <= my) {
+#pragma unroll
+                    for (int m = 0; m < MEQN; m++) pv[m] = qx[m * my + j];
+                }
+                if constexpr (MAUX > 0) {
+#pragma unroll
+                    for (int m = 0; m < MAUX; m++) pa[m] = (R) ap[m * plane];
+                    ap += nxp;
+                }
+                qp += nxp;
+            }
+            if constexpr (REGS && !FLUXFORM) {
+                // FP64 form: conservative flux of the pre-step state at the first
+                // interior and first ghost cell of every patch edge
+                // (clawpack46_time_sync.f:58-147)
+                double ac[MAD], fl[MEQN];
+#pragma unroll
+                for (int m = 0; m < MAD; m++) ac[m] = MAUX > 0 ? (double) ar[C][m] : 0.0;
+                const int b = n - 2;          // interior row of the strip
+                if (byface && b >= own_y && b >= 0 && b < H) {
+                    RP::template consflux<1>(qr[C], ac, a.pp, fl);
+                    double* r = rx + b + (i == 0 || i == mx + 1 ? REG_EFOUT : REG_EFIN) * MEQN * mx;
+#pragma unroll
+                    for (int m = 0; m < MEQN; m++) reg_put<ACC>(r + m * mx, dtdy_el * fl[m]);
+                }
+                const bool below = bottom && (b == -1 || b == 0), above = top && (b == H - 1 || b == H);
+                if ((below || above) && incol) {
+                    RP::template consflux<2>(qr[C], ac, a.pp, fl);
+                    double el;
+                    // (a strip of one row has both faces, one after the other)
+                    if (below) {
+                        double* r = yreg(2, &el) + (b < 0 ? REG_EFOUT : REG_EFIN) * MEQN * mx;
+#pragma unroll
+                        for (int m = 0; m < MEQN; m++) reg_put<ACC>(r + m * mx, el * fl[m]);
+                    }
+                    if (above) {
+                        double* r = yreg(3, &el) + (b == H ? REG_EFOUT : REG_EFIN) * MEQN * mx;
+#pragma unroll
+                        for (int m = 0; m < MEQN; m++) reg_put<ACC>(r + m * mx, el * fl[m]);
+                    }
+                }
+            }
+            if constexpr (NC > 0) {
+                R q[MEQN];
+#pragma unroll
+                for (int m = 0; m < MEQN; m++) q[m] = (R) qr[C][m];
+                RP::template cell<1>(q, a.pp, cx[P]);
+                RP::template cell<2>(q, a.pp, cy[P]);
+            }
+
+            // ---- x sweep of row B (n - 1) ----
+            R gt[MEQN], gm[MEQN];             // of the y-face between rows A and B: transverse part, flux part
+            if (n >= 2) {
+                R qL[MEQN], qR[MEQN], auxL[MAD];
+#pragma unroll
+                for (int m = 0; m < MEQN; m++) { qR[m] = (R) qr[B][m]; qL[m] = prev_lane(qR[m]); }
+#pragma unroll
+                for (int m = 0; m < MAD; m++) auxL[m] = MAUX > 0 ? prev_lane(ar[B][m]) : R(0);
+                R w[MW][MEQN], s[MW], amdq[MEQN], apdq[MEQN], roe[NROE];
+                if constexpr (NC > 0) {
+                    R cL[NCD];
+#pragma unroll
+                    for (int c = 0; c < NC; c++) cL[c] = prev_lane(cx[O][c]);
+                    RP::template rpn2c<1>(qL, qR, cL, cx[O], auxL, ar[B], a.pp, w, s, amdq, apdq, roe);
+                } else {
+                    RP::template rpn2<1>(qL, qR, auxL, ar[B], a.pp, w, s, amdq, apdq, roe);
+                }
+#pragma unroll
+                for (int mw = 0; mw < MW; mw++) smaxx = fmax(smaxx, fabs(s[mw]));
+                R cq[MEQN];
+#pragma unroll
+                for (int m = 0; m < MEQN; m++) cq[m] = R(0);
+                if (STD || a.order2) {
+                    R dotl[MW], dotr[MW];
+#pragma unroll
+                    for (int mw = 0; mw < MW; mw++) {
+                        R d = R(0);
+#pragma unroll
+                        for (int m = 0; m < MEQN; m++) {
+                            if (WZ1::at(mw, m)) continue;
+                            const R wl = prev_lane(w[mw][m]);
+                            d = mad(wl, w[mw][m], d);
+                        }
+                        dotl[mw] = d;
+                        dotr[mw] = next_lane(d);
+                    }
+                    limited_correction<RP, R, 1, STD>(a, w, s, dotl, dotr, dtdx, cq);
+                }
+#pragma unroll
+                for (int m = 0; m < MEQN; m++) {
+                    fxm[P][m] = mad(R(0.5), cq[m], zadd(amdq[m]));
+                    if constexpr (!FLUXFORM) fxp[P][m] = mad(R(0.5), cq[m], zsub(apdq[m]));
+                }
+                if (STD || a.transverse) {
+                    if (STD || (a.order2 && a.transverse == 2)) {
+#pragma unroll
+                        for (int m = 0; m < MEQN; m++) { amdq[m] = amdq[m] + cq[m]; apdq[m] = apdq[m] - cq[m]; }
+                    }
+                    if constexpr (PRE) {
+#pragma unroll
+                        for (int m = 0; m < MEQN; m++) { amdq[m] = halfx * amdq[m]; apdq[m] = halfx * apdq[m]; }
+                    }
+                    R bmA[MEQN], bpA[MEQN], bmP[MEQN], bpP[MEQN];
+                    R a1[MAD], a3[MAD];
+#pragma unroll
+                    for (int m = 0; m < MAD; m++) {
+                        a1[m] = MAUX > 0 ? prev_lane(ar[A][m]) : R(0);
+                        a3[m] = MAUX > 0 ? prev_lane(ar[C][m]) : R(0);
+                    }
+                    RP::template rpt2<1>(roe, amdq, a1, auxL, a3, a.pp, bmA, bpA);
+                    RP::template rpt2<1>(roe, apdq, ar[A], ar[B], ar[C], a.pp, bmP, bpP);
+#pragma unroll
+                    for (int m = 0; m < MEQN; m++) {
+                        const R gAd = PRE ? bmA[m] : halfx * bmA[m], gAu = PRE ? bpA[m] : halfx * bpA[m];
+                        const R gBd = PRE ? bmP[m] : halfx * bmP[m], gBu = PRE ? bpP[m] : halfx * bpP[m];
+                        gt[m] = zadd(tu[O][m]) + (zsub(next_lane(gAd)) - gBd);
+                        tu[P][m] = zsub(next_lane(gAu)) - gBu;
+                    }
+                } else {
+#pragma unroll
+                    for (int m = 0; m < MEQN; m++) { gt[m] = R(0); tu[P][m] = R(0); }
+                }
+            } else {
+                unset(gt); unset(tu[P]); unset(fxm[P]); unset(fxp[P]);
+            }
+
+            // ---- the y-interface between rows B and C, as solved ----
+            if (n >= 1) {
+                R qL[MEQN], qR[MEQN];
+#pragma unroll
+                for (int m = 0; m < MEQN; m++) { qL[m] = (R) qr[B][m]; qR[m] = (R) qr[C][m]; }
+                if constexpr (NC > 0)
+                    RP::template rpn2c<2>(qL, qR, cy[O], cy[P], ar[B], ar[C], a.pp, wv[P], sv[P], am[P], apq[P], ro[P]);
+                else
+                    RP::template rpn2<2>(qL, qR, ar[B], ar[C], a.pp, wv[P], sv[P], am[P], apq[P], ro[P]);
+#pragma unroll
+                for (int mw = 0; mw < MW; mw++) {
+                    R d = R(0);
+#pragma unroll
+                    for (int m = 0; m < MEQN; m++)
+                        if (!WZ2::at(mw, m)) d = mad(wv[O][mw][m], wv[P][mw][m], d);
+                    dl[P][mw] = d;
+                }
+            } else {
+#pragma unroll
+                for (int mw = 0; mw < MW; mw++) unset(wv[P][mw]);
+                unset(sv[P]); unset(am[P]); unset(apq[P]); unset(ro[P]); unset(dl[P]);
+            }
+
+            double out[MEQN], Fx[MEQN];       // row A's new values; x-flux left of the cell
+            R fm[MEQN], fp[MEQN];
+            if (n >= 3) {
+                // ---- the y-interface between rows A and B: limiter, flux, transverse ----
+                R so[MW];
+                if constexpr (roe_speeds<RP>::value) {
+                    RP::speeds(ro[O], so);
+                } else {
+#pragma unroll
+                    for (int mw = 0; mw < MW; mw++) so[mw] = sv[O][mw];
+                }
+#pragma unroll
+                for (int mw = 0; mw < MW; mw++) smaxy = fmax(smaxy, fabs(so[mw]));
+                R cq[MEQN];
+#pragma unroll
+                for (int m = 0; m < MEQN; m++) cq[m] = R(0);
+                if (STD || a.order2) limited_correction<RP, R, 2, STD>(a, wv[O], so, dl[O], dl[P], dtdy, cq);
+#pragma unroll
+                for (int m = 0; m < MEQN; m++) {
+                    gm[m] = gt[m] + mad(R(0.5), cq[m], zadd(am[O][m]));
+                    if constexpr (!FLUXFORM) gpl[P][m] = gt[m] + mad(R(0.5), cq[m], zsub(apq[O][m]));
+                }
+                R nAd[MEQN], nAu[MEQN];
+                if (STD || a.transverse) {
+                    R amdq[MEQN], apdq[MEQN];
+#pragma unroll
+                    for (int m = 0; m < MEQN; m++) { amdq[m] = am[O][m]; apdq[m] = apq[O][m]; }
+                    if (STD || (a.order2 && a.transverse == 2)) {
+#pragma unroll
+                        for (int m = 0; m < MEQN; m++) { amdq[m] = amdq[m] + cq[m]; apdq[m] = apdq[m] - cq[m]; }
+                    }
+                    if constexpr (PRE) {
+#pragma unroll
+                        for (int m = 0; m < MEQN; m++) { amdq[m] = halfy * amdq[m]; apdq[m] = halfy * apdq[m]; }
+                    }
+                    R a1[MAD], a3[MAD];
+#pragma unroll
+                    for (int m = 0; m < MAD; m++) {
+                        a1[m] = MAUX > 0 ? prev_lane(ar[A][m]) : R(0);
+                        a3[m] = MAUX > 0 ? next_lane(ar[A][m]) : R(0);
+                    }
+                    RP::template rpt2<2>(ro[O], amdq, a1, ar[A], a3, a.pp, nAd, nAu);
+#pragma unroll
+                    for (int m = 0; m < MAD; m++) {
+                        a1[m] = MAUX > 0 ? prev_lane(ar[B][m]) : R(0);
+                        a3[m] = MAUX > 0 ? next_lane(ar[B][m]) : R(0);
+                    }
+                    RP::template rpt2<2>(ro[O], apdq, a1, ar[B], a3, a.pp, gPd[P], gPu[P]);
+                    if constexpr (!PRE) {
+#pragma unroll
+                        for (int m = 0; m < MEQN; m++) {
+                            nAd[m] = halfy * nAd[m]; nAu[m] = halfy * nAu[m];
+                            gPd[P][m] = halfy * gPd[P][m]; gPu[P][m] = halfy * gPu[P][m];
+                        }
+                    }
+                } else {
+#pragma unroll
+                    for (int m = 0; m < MEQN; m++) nAd[m] = nAu[m] = gPd[P][m] = gPu[P][m] = R(0);
+                }
+                // ---- row A: x-fluxes with the transverse parts of its two y-interfaces, update ----
+#pragma unroll
+                for (int m = 0; m < MEQN; m++) {
+                    const R t1 = zsub(nAd[m]) - gPd[O][m];      // into the x-face left of the cell
+                    const R t2 = zsub(nAu[m]) - gPu[O][m];      // into the one right of it
+                    const R t2l = prev_lane(t2);
+                    fm[m] = (zadd(fxm[O][m]) + t2l) + t1;
+                    if constexpr (!FLUXFORM) fp[m] = (zadd(fxp[O][m]) + t2l) + t1;
+                }
+                if constexpr (FLUXFORM) {
+                    // FP64 fluxes f and g of the row's cells, each evaluated once: the
+                    // flux right of a cell is its f plus the next interface's fm, the
+                    // one above it its g plus gm, and each is the next cell's too
+                    double f[MEQN], g[MEQN], ac[MAD];
+#pragma unroll
+                    for (int m = 0; m < MAD; m++) ac[m] = MAUX > 0 ? (double) ar[A][m] : 0.0;
+                    RP::fluxes(qr[A], ac, a.pp, f, g);
+#pragma unroll
+                    for (int m = 0; m < MEQN; m++) {
+                        G[P][m] = g[m] + (double) gm[m];
+                        const double Fr = f[m] + (double) next_lane(fm[m]);
+                        Fx[m] = prev_lane(Fr);
+                        out[m] = fmad64(-dtdy64, G[P][m] - G[O][m], fmad64(-dtdx64, Fr - Fx[m], qr[A][m]));
+                    }
+                } else {
+#pragma unroll
+                    for (int m = 0; m < MEQN; m++) {
+                        const R Dx = next_lane(fm[m]) - fp[m];
+                        const R Dy = gm[m] - gpl[O][m];
+                        if constexpr (sizeof(R) == sizeof(double)) out[m] = (qr[A][m] - dtdx * Dx) - dtdy * Dy;
+                        else out[m] = fmad64(-dtdy64, (double) Dy, fmad64(-dtdx64, (double) Dx, qr[A][m]));
+                    }
+                }
+            } else {
+                unset(gPd[P]); unset(gPu[P]); unset(gpl[P]); unset(G[P]);
+                unset(out); unset(Fx); unset(gm); unset(fm); unset(fp);
+            }
+
+            // ---- the row in flight into N, with the pending fix-up of its edge
+            // cells in the reference's order (same-size faces before coarse/fine
+            // ones).  The wait for the row is here and not where it is first used:
+            // the stores of the row just updated come in between, and a wait after
+            // them would be for them too ----
+#pragma unroll
+            for (int m = 0; m < MEQN; m++) {
+                asm volatile("" : "+v"(pq[m]));
+                qr[N][m] = pq[m];
+            }
+#pragma unroll
+            for (int m = 0; m < MAUX; m++) {
+                asm volatile("" : "+v"(pa[m]));
+                ar[N][m] = pa[m];
+            }
+            if (a.qcorr) {
+                const bool onx = fix && j >= 1 && j <= my;
+                bool done = false;
+                if ((j == 1 || j == my) && i >= 1 && i <= mx) {
+                    const int sl = opaque(slot), fy = j == 1 ? 2 : 3, mask = a.cmask[sl];
+                    if ((mask >> fy) & 1) {
+                        const double* qy = a.qcorr + (long long) sl * a.cstride + fy * MEQN * mx + i - 1;
+                        const bool yfirst = !onx || sync_y_first(mask, i == 1 ? 0 : 1, fy);
+                        done = true;
+#pragma unroll
+                        for (int m = 0; m < MEQN; m++) {
+                            const double w = qy[m * mx], v = onx ? pv[m] : 0.0;
+                            double q = qr[N][m];
+                            if (yfirst) q = q + w;
+                            if (onx) q = q + v;
+                            if (!yfirst) q = q + w;
+                            qr[N][m] = q;
+                        }
+                    }
+                }
+                if (onx && !done) {
+#pragma unroll
+                    for (int m = 0; m < MEQN; m++) qr[N][m] = qr[N][m] + pv[m];
+                }
+            }
+
+            if (n >= 3) {
+                if constexpr (REGS) {
+                    // the y-flux (FP64: both flux parts) through the patch's bottom and top edges
+                    const int face = bottom && n == 3 ? 2 : top && n == H + 3 ? 3 : -1;
+                    if (face >= 0 && incol) {
+                        double el, *r = yreg(face, &el);
+#pragma unroll
+                        for (int m = 0; m < MEQN; m++) {
+                            if constexpr (FLUXFORM) {
+                                reg_put<ACC>(r + (REG_EFIN * MEQN + m) * mx, el * G[P][m]);
+                            } else {
+                                reg_put<ACC>(r + (REG_FM * MEQN + m) * mx, el * (double) gm[m]);
+                                reg_put<ACC>(r + (REG_FP * MEQN + m) * mx, -(el * (double) gpl[P][m]));
+                            }
+                        }
+                    }
+                }
+            }
+            if (n >= 4) {
+                // ---- the strip's interior row n - 4 out ----
+                if (incol) {
+#pragma unroll
+                    for (int m = 0; m < MEQN; m++) qo[m * plane] = out[m];
+                }
+                if constexpr (REGS) {
+                    const int b = n - 4;
+                    if (onface && b >= own_y) {
+                        double* r = rx + b;
+#pragma unroll
+                        for (int m = 0; m < MEQN; m++) {
+                            if constexpr (FLUXFORM) {
+                                reg_put<ACC>(r + (REG_EFIN * MEQN + m) * mx, dtdy_el * Fx[m]);
+                            } else {
+                                reg_put<ACC>(r + (REG_FM * MEQN + m) * mx, dtdy_el * (double) fm[m]);
+                                reg_put<ACC>(r + (REG_FP * MEQN + m) * mx, -(dtdy_el * (double) fp[m]));
+                            }
+                        }
+                    }
+                }
+                qo += nxp;
+            }
+            j++;
+        }
+        if constexpr (U == 2) {
+#pragma unroll
+            for (int m = 0; m < MEQN; m++) {
+                const double t = qr[0][m];
+                qr[0][m] = qr[2][m];
+                qr[1][m] = qr[3][m];
+                qr[2][m] = t;
+            }
+#pragma unroll
+            for (int m = 0; m < MAUX; m++) {
+                const R t = ar[0][m];
+                ar[0][m] = ar[2][m];
+                ar[1][m] = ar[3][m];
+                ar[2][m] = t;
+            }
+        } else {
+#pragma unroll
+            for (int m = 0; m < MEQN; m++) {
+                qr[0][m] = qr[1][m]; qr[1][m] = qr[2][m]; qr[2][m] = qr[3][m];
+                am[1][m] = am[0][m]; apq[1][m] = apq[0][m];
+                tu[1][m] = tu[0][m]; fxm[1][m] = fxm[0][m]; fxp[1][m] = fxp[0][m];
+                gPd[1][m] = gPd[0][m]; gPu[1][m] = gPu[0][m]; gpl[1][m] = gpl[0][m];
+                G[1][m] = G[0][m];
+            }
+#pragma unroll
+            for (int m = 0; m < MAUX; m++) { ar[0][m] = ar[1][m]; ar[1][m] = ar[2][m]; ar[2][m] = ar[3][m]; }
+#pragma unroll
+            for (int m = 0; m < NCD; m++) { cx[1][m] = cx[0][m]; cy[1][m] = cy[0][m]; }
+#pragma unroll
+            for (int mw = 0; mw < MW; mw++) {
+                sv[1][mw] = sv[0][mw]; dl[1][mw] = dl[0][mw];
+#pragma unroll
+                for (int m = 0; m < MEQN; m++) wv[1][mw][m] = wv[0][mw][m];
+            }
+#pragma unroll
+            for (int m = 0; m < NROE; m++) ro[1][m] = ro[0][m];
+        }
+    }
+
+    // ---- CFL: wave64 max over the lanes' interfaces, one atomic per wave ----
+    double cfl = fmax(ifx ? dtdx64 * (double) smaxx : 0.0, ify ? dtdy64 * (double) smaxy : 0.0);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) cfl = fmax(cfl, __shfl_xor(cfl, off, 64));
+    if (lane == 0 && cfl > 0.0)
+        atomicMax(a.cfl + (wid & (CFL_WORDS - 1)) * CFL_STRIDE, (unsigned long long) __double_as_longlong(cfl));
+}
+
+}  // namespace hipclaw

@@ -58,8 +58,11 @@ typedef struct hipclaw_config {
     double grav;     /* shallow water */
     double gamma;    /* Euler */
     int tile;        /* cells per tile side (8, 16, 32; at most mx and my); 0 = tuned
-                        default.  A tile that does not divide the patch overlaps its
-                        last tile with the one before */
+                        default.  Solvers with meqn x mwaves > 16 are updated tile by
+                        tile (a tile that does not divide the patch overlaps its last
+                        tile with the one before), the others in strips laid out by
+                        the patch size; for them the tile only says whether one
+                        covers a patch */
     int time_sync;   /* keep flux registers for the conservation fix-up
                         (fclaw_options time-sync, src/fclaw_options.c:110); needs mx == my */
     int subcycle;    /* keep the state before each update and time-interpolated
@@ -267,11 +270,11 @@ int hipclaw_set_dt_scale(hipclaw_state_t *s, const double *scale);
  * for all patches at once, as save_time_step / restore_time_step of the run
  * loop use them to reject a step whose Courant number exceeds max_cfl
  * (src/fclaw2d_run.c:47-80).  Restoring without a saved state, or after a
- * regrid (the slots changed), is an error.  With two slabs (tile smaller
- * than the patch) the saved state stays in its slab without a copy while
+ * regrid (the slots changed), is an error.  With two slabs the saved state stays in its slab without a copy while
  * only a one-step advance runs (it writes the other slab); any other call
  * that may write that slab copies it first.  A restore may so make the
- * other slab current: a graph captured before then refuses to replay. */
+ * other slab current: a graph captured before then refuses to replay, or, where
+ * a tile covers a patch, first copies the state to the slab it starts from. */
 int hipclaw_save_step(hipclaw_state_t *s);
 int hipclaw_restore_step(hipclaw_state_t *s);
 
@@ -292,11 +295,9 @@ int hipclaw_restore_step(hipclaw_state_t *s);
 int hipclaw_set_ghost_layout(hipclaw_state_t *s, int layout);
 int hipclaw_ghost_layout(const hipclaw_state_t *s);
 
-/* Waves per workgroup of the 16 x 16 update tile: 2, 3 or 4 (0 = the
- * default: 2 for the FP32-bulk form, 4 for FP64).  A sweep has six row
- * groups: two waves take three each, three take two, four take two, two, one
- * and one; fewer waves per workgroup hold fewer staging registers, and more
- * workgroups share a CU when the tile's LDS allows.
+/* Waves per workgroup of the update, for the 16 x 16 tile: 2, 3 or 4 (0 = the
+ * default: 1; for solvers with meqn x mwaves > 16, whose waves share a tile in
+ * LDS, 2 in the FP32-bulk form and 4 in FP64).
  * hipclaw_waves returns the waves the next update uses (0 for tiles without
  * a choice).  No counterpart in the reference (128 threads per patch). */
 int hipclaw_set_waves(hipclaw_state_t *s, int waves);
