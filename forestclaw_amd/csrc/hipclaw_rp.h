@@ -61,6 +61,14 @@ __device__ __forceinline__ double mad(double a, double b, double c) {
 }
 __device__ __forceinline__ float mad(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
+// The next term a b of an unrolled sum, which its first term starts.
+template <typename R>
+__device__ __forceinline__ void sum_term(R& sum, R a, R b, bool& first) {
+#pragma clang fp contract(off)
+    sum = first ? R(a * b) : mad(a, b, sum);
+    first = false;
+}
+
 // Division and square root.  FP64 keeps IEEE-correct operations (the parity
 // form); the FP32-bulk form uses the hardware reciprocal and square root
 // (v_rcp_f32, v_sqrt_f32, 1 ulp), whose error is far below the form's
@@ -303,9 +311,10 @@ struct RPShallow {
 #pragma unroll
         for (int m = 0; m < 3; m++) {
             R df = R(0);
+            bool first = true;
 #pragma unroll
             for (int mw = 0; mw < 3; mw++)
-                if (!wave_zero<IXY>(mw, m)) df = df + s[mw] * wave[mw][m];
+                if (!wave_zero<IXY>(mw, m)) sum_term(df, s[mw], wave[mw][m], first);
             apdq[m] = df - amdq[m];
         }
     }
@@ -343,9 +352,9 @@ struct RPShallow {
         wb[2][0] = a3;   wb[2][mu] = a3 * u; wb[2][mv] = a3 * (v + a); sb[2] = v + a;
 #pragma unroll
         for (int m = 0; m < 3; m++) {
-            R m_ = R(0), p_ = R(0);
+            R m_ = rmin(sb[0], R(0)) * wb[0][m], p_ = rmax(sb[0], R(0)) * wb[0][m];
 #pragma unroll
-            for (int mw = 0; mw < 3; mw++) {
+            for (int mw = 1; mw < 3; mw++) {
                 if (mw == 1 && m != mu) continue;   // wb[1][0], wb[1][mv] are zero
                 m_ = m_ + rmin(sb[mw], R(0)) * wb[mw][m];
                 p_ = p_ + rmax(sb[mw], R(0)) * wb[mw][m];
@@ -567,9 +576,10 @@ struct RPEuler {
 #pragma unroll
         for (int m = 0; m < 4; m++) {
             R df = R(0);
+            bool first = true;
 #pragma unroll
             for (int mw = 0; mw < 4; mw++)
-                if (!wave_zero<IXY>(mw, m)) df = mad(s[mw], wave[mw][m], df);
+                if (!wave_zero<IXY>(mw, m)) sum_term(df, s[mw], wave[mw][m], first);
             apdq[m] = df - amdq[m];
         }
     }
@@ -615,9 +625,9 @@ struct RPEuler {
         wb[2][3] = a4 * (enth + v * a); sb[2] = v + a;
 #pragma unroll
         for (int m = 0; m < 4; m++) {
-            R m_ = R(0), p_ = R(0);
+            R m_ = rmin(sb[0], R(0)) * wb[0][m], p_ = rmax(sb[0], R(0)) * wb[0][m];
 #pragma unroll
-            for (int mw = 0; mw < 3; mw++) {
+            for (int mw = 1; mw < 3; mw++) {
                 m_ = m_ + rmin(sb[mw], R(0)) * wb[mw][m];
                 p_ = p_ + rmax(sb[mw], R(0)) * wb[mw][m];
             }

@@ -13,7 +13,12 @@
 //   * updates and stores row n - 2.
 //
 // Every sum is taken in the order step_tiles takes it, so the FP64 form gives
-// the same bits.
+// the same bits.  Sums do not start from a zero, which the reference's do and
+// which only turns a sum of -0 into +0: the two flux parts fm and gm whose
+// differences enter the update keep theirs (zadd), so that no difference is -0
+// where the reference's is +0, and no other use of a sum tells the zeros apart
+// (60 fewer FP64 additions per row for shallow water, 80 for Euler: batched
+// 24 x 20 shallow water 138 -> 133 us, dam break 255 -> 248 us per step).
 #pragma once
 
 #include <type_traits>
@@ -43,9 +48,10 @@ __device__ __forceinline__ void limited_correction(const StepArgs& a, const R wa
         const int mth = STD ? 4 : a.mthlim[mw];
         if (mth == 0) continue;
         R wn = R(0);
+        bool first = true;
 #pragma unroll
         for (int m = 0; m < MEQN; m++)
-            if (!WZ::at(mw, m)) wn = mad(wave[mw][m], wave[mw][m], wn);
+            if (!WZ::at(mw, m)) sum_term(wn, wave[mw][m], wave[mw][m], first);
         const R d = s[mw] > R(0) ? +dotl[mw] : +dotr[mw];
         if constexpr (sizeof(R) == 4) {
             const float r = d * __builtin_amdgcn_rcpf(rmax(wn, 1.17549435e-38f));
@@ -65,11 +71,12 @@ __device__ __forceinline__ void limited_correction(const StepArgs& a, const R wa
 #pragma unroll
     for (int m = 0; m < MEQN; m++) {
         R sum = R(0);
+        bool first = true;
 #pragma unroll
         for (int mw = 0; mw < MW; mw++) {
             if (WZ::at(mw, m)) continue;
-            if constexpr (sizeof(R) == 4) sum = mad(c[mw], wave[mw][m], sum);
-            else sum = sum + c[mw] * (phi[mw] * wave[mw][m]);
+            if constexpr (sizeof(R) == 4) sum_term(sum, c[mw], wave[mw][m], first);
+            else sum_term(sum, c[mw], phi[mw] * wave[mw][m], first);
         }
         cqxx[m] = sum;
     }
@@ -336,11 +343,12 @@ step_strips(StepArgs a, StripShape sh) {
 #pragma unroll
                     for (int mw = 0; mw < MW; mw++) {
                         R d = R(0);
+                        bool first = true;
 #pragma unroll
                         for (int m = 0; m < MEQN; m++) {
                             if (WZ1::at(mw, m)) continue;
                             const R wl = prev_lane(w[mw][m]);
-                            d = mad(wl, w[mw][m], d);
+                            sum_term(d, wl, w[mw][m], first);
                         }
                         dotl[mw] = d;
                         dotr[mw] = next_lane(d);
@@ -350,7 +358,7 @@ step_strips(StepArgs a, StripShape sh) {
 #pragma unroll
                 for (int m = 0; m < MEQN; m++) {
                     fxm[P][m] = mad(R(0.5), cq[m], zadd(amdq[m]));
-                    if constexpr (!FLUXFORM) fxp[P][m] = mad(R(0.5), cq[m], zsub(apdq[m]));
+                    if constexpr (!FLUXFORM) fxp[P][m] = mad(R(0.5), cq[m], -apdq[m]);
                 }
                 if (STD || a.transverse) {
                     if (STD || (a.order2 && a.transverse == 2)) {
@@ -374,8 +382,8 @@ step_strips(StepArgs a, StripShape sh) {
                     for (int m = 0; m < MEQN; m++) {
                         const R gAd = PRE ? bmA[m] : halfx * bmA[m], gAu = PRE ? bpA[m] : halfx * bpA[m];
                         const R gBd = PRE ? bmP[m] : halfx * bmP[m], gBu = PRE ? bpP[m] : halfx * bpP[m];
-                        gt[m] = zadd(tu[O][m]) + (zsub(next_lane(gAd)) - gBd);
-                        tu[P][m] = zsub(next_lane(gAu)) - gBu;
+                        gt[m] = tu[O][m] + (-next_lane(gAd) - gBd);
+                        tu[P][m] = -next_lane(gAu) - gBu;
                     }
                 } else {
 #pragma unroll
@@ -397,9 +405,10 @@ step_strips(StepArgs a, StripShape sh) {
 #pragma unroll
                 for (int mw = 0; mw < MW; mw++) {
                     R d = R(0);
+                    bool first = true;
 #pragma unroll
                     for (int m = 0; m < MEQN; m++)
-                        if (!WZ2::at(mw, m)) d = mad(wv[O][mw][m], wv[P][mw][m], d);
+                        if (!WZ2::at(mw, m)) sum_term(d, wv[O][mw][m], wv[P][mw][m], first);
                     dl[P][mw] = d;
                 }
             } else {
@@ -428,7 +437,7 @@ step_strips(StepArgs a, StripShape sh) {
 #pragma unroll
                 for (int m = 0; m < MEQN; m++) {
                     gm[m] = gt[m] + mad(R(0.5), cq[m], zadd(am[O][m]));
-                    if constexpr (!FLUXFORM) gpl[P][m] = gt[m] + mad(R(0.5), cq[m], zsub(apq[O][m]));
+                    if constexpr (!FLUXFORM) gpl[P][m] = gt[m] + mad(R(0.5), cq[m], -apq[O][m]);
                 }
                 R nAd[MEQN], nAu[MEQN];
                 if (STD || a.transverse) {
@@ -470,11 +479,11 @@ step_strips(StepArgs a, StripShape sh) {
                 // ---- row A: x-fluxes with the transverse parts of its two y-interfaces, update ----
 #pragma unroll
                 for (int m = 0; m < MEQN; m++) {
-                    const R t1 = zsub(nAd[m]) - gPd[O][m];      // into the x-face left of the cell
-                    const R t2 = zsub(nAu[m]) - gPu[O][m];      // into the one right of it
+                    const R t1 = -nAd[m] - gPd[O][m];      // into the x-face left of the cell
+                    const R t2 = -nAu[m] - gPu[O][m];      // into the one right of it
                     const R t2l = prev_lane(t2);
-                    fm[m] = (zadd(fxm[O][m]) + t2l) + t1;
-                    if constexpr (!FLUXFORM) fp[m] = (zadd(fxp[O][m]) + t2l) + t1;
+                    fm[m] = (fxm[O][m] + t2l) + t1;
+                    if constexpr (!FLUXFORM) fp[m] = (fxp[O][m] + t2l) + t1;
                 }
                 if constexpr (FLUXFORM) {
                     // FP64 fluxes f and g of the row's cells, each evaluated once: the
