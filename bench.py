@@ -59,8 +59,8 @@ def run_form(fa, prob, forest, q0, aux, precision, dt, steps, warmup, tile, use_
     if warmup > 0:
         sv.advance_async(dt, warmup)
     sv.sync()
-    # kernel timing: an eager pass whose update launches carry HIP events bound
-    # to each kernel's own start and end
+    # kernel timing: an eager pass (the update kernels note the device's clock
+    # at their own start and end)
     sv.advance_async(dt, steps)
     sv.sync()
     _, kernel_ms = sv.timing(steps)

@@ -78,12 +78,11 @@ struct SyncProgram {
     bool set = false;         // installed since the last regrid
 };
 
-constexpr size_t CFL_BYTES = sizeof(unsigned long long) * hipclaw::CFL_WORDS * hipclaw::CFL_STRIDE;
+constexpr size_t CFL_BYTES = sizeof(unsigned long long) * hipclaw::CFL_BLOCK;
 
-// The Courant number in the CFL words of a step (StepArgs::cfl), on the host.
-static double largest_cfl(const unsigned long long* words) {
-    unsigned long long bits = 0;
-    for (int k = 0; k < hipclaw::CFL_WORDS; k++) bits = std::max(bits, words[k * hipclaw::CFL_STRIDE]);
+constexpr size_t HSUM_BYTES = sizeof(unsigned long long) * 2 * hipclaw::STEP_SUMS;
+
+static double as_double(unsigned long long bits) {
     double v;
     std::memcpy(&v, &bits, sizeof(v));
     return v;
@@ -105,7 +104,6 @@ struct hipclaw_state {
     int* all_slots = nullptr;
     int* batch_slots = nullptr;
     GhostProgram gp[HIPCLAW_MAX_PROGRAMS];
-    unsigned long long* cfl = nullptr;
     double* mass_buf = nullptr;
     // time synchronisation: flux registers and the per-destination op groups
     double* reg = nullptr;
@@ -142,8 +140,19 @@ struct hipclaw_state {
     hipGraphExec_t gexec = nullptr;
     int graph_steps = 0;
     int graph_cur = 0;            // the slab a captured advance graph starts from
-    // timing of the update kernel inside advance_async
-    bool time_kernels = true;
+    // The steps of an advance write their Courant number and clock words into
+    // STEP_BLOCKS blocks in turn (StepArgs::cfl); the advance's last launch
+    // collects them into hsum, host memory (launch_collect_steps), and leaves
+    // the blocks clear for the next one.  A batch's go behind the advance's, whose
+    // times stay.
+    unsigned long long* cfl = nullptr;
+    unsigned long long* sum = nullptr;
+    unsigned long long* hsum = nullptr;
+    bool cfl_clear = false;       // the blocks and sum are (or will be, in stream order) zero
+    // Timing of the last advance, replay or subcycled advance.  A registered
+    // solver's step kernel need not keep clock words: its launches carry events,
+    // as replays and subcycled advances are enclosed by them.
+    bool by_clock = false;
     std::vector<hipEvent_t> kev;  // pairs (kernel start, kernel end) per step
     int timed_steps = 0;
     hipEvent_t region[2] = {nullptr, nullptr};
@@ -568,7 +577,8 @@ int hipclaw_create(const hipclaw_config_t* cfg, int max_patches, hipclaw_state_t
     ALLOC(s->dys, sizeof(double) * max_patches);
     ALLOC(s->all_slots, sizeof(int) * max_patches);
     ALLOC(s->batch_slots, sizeof(int) * max_patches);
-    ALLOC(s->cfl, CFL_BYTES);
+    ALLOC(s->cfl, CFL_BYTES * hipclaw::STEP_BLOCKS);
+    ALLOC(s->sum, sizeof(unsigned long long) * hipclaw::STEP_SUMS);
     ALLOC(s->mass_buf, sizeof(double) * 2 * cfg->meqn * (size_t) max_patches);
     if (cfg->subcycle) {
         ALLOC(s->qlast, sizeof(double) * s->pstride * max_patches);
@@ -593,6 +603,9 @@ int hipclaw_create(const hipclaw_config_t* cfg, int max_patches, hipclaw_state_t
         return cleanup(fail(HIPCLAW_EDEVICE, "initial device copies failed%s"));
     if (s->q[1] && hipMemset(s->q[1], 0, sizeof(double) * s->pstride * max_patches) != hipSuccess)
         return cleanup(fail(HIPCLAW_EDEVICE, "initial device copies failed%s"));
+    if (hipHostMalloc((void**) &s->hsum, HSUM_BYTES, hipHostMallocDefault) != hipSuccess)
+        return cleanup(fail(HIPCLAW_ENOMEM, "hipHostMalloc failed%s"));
+    std::memset(s->hsum, 0, HSUM_BYTES);
     if (hipEventCreate(&s->region[0]) != hipSuccess || hipEventCreate(&s->region[1]) != hipSuccess)
         return cleanup(fail(HIPCLAW_EDEVICE, "hipEventCreate failed%s"));
     *out = s;
@@ -631,6 +644,8 @@ void hipclaw_destroy(hipclaw_state_t* s) {
     }
     hipFree(s->qsave);
     hipFree(s->cfl);
+    hipFree(s->sum);
+    if (s->hsum) hipHostFree(s->hsum);
     hipFree(s->mass_buf);
     hipFree(s->reg);
     hipFree(s->band);
@@ -1504,7 +1519,10 @@ int hipclaw_restore_step(hipclaw_state_t* s) {
     return HIPCLAW_OK;
 }
 
-static int advance_launches(hipclaw_state_t* s, double dt, int nsteps, bool timed);
+// How an advance's steps are timed: by their clock words, by events bound to
+// their launches, or, in a captured graph, not at all.
+enum class StepTimer { none, clock, events };
+static int advance_launches(hipclaw_state_t* s, double dt, int nsteps, StepTimer timer);
 static int subcycle_launches(hipclaw_state_t* s, double dt, int ncoarse);
 static int subcycle_ready(hipclaw_state_t* s);
 
@@ -1586,7 +1604,10 @@ int hipclaw_autotune(hipclaw_state_t* s, double dt, int nsteps, int* tiles, int*
     if (s->npatch == 0) return HIPCLAW_OK;
     if (sub)
         if (int rc = subcycle_ready(s)) return rc;
-    auto trial_steps = [&](int n) { return sub ? subcycle_launches(s, dt, n) : advance_launches(s, dt, n, false); };
+    s->cfl_clear = false;   // (the trials' words are nobody's result)
+    auto trial_steps = [&](int n) {
+        return sub ? subcycle_launches(s, dt, n) : advance_launches(s, dt, n, StepTimer::none);
+    };
     // the trials step through both slabs: the state is copied, not kept in its slab
     if (int rc = copy_to_save(s, s->cur)) return rc;
     s->save_lazy = false;
@@ -1734,13 +1755,27 @@ static int launch_step(hipclaw_state_t* s, const hipclaw::StepArgs& a, hipEvent_
     return HIPCLAW_OK;
 }
 
-static double read_cfl(hipclaw_state_t* s, int* rc) {
-    unsigned long long words[CFL_BYTES / sizeof(unsigned long long)];
-    hipError_t e = hipMemcpyAsync(words, s->cfl, CFL_BYTES, hipMemcpyDeviceToHost, s->st);
-    if (e == hipSuccess) e = hipStreamSynchronize(s->st);
-    if (e != hipSuccess) { *rc = hipfail(e, "reading the CFL number"); return 0.0; }
-    *rc = HIPCLAW_OK;
-    return largest_cfl(words);
+// The blocks of CFL and clock words clear before an advance writes them.
+static int clear_cfl(hipclaw_state_t* s) {
+    if (s->cfl_clear) { s->cfl_clear = false; return HIPCLAW_OK; }
+    if (int e = hipclaw::launch_reset_cfl(s->cfl, hipclaw::STEP_BLOCKS, s->sum, s->st)) return hipfail((hipError_t) e, "reset");
+    return HIPCLAW_OK;
+}
+
+// The last launch of an advance, or of a batch, whose steps wrote the first
+// `blocks` blocks.
+static int finish_cfl(hipclaw_state_t* s, int blocks, bool batch = false) {
+    unsigned long long* out = s->hsum + (batch ? hipclaw::STEP_SUMS : 0);
+    if (int e = hipclaw::launch_collect_steps(s->cfl, blocks, s->sum, out, s->st))
+        return hipfail((hipError_t) e, "collect_steps launch");
+    s->cfl_clear = true;
+    return HIPCLAW_OK;
+}
+
+static int read_cfl(hipclaw_state_t* s, double* maxcfl, bool batch = false) {
+    HIP_TRY(hipStreamSynchronize(s->st));
+    if (maxcfl) *maxcfl = as_double(s->hsum[batch ? hipclaw::STEP_SUMS : 0]);
+    return HIPCLAW_OK;
 }
 
 int hipclaw_step_batch(hipclaw_state_t* s, const int* slots, int nslots, double t, double dt,
@@ -1754,7 +1789,7 @@ int hipclaw_step_batch(hipclaw_state_t* s, const int* slots, int nslots, double 
     if (maxcfl) *maxcfl = 0.0;
     if (nslots == 0) return HIPCLAW_OK;
     HIP_TRY(hipMemcpyAsync(s->batch_slots, slots, sizeof(int) * nslots, hipMemcpyHostToDevice, s->st));
-    if (int e = hipclaw::launch_reset_cfl(s->cfl, s->st)) return hipfail((hipError_t) e, "reset");
+    if (int rc = clear_cfl(s)) return rc;
     if (s->qlast) {  // fclaw2d_clawpatch_save_current_step before every update
         int e = hipclaw::launch_copy_patches(s->q[s->cur], s->qlast, s->batch_slots, nslots,
                                              s->pstride, s->st);
@@ -1768,11 +1803,8 @@ int hipclaw_step_batch(hipclaw_state_t* s, const int* slots, int nslots, double 
                                               s->cfg.mx, s->cfg.my, s->cfg.mbc, s->cfg.meqn, s->st);
         if (e) return hipfail((hipError_t) e, "copy_interior launch");
     }
-    int rc;
-    const double c = read_cfl(s, &rc);
-    if (rc) return rc;
-    if (maxcfl) *maxcfl = c;
-    return HIPCLAW_OK;
+    if (int rc = finish_cfl(s, 1, true)) return rc;
+    return read_cfl(s, maxcfl, true);
 }
 
 int hipclaw_step_batch_noalloc(const hipclaw_config_t* cfg, int npatch, const double* q_in,
@@ -1804,7 +1836,7 @@ int hipclaw_step_batch_noalloc(const hipclaw_config_t* cfg, int npatch, const do
     int* dslots = reinterpret_cast<int*>(base + NOALLOC_CFL_BYTES);
     hipStream_t st = static_cast<hipStream_t>(stream);
     HIP_TRY(hipMemcpyAsync(dslots, slots, sizeof(int) * (size_t) nslots, hipMemcpyHostToDevice, st));
-    if (int e = hipclaw::launch_reset_cfl(dcfl, st)) return hipfail((hipError_t) e, "reset");
+    if (int e = hipclaw::launch_reset_cfl(dcfl, 1, nullptr, st)) return hipfail((hipError_t) e, "reset");
     hipclaw::StepArgs a;
     a.qsrc = q_in;
     a.qdst = q_out;
@@ -1831,12 +1863,28 @@ int hipclaw_step_batch_noalloc(const hipclaw_config_t* cfg, int npatch, const do
     unsigned long long words[CFL_BYTES / sizeof(unsigned long long)];
     HIP_TRY(hipMemcpyAsync(words, dcfl, CFL_BYTES, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
-    if (maxcfl) *maxcfl = largest_cfl(words);
+    unsigned long long bits = 0;
+    for (int k = 0; k < hipclaw::CFL_WORDS; k++) bits = std::max(bits, words[k * hipclaw::CFL_STRIDE]);
+    if (maxcfl) *maxcfl = as_double(bits);
     return HIPCLAW_OK;
 }
 
-static int advance_launches(hipclaw_state_t* s, double dt, int nsteps, bool timed) {
-    if (timed) {
+// The step of an advance that writes block `step % STEP_BLOCKS`; blocks about to
+// be written again are collected first.
+static int advance_step(hipclaw_state_t* s, hipclaw::StepArgs& a, int step, StepTimer timer) {
+    if (timer == StepTimer::events) return launch_step(s, a, s->kev[2 * step], s->kev[2 * step + 1]);
+    if (timer == StepTimer::clock) {
+        const int block = step % hipclaw::STEP_BLOCKS;
+        if (step > 0 && block == 0)
+            if (int e = hipclaw::launch_collect_steps(s->cfl, hipclaw::STEP_BLOCKS, s->sum, nullptr, s->st))
+                return hipfail((hipError_t) e, "collect_steps launch");
+        a.cfl = s->cfl + (size_t) block * hipclaw::CFL_BLOCK;
+    }
+    return launch_step(s, a);
+}
+
+static int advance_launches(hipclaw_state_t* s, double dt, int nsteps, StepTimer timer) {
+    if (timer == StepTimer::events) {
         const size_t need = 2 * (size_t) nsteps;
         while (s->kev.size() < need) {
             hipEvent_t e;
@@ -1844,7 +1892,6 @@ static int advance_launches(hipclaw_state_t* s, double dt, int nsteps, bool time
             s->kev.push_back(e);
         }
     }
-    if (int e = hipclaw::launch_reset_cfl(s->cfl, s->st)) return hipfail((hipError_t) e, "reset");
     if (s->ghost_layout == 2 && s->fused_ok && !s->reg_accumulate) {
         // two launches per step: the update (staging the corrected edge cells of
         // the last synchronisation) and the fused ghost fill + time sync; the
@@ -1864,7 +1911,7 @@ static int advance_launches(hipclaw_state_t* s, double dt, int nsteps, bool time
             // its ghost cells are the copies made before that synchronisation.
             const bool pull = s->pull_ok && !s->inplace;
             if (pull && n > 0) a.pull = s->pull;
-            if (int rc = timed ? launch_step(s, a, s->kev[2 * n], s->kev[2 * n + 1]) : launch_step(s, a)) return rc;
+            if (int rc = advance_step(s, a, n, timer)) return rc;
             if (!s->inplace) s->cur = 1 - s->cur;
             if (int rc = ghost_flat_async(s, !pull || n == nsteps - 1, s->fsync)) return rc;
         }
@@ -1879,8 +1926,8 @@ static int advance_launches(hipclaw_state_t* s, double dt, int nsteps, bool time
     for (int n = 0; n < nsteps; n++) {
         double* src = s->q[s->cur];
         double* dst = s->inplace ? src : s->q[1 - s->cur];
-        const hipclaw::StepArgs a = step_args(s, src, dst, s->all_slots, s->npatch, dt);
-        if (int rc = timed ? launch_step(s, a, s->kev[2 * n], s->kev[2 * n + 1]) : launch_step(s, a)) return rc;
+        hipclaw::StepArgs a = step_args(s, src, dst, s->all_slots, s->npatch, dt);
+        if (int rc = advance_step(s, a, n, timer)) return rc;
         if (!s->inplace) s->cur = 1 - s->cur;
         if (int rc = ghost_fill_async(s, 0)) return rc;
         if (int rc = time_sync_async(s, 0)) return rc;
@@ -1952,7 +1999,6 @@ static int subcycle_level(hipclaw_state_t* s, int level, int curr_fine_step, Lev
 
 static int subcycle_launches(hipclaw_state_t* s, double dt, int ncoarse) {
     const int lmin = s->lmin, lmax = s->lmax, nl = lmax - lmin + 1;
-    if (int e = hipclaw::launch_reset_cfl(s->cfl, s->st)) return hipfail((hipError_t) e, "reset");
     for (int c = 0; c < ncoarse; c++) {
         LevelCounter tc[HIPCLAW_MAX_PROGRAMS];
         for (int l = 0; l < nl; l++) {   // initialize_timestep_counters (:54-110)
@@ -2027,20 +2073,18 @@ int hipclaw_advance_subcycle_async(hipclaw_state_t* s, double dt, int ncoarse) {
     if (!s || ncoarse < 0 || !(dt > 0.0)) return fail(HIPCLAW_EINVAL, "hipclaw_advance_subcycle: bad arguments%s");
     if (int rc = subcycle_ready(s)) return rc;
     if (int rc = guard_save(s)) return rc;
+    if (int rc = clear_cfl(s)) return rc;
     HIP_TRY(hipEventRecord(s->region[0], s->st));
     if (int rc = subcycle_launches(s, dt, ncoarse)) return rc;
     HIP_TRY(hipEventRecord(s->region[1], s->st));
     s->timed_steps = 0;
-    return HIPCLAW_OK;
+    s->by_clock = false;
+    return finish_cfl(s, 1);
 }
 
 int hipclaw_advance_subcycle(hipclaw_state_t* s, double dt, int ncoarse, double* maxcfl) {
     if (int rc = hipclaw_advance_subcycle_async(s, dt, ncoarse)) return rc;
-    int rc;
-    const double c = read_cfl(s, &rc);
-    if (rc) return rc;
-    if (maxcfl) *maxcfl = c;
-    return HIPCLAW_OK;
+    return read_cfl(s, maxcfl);
 }
 
 int hipclaw_capture_subcycle_graph(hipclaw_state_t* s, double dt, int ncoarse) {
@@ -2071,11 +2115,19 @@ int hipclaw_advance_async(hipclaw_state_t* s, double dt, int nsteps) {
     if (!(s->ghost_layout == 2 && s->fused_ok && !s->reg_accumulate))
         if (int rc = ensure_layouts(s)) return rc;
     if (int rc = guard_save(s, nsteps == 1)) return rc;
+    if (int rc = clear_cfl(s)) return rc;
+    s->timed_steps = 0;
+    if (!user_solver(s->cfg.solver)) {
+        if (int rc = advance_launches(s, dt, nsteps, StepTimer::clock)) return rc;
+        s->by_clock = true;
+        return finish_cfl(s, std::min(nsteps - (nsteps - 1) / hipclaw::STEP_BLOCKS * hipclaw::STEP_BLOCKS, nsteps));
+    }
     HIP_TRY(hipEventRecord(s->region[0], s->st));
-    if (int rc = advance_launches(s, dt, nsteps, s->time_kernels)) return rc;
+    if (int rc = advance_launches(s, dt, nsteps, StepTimer::events)) return rc;
     HIP_TRY(hipEventRecord(s->region[1], s->st));
-    s->timed_steps = s->time_kernels ? nsteps : 0;
-    return HIPCLAW_OK;
+    s->timed_steps = nsteps;
+    s->by_clock = false;
+    return finish_cfl(s, 1);
 }
 
 int hipclaw_sync(hipclaw_state_t* s) {
@@ -2086,11 +2138,7 @@ int hipclaw_sync(hipclaw_state_t* s) {
 
 int hipclaw_advance(hipclaw_state_t* s, double dt, int nsteps, double* maxcfl) {
     if (int rc = hipclaw_advance_async(s, dt, nsteps)) return rc;
-    int rc;
-    const double c = read_cfl(s, &rc);
-    if (rc) return rc;
-    if (maxcfl) *maxcfl = c;
-    return HIPCLAW_OK;
+    return read_cfl(s, maxcfl);
 }
 
 int hipclaw_capture_graph(hipclaw_state_t* s, double dt, int nsteps) {
@@ -2106,7 +2154,7 @@ int hipclaw_capture_graph(hipclaw_state_t* s, double dt, int nsteps) {
     const int cur0 = s->cur;
     s->graph_cur = cur0;
     HIP_TRY(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
-    int rc = advance_launches(s, dt, nsteps, false);
+    int rc = advance_launches(s, dt, nsteps, StepTimer::none);
     if (!rc && s->cur != cur0) {   // an odd number of steps: the result back into the slab the next replay starts from
         if (int c = hipclaw::launch_copy_patches(s->q[s->cur], s->q[cur0], s->all_slots, s->npatch, s->pstride, s->st))
             rc = hipfail((hipError_t) c, "copy_patches launch");
@@ -2134,10 +2182,12 @@ int hipclaw_replay_graph(hipclaw_state_t* s) {
             return hipfail((hipError_t) e, "copy_patches launch");
         s->cur = s->graph_cur;
     }
+    s->cfl_clear = false;   // (a captured step leaves its words as they are)
     HIP_TRY(hipEventRecord(s->region[0], s->st));
     HIP_TRY(hipGraphLaunch(s->gexec, s->st));
     HIP_TRY(hipEventRecord(s->region[1], s->st));
     s->timed_steps = 0;
+    s->by_clock = false;
     // an even number of ping-pong steps leaves the current slab unchanged
     return HIPCLAW_OK;
 }
@@ -2145,6 +2195,15 @@ int hipclaw_replay_graph(hipclaw_state_t* s) {
 int hipclaw_timing(hipclaw_state_t* s, int nsteps, double* total_ms, double* step_kernel_ms) {
     if (!s) return fail(HIPCLAW_EINVAL, "null state%s");
     HIP_TRY(hipStreamSynchronize(s->st));
+    if (s->by_clock) {
+        int dev = 0, khz = 0;
+        HIP_TRY(hipGetDevice(&dev));
+        HIP_TRY(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+        const unsigned long long* t = s->hsum;
+        if (total_ms) *total_ms = t[3] && t[4] > t[3] ? (double) (t[4] - t[3]) / khz : 0.0;
+        if (step_kernel_ms) *step_kernel_ms = nsteps > 0 && t[2] ? (double) t[1] / (double) t[2] / khz : 0.0;
+        return HIPCLAW_OK;
+    }
     float ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms, s->region[0], s->region[1]));
     if (total_ms) *total_ms = ms;

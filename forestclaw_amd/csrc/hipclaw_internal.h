@@ -125,8 +125,16 @@ int launch_apply_qcorr(double* q, const double* qcorr, const int* cmask, const i
                        hipStream_t st);
 int launch_step_fp64(int solver, int tile, int waves, const StepArgs& a, const StepLaunch& st);
 int launch_step_fp32(int solver, int tile, int waves, const StepArgs& a, const StepLaunch& st);
-// The CFL words (StepArgs::cfl) to zero.
-int launch_reset_cfl(unsigned long long* p, hipStream_t st);
+// `blocks` blocks of CFL and clock words (StepArgs::cfl) and, if given, the sums to zero.
+int launch_reset_cfl(unsigned long long* p, int blocks, unsigned long long* sum, hipStream_t st);
+// What an advance's steps left in the first `blocks` blocks (at most
+// STEP_BLOCKS) added to sum, and the blocks cleared.  With out (host memory),
+// the sum goes there, and is cleared: out[0] the Courant number's bits, out[1]
+// the clock ticks of the step launches, out[2] their number, out[3] when the
+// first one began, out[4] the time now.
+constexpr int STEP_BLOCKS = 64, STEP_SUMS = 5;
+int launch_collect_steps(unsigned long long* cfl, int blocks, unsigned long long* sum, unsigned long long* out,
+                         hipStream_t st);
 // Whole patch slabs src[slot] -> dst[slot].
 int launch_copy_patches(const double* src, double* dst, const int* slots, int n, long long pstride,
                         hipStream_t st);

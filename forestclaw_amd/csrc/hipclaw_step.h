@@ -37,6 +37,7 @@
 namespace hipclaw {
 
 constexpr int CFL_WORDS = 16, CFL_STRIDE = 32;   // (256 bytes apart)
+constexpr int CFL_BLOCK = CFL_WORDS * CFL_STRIDE;
 
 struct StepArgs {
     const double* qsrc;        // [slot][meqn][my+2mbc][mx+2mbc]
@@ -48,6 +49,9 @@ struct StepArgs {
     // Courant number: FP64 bits, atomic max (non-negative doubles order as
     // integers).  CFL_WORDS words CFL_STRIDE apart, the result being the largest
     // of them: atomics on one word are served one after another, ~11 ns each.
+    // Beside each of them stands a clock word, the largest of which is when the
+    // launch's last wave ended, and beside that, in the first, when the launch
+    // began (step_strips; wall clock ticks).
     unsigned long long* cfl;
     long long pstride;         // doubles per patch in q
     long long astride;         // doubles per patch in aux

@@ -148,6 +148,7 @@ step_strips(StepArgs a, StripShape sh) {
     // share in the same L2.  (The grid is a multiple of 8.)
     const int blk = (int) (blockIdx.x & 7) * (int) (gridDim.x >> 3) + (int) (blockIdx.x >> 3);
     const int wid = blk * (int) (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (wid == 0 && lane == 0) a.cfl[2] = __builtin_amdgcn_s_memrealtime();   // (of the first workgroup)
     const int pw = wid / sh.nsy, ty = wid - pw * sh.nsy;
     const int round = pw / sh.waves, wk = pw - round * sh.waves;
     const int patch0 = round * sh.patches;
@@ -637,12 +638,15 @@ step_strips(StepArgs a, StripShape sh) {
         }
     }
 
-    // ---- CFL: wave64 max over the lanes' interfaces, one atomic per wave ----
+    // ---- CFL: wave64 max over the lanes' interfaces; the wave's end ----
     double cfl = fmax(ifx ? dtdx64 * (double) smaxx : 0.0, ify ? dtdy64 * (double) smaxy : 0.0);
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) cfl = fmax(cfl, __shfl_xor(cfl, off, 64));
-    if (lane == 0 && cfl > 0.0)
-        atomicMax(a.cfl + (wid & (CFL_WORDS - 1)) * CFL_STRIDE, (unsigned long long) __double_as_longlong(cfl));
+    if (lane == 0) {
+        unsigned long long* w = a.cfl + (wid & (CFL_WORDS - 1)) * CFL_STRIDE;
+        if (cfl > 0.0) atomicMax(w, (unsigned long long) __double_as_longlong(cfl));
+        atomicMax(w + 1, (unsigned long long) __builtin_amdgcn_s_memrealtime());
+    }
 }
 
 }  // namespace hipclaw

@@ -361,10 +361,11 @@ int hipclaw_replay_graph(hipclaw_state_t *s);
  * (src/patches/clawpatch/fort_4.6/fclaw2d_clawpatch46_diagnostics.f:13-55). */
 int hipclaw_mass(hipclaw_state_t *s, double *sum_hi, double *sum_lo);
 
-/* Timing of the last hipclaw_advance_async/replay region, measured with HIP
- * events on the state's stream: total milliseconds and milliseconds spent in
- * the patch-update kernel alone (per launch average, from events bound to each
- * update kernel's own start and end, as a kernel trace reports it). */
+/* Timing of the last advance, subcycled advance or replay: total milliseconds
+ * on the device and, for an advance, milliseconds spent in the patch-update
+ * kernel alone (per launch average).  The update kernels of the built-in solvers
+ * note the device's clock at their own start and end; a registered solver's
+ * launches, replays and subcycled advances are timed with HIP events. */
 int hipclaw_timing(hipclaw_state_t *s, int nsteps, double *total_ms, double *step_kernel_ms);
 
 /* Levels of slots 0..npatch-1 (npatch = the current patch count), for the
