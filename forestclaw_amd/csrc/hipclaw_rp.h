@@ -32,17 +32,55 @@ struct PhysParams {
     double p[8];
 };
 
+// c ? a : b.  A 64-bit select is two 32-bit ones, and the short encoding of
+// v_cndmask, whose mask is VCC, takes 9.6 ns when another one comes right before
+// it (2.2 ns otherwise; two waves per SIMD): a compare and two of them 16 to 20
+// ns, with the long encoding, whose mask is any scalar pair, 6.5 ns.  The wait
+// states are those a vector instruction needs before it reads a mask that one
+// wrote.
+__device__ __forceinline__ double pick(bool c, double a, double b) {
+    const unsigned long long m = __builtin_amdgcn_ballot_w64(c);
+    int lo, hi;
+    asm("s_nop 1\n\tv_cndmask_b32_e64 %0, %2, %3, %6\n\tv_cndmask_b32_e64 %1, %4, %5, %6"
+        : "=&v"(lo), "=v"(hi)
+        : "v"(__double2loint(b)), "v"(__double2loint(a)), "v"(__double2hiint(b)), "v"(__double2hiint(a)), "s"(m));
+    return __hiloint2double(hi, lo);
+}
+// c ? 0 : b
+__device__ __forceinline__ double pick_zero(bool c, double b) {
+    const unsigned long long m = __builtin_amdgcn_ballot_w64(c);
+    int lo, hi;
+    asm("s_nop 1\n\tv_cndmask_b32_e64 %0, %2, 0, %4\n\tv_cndmask_b32_e64 %1, %3, 0, %4"
+        : "=&v"(lo), "=v"(hi)
+        : "v"(__double2loint(b)), "v"(__double2hiint(b)), "s"(m));
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ float pick(bool c, float a, float b) { return c ? a : b; }
+
 // min / max.  FP64 selects as the reference's MIN / MAX (a compare and a
 // select); FP32 uses the hardware v_min_f32 / v_max_f32, which differ only
 // for NaN operands.
 template <typename R>
-__device__ __forceinline__ R rmin(R a, R b) { return a < b ? a : b; }
+__device__ __forceinline__ R rmin(R a, R b) { return pick(a < b, a, b); }
 template <typename R>
-__device__ __forceinline__ R rmax(R a, R b) { return a > b ? a : b; }
+__device__ __forceinline__ R rmax(R a, R b) { return pick(a > b, a, b); }
 template <>
 __device__ __forceinline__ float rmin<float>(float a, float b) { return __builtin_fminf(a, b); }
 template <>
 __device__ __forceinline__ float rmax<float>(float a, float b) { return __builtin_fmaxf(a, b); }
+// min(x, c) with c a number: of a NaN, c, as the select's.
+__device__ __forceinline__ double rcap(double x, double c) { return __builtin_fmin(x, c); }
+__device__ __forceinline__ float rcap(float x, float c) { return __builtin_fminf(x, c); }
+// max(0, x), a NaN staying one
+__device__ __forceinline__ double rpos0(double x) { return pick_zero(0.0 > x, x); }
+__device__ __forceinline__ float rpos0(float x) { return __builtin_fmaxf(0.0f, x); }
+// The parts of a speed below and above zero: of a NaN, 0, as the selects
+// min(x, 0) and max(x, 0); they differ from those in the sign of a zero, which
+// no sum they enter keeps.
+__device__ __forceinline__ double rneg(double x) { return __builtin_fmin(x, 0.0); }
+__device__ __forceinline__ double rplus(double x) { return __builtin_fmax(x, 0.0); }
+__device__ __forceinline__ float rneg(float x) { return __builtin_fminf(x, 0.0f); }
+__device__ __forceinline__ float rplus(float x) { return __builtin_fmaxf(x, 0.0f); }
 
 // Sums that start at zero: 0 + x and 0 - x.  FP64 keeps the reference's
 // accumulations from zero, whose only effect is the sign of a zero result;
@@ -94,6 +132,62 @@ __device__ __forceinline__ R sq(R a) { return sqrt(a); }
 template <>
 __device__ __forceinline__ float sq<float>(float a) { return __builtin_amdgcn_sqrtf(a); }
 
+// FP64 quotients q = n / b of one b, as IEEE rounds them.  With `fast` (the same
+// in every lane) b's reciprocal is refined once and each quotient corrected by
+// its exact residual (Markstein, "Computation of elementary functions on the IBM
+// RISC System/6000 processor", 1990), without the scaling that a general division
+// needs: b and 1 / b have to be normal numbers and every n zero, infinite, not a
+// number, or within FAST_EXP powers of two of 1.  A general division takes 27 ns,
+// the reciprocal 18 and each quotient 10 (per SIMD, two waves on it).
+constexpr int FAST_EXP = 900;
+template <int N>
+__device__ __forceinline__ void quotients(const double (&n)[N], double b, bool fast, double (&q)[N]) {
+    if (fast) {
+        const double y = flux_rcp(b);
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+            const double t = n[k] * y;
+            q[k] = __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, t, n[k]), y, t), b, n[k]);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < N; k++) q[k] = n[k] / b;
+    }
+}
+// The correctly rounded square root of a number between 2^-900 and 2^900
+// (Goldschmidt's iteration from the hardware estimate, then two corrections by
+// the exact residual): 26 ns where the general one takes 39.
+__device__ __forceinline__ double fast_root(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, r, g);
+    h = __builtin_fma(h, r, h);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
+__device__ __forceinline__ bool all_lanes(bool x) { return __builtin_amdgcn_ballot_w64(!x) == 0; }
+// x > 0 and within 2^+-100; |x| zero, infinite, not a number or between 2^lo and
+// 2^hi.
+__device__ __forceinline__ bool moderate(double x) {
+    return (unsigned) (__double2hiint(x) - ((1023 - 100) << 20)) < 200u << 20;
+}
+__device__ __forceinline__ bool exponent_within(double x, int lo, int hi) {
+    return (unsigned) (__builtin_amdgcn_frexp_exp(x) - lo) <= (unsigned) (hi - lo);
+}
+
+// A solver that divides by one value several times (RP::RANGED; with the tests
+// that spare the entropy fix its divisions, 100 dam break steps 24.2 -> 23.3 ms,
+// 100 shock-bubble steps 12.5 -> 11.7 ms, batched 24 x 20 shallow water 134 -> 125
+// us): RP::in_range(q,
+// pp) says whether a cell's values allow the fast forms above, RP::cells gives
+// `cell` in both directions, rpn2c takes whether both cells are in range, and
+// rpt2_pair splits both fluctuations of an interface.
+template <class RP, class = void>
+struct ranged : std::false_type {};
+template <class RP>
+struct ranged<RP, std::enable_if_t<RP::RANGED>> : std::true_type {};
+
 // A solver whose rpt2 is linear in asdq (RP::RPT2_LINEAR): the FP32 form then
 // scales asdq by dt / (2 dx) before the transverse solve instead of scaling
 // both results after it.  Solvers without the flag keep the reference's order.
@@ -136,6 +230,7 @@ struct RPShallow {
     static constexpr bool CONSERVATIVE = true;  // amdq + apdq = f(qR) - f(qL)
     static constexpr bool RPT2_LINEAR = true;   // bm, bp linear in asdq
     static constexpr bool EXPLICIT_FMA = true;  // no contraction left to the compiler (mad)
+    static constexpr bool RANGED = sizeof(R) == 8;
     // u, v, a (and in FP32 1 / (2 a), which rpt2 then takes from the normal solve)
     static constexpr int NROE = sizeof(R) == 4 ? 4 : 3;
 
@@ -179,6 +274,37 @@ struct RPShallow {
         }
     }
 
+    // Depth and gravity within 2^+-100, momenta zero or between 2^-600 and
+    // 2^200: u is then zero or above 2^-760, u + a and a difference of depths or
+    // momenta zero or above a sum's last place, 2^-155, 2^-152 and 2^-652, so the
+    // numerators of rpn2 are zero or above 2^-760 and all below 2^410.
+    __device__ __forceinline__ static bool in_range(const double* q, const PhysParams& pp) {
+        return moderate(q[0]) && moderate(pp.grav) && exponent_within(q[1], -600, 200) && exponent_within(q[2], -600, 200);
+    }
+
+    __device__ __forceinline__ static void cells(const double* q, const PhysParams& pp, bool fast, double cx[NCELL],
+                                                 double cy[NCELL]) {
+        const double n[2] = {q[1], q[2]};
+        double hs, c, r[2], u[2];
+        if (fast) {
+            hs = fast_root(q[0]);
+            c = fast_root(pp.grav * q[0]);
+            quotients(n, hs, true, r);
+            quotients(n, q[0], true, u);
+        } else {
+            hs = sqrt(q[0]);
+            c = sqrt(pp.grav * q[0]);
+            quotients(n, hs, false, r);
+            quotients(n, q[0], false, u);
+        }
+        cx[0] = cy[0] = hs;
+        cx[1] = cy[2] = r[0];
+        cx[2] = cy[1] = r[1];
+        cx[3] = u[0];
+        cy[3] = u[1];
+        cx[4] = cy[4] = c;
+    }
+
     // sqrt(g) in FP32 (uniform; the compiler keeps it out of the sweeps' loops)
     __device__ __forceinline__ static float sqrt_grav(const PhysParams& pp) {
         return __builtin_amdgcn_sqrtf((float) pp.grav);
@@ -208,9 +334,9 @@ struct RPShallow {
                                                  const R* cR, const R* /*auxL*/,
                                                  const R* /*auxR*/, const PhysParams& pp,
                                                  R wave[MWAVES][MEQN], R s[MWAVES], R amdq[MEQN],
-                                                 R apdq[MEQN], R roe[NROE]) {
+                                                 R apdq[MEQN], R roe[NROE], bool fast = false) {
         if constexpr (sizeof(R) == 4) rpn2c_fp32<IXY>(qL, qR, cL, cR, pp, wave, s, amdq, apdq, roe);
-        else rpn2c_fp64<IXY>(qL, qR, cL, cR, pp, wave, s, amdq, apdq, roe);
+        else rpn2c_fp64<IXY>(qL, qR, cL, cR, pp, wave, s, amdq, apdq, roe, fast);
     }
 
     // FP32: one reciprocal and one reciprocal square root for the Roe averages
@@ -241,10 +367,10 @@ struct RPShallow {
         const float lL = cL[3] - cL[4], lR = cR[3] + cR[4], l1 = um - cm, l3 = um + cm;
         const bool t1 = lL < 0.0f && l1 > 0.0f, t3 = l3 < 0.0f && lR > 0.0f;
         const float r = __builtin_amdgcn_rcpf(t3 ? lR - l3 : l1 - lL);
-        const float f1 = t1 ? lL * ((l1 - s0) * r) : rmin(s0, 0.0f);
-        float f3 = t3 ? l3 * ((lR - s2) * r) : rmin(s2, 0.0f);
+        const float f1 = t1 ? lL * ((l1 - s0) * r) : rneg(s0);
+        float f3 = t3 ? l3 * ((lR - s2) * r) : rneg(s2);
         f3 = u > 0.0f ? 0.0f : f3;
-        const float f2 = rmin(u, 0.0f), g1 = s0 - f1, g2 = rmax(u, 0.0f), g3 = s2 - f3;
+        const float f2 = rneg(u), g1 = s0 - f1, g2 = rplus(u), g3 = s2 - f3;
         amdq[0] = mad(f3, a3, f1 * a1);
         amdq[mu] = mad(f3, wave[2][mu], f1 * wave[0][mu]);
         amdq[mv] = mad(f2, a2, mad(f3, wave[2][mv], f1 * wave[0][mv]));
@@ -253,10 +379,19 @@ struct RPShallow {
         apdq[mv] = mad(g2, a2, mad(g3, wave[2][mv], g1 * wave[0][mv]));
     }
 
+    // Whether the entropy fix has to look at the speed of an intermediate state:
+    // not if that is subcritical by a margin above all rounding,
+    // (hu)^2 < 0.998 g h^3, since hu / h -+ sqrt(g h) then has the sign of -+1.
+    __device__ __forceinline__ static bool near_critical(R hu, R h, const PhysParams& pp) {
+        const R t = (R) pp.grav * h * h * h;
+        return !(hu * hu < R(0.998) * t && t > R(1e-200) && t < R(1e300));
+    }
+
     template <int IXY>
     __device__ __forceinline__ static void rpn2c_fp64(const R* qL, const R* qR, const R* cL, const R* cR,
                                                       const PhysParams& pp, R wave[MWAVES][MEQN],
-                                                      R s[MWAVES], R amdq[MEQN], R apdq[MEQN], R roe[NROE]) {
+                                                      R s[MWAVES], R amdq[MEQN], R apdq[MEQN], R roe[NROE],
+                                                      bool fast) {
         constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
         const R grav = (R) pp.grav;
         const R h = dv(qL[0] + qR[0], R(2));
@@ -264,11 +399,17 @@ struct RPShallow {
         const R hsqrtr = cR[0];
         const R hsq2 = hsqrtl + hsqrtr;
         const R d0 = qR[0] - qL[0], d1 = qR[mu] - qL[mu], d2 = qR[mv] - qL[mv];
-        const R u = dv(cL[1] + cR[1], hsq2);
-        const R v = dv(cL[2] + cR[2], hsq2);
-        const R a = sq(grav * h);
-        const R a1 = dv((u + a) * d0 - d1, R(2) * a);
-        const R a3 = dv(-((u - a) * d0) + d1, R(2) * a);
+        const R nu[2] = {cL[1] + cR[1], cL[2] + cR[2]};
+        R uv[2], a13[2], a;
+        auto averages = [&](bool f) __attribute__((always_inline)) {
+            quotients(nu, hsq2, f, uv);
+            a = f ? fast_root(grav * h) : sqrt(grav * h);
+            const R na[2] = {(uv[0] + a) * d0 - d1, -((uv[0] - a) * d0) + d1};
+            quotients(na, R(2) * a, f, a13);
+        };
+        if (fast) averages(true);
+        else averages(false);
+        const R u = uv[0], v = uv[1], a1 = a13[0], a3 = a13[1];
         roe[0] = u; roe[1] = v; roe[2] = a;
         const R a2 = -(v * d0) + d2;
 
@@ -284,11 +425,11 @@ struct RPShallow {
         } else {
             const R h1 = qL[0] + wave[0][0];
             const R hu1 = qL[mu] + wave[0][mu];
-            const R s1 = char_speed<-1>(hu1, h1, pp);
-            R sfract;
-            if (s0 < R(0) && s1 > R(0)) sfract = s0 * dv(s1 - s[0], s1 - s0);
-            else if (s[0] < R(0)) sfract = s[0];
-            else sfract = R(0);
+            R sfract = rneg(s[0]);
+            if (near_critical(hu1, h1, pp)) {
+                const R s1 = char_speed<-1>(hu1, h1, pp);
+                if (s0 < R(0) && s1 > R(0)) sfract = s0 * dv(s1 - s[0], s1 - s0);
+            }
 #pragma unroll
             for (int m = 0; m < 3; m++) amdq[m] = sfract * wave[0][m];
             if (!(s[1] > R(0))) {
@@ -297,11 +438,15 @@ struct RPShallow {
                 const R s03 = cR[3] + cR[4];   // dv(qR[mu], qR[0]) + sq(grav * qR[0])
                 const R h3 = qR[0] - wave[2][0];
                 const R hu3 = qR[mu] - wave[2][mu];
-                const R s3 = char_speed<1>(hu3, h3, pp);
-                bool add = true;
-                if (s3 < R(0) && s03 > R(0)) sfract = s3 * dv(s03 - s[2], s03 - s3);
-                else if (s[2] < R(0)) sfract = s[2];
-                else add = false;
+                bool add = s[2] < R(0);
+                sfract = s[2];
+                if (near_critical(hu3, h3, pp)) {
+                    const R s3 = char_speed<1>(hu3, h3, pp);
+                    if (s3 < R(0) && s03 > R(0)) {
+                        sfract = s3 * dv(s03 - s[2], s03 - s3);
+                        add = true;
+                    }
+                }
                 if (add) {
 #pragma unroll
                     for (int m = 0; m < 3; m++) amdq[m] = amdq[m] + sfract * wave[2][m];
@@ -333,18 +478,45 @@ struct RPShallow {
             const float r2 = roe[NROE - 1];
             const float a1 = mad(v + a, asdq[0], -asdq[mv]) * r2, a3 = mad(a - v, asdq[0], asdq[mv]) * r2;
             const float a2 = mad(-u, asdq[0], asdq[mu]);
-            const float m1 = rmin(v - a, 0.0f) * a1, m3 = rmin(v + a, 0.0f) * a3;
-            const float p1 = rmax(v - a, 0.0f) * a1, p3 = rmax(v + a, 0.0f) * a3;
+            const float m1 = rneg(v - a) * a1, m3 = rneg(v + a) * a3;
+            const float p1 = rplus(v - a) * a1, p3 = rplus(v + a) * a3;
             bm[0] = m1 + m3;
-            bm[mu] = mad(u, bm[0], rmin(v, 0.0f) * a2);
+            bm[mu] = mad(u, bm[0], rneg(v) * a2);
             bm[mv] = mad(v, bm[0], a * (m3 - m1));
             bp[0] = p1 + p3;
-            bp[mu] = mad(u, bp[0], rmax(v, 0.0f) * a2);
+            bp[mu] = mad(u, bp[0], rplus(v) * a2);
             bp[mv] = mad(v, bp[0], a * (p3 - p1));
-            return;
+        } else {
+            const R a1 = dv((v + a) * asdq[0] - asdq[mv], R(2) * a);
+            const R a3 = dv(-((v - a) * asdq[0]) + asdq[mv], R(2) * a);
+            split<IXY>(roe, asdq, a1, a3, bm, bp);
         }
-        const R a1 = dv((v + a) * asdq[0] - asdq[mv], R(2) * a);
-        const R a3 = dv(-((v - a) * asdq[0]) + asdq[mv], R(2) * a);
+    }
+
+    // both fluctuations of an interface; fast: its cells are in range
+    template <int IXY>
+    __device__ __forceinline__ static void rpt2_pair(const double roe[NROE], const double amdq[MEQN],
+                                                     const double apdq[MEQN], bool fast, double bmA[MEQN],
+                                                     double bpA[MEQN], double bmP[MEQN], double bpP[MEQN]) {
+        constexpr int mv = IXY == 1 ? 2 : 1;
+        const double v = roe[1], a = roe[2];
+        const double n[4] = {(v + a) * amdq[0] - amdq[mv], -((v - a) * amdq[0]) + amdq[mv],
+                             (v + a) * apdq[0] - apdq[mv], -((v - a) * apdq[0]) + apdq[mv]};
+        bool ok = true;
+#pragma unroll
+        for (int k = 0; k < 4; k++) ok = ok && exponent_within(n[k], -FAST_EXP, FAST_EXP);
+        double w[4];
+        if (fast && all_lanes(ok)) quotients(n, 2.0 * a, true, w);
+        else quotients(n, 2.0 * a, false, w);
+        split<IXY>(roe, amdq, w[0], w[1], bmA, bpA);
+        split<IXY>(roe, apdq, w[2], w[3], bmP, bpP);
+    }
+
+    template <int IXY>
+    __device__ __forceinline__ static void split(const R roe[NROE], const R asdq[MEQN], R a1, R a3, R bm[MEQN],
+                                                 R bp[MEQN]) {
+        constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
+        const R u = roe[0], v = roe[1], a = roe[2];
         const R a2 = asdq[mu] - u * asdq[0];
         R wb[3][3], sb[3];
         wb[0][0] = a1;   wb[0][mu] = a1 * u; wb[0][mv] = a1 * (v - a); sb[0] = v - a;
@@ -352,12 +524,12 @@ struct RPShallow {
         wb[2][0] = a3;   wb[2][mu] = a3 * u; wb[2][mv] = a3 * (v + a); sb[2] = v + a;
 #pragma unroll
         for (int m = 0; m < 3; m++) {
-            R m_ = rmin(sb[0], R(0)) * wb[0][m], p_ = rmax(sb[0], R(0)) * wb[0][m];
+            R m_ = rneg(sb[0]) * wb[0][m], p_ = rplus(sb[0]) * wb[0][m];
 #pragma unroll
             for (int mw = 1; mw < 3; mw++) {
                 if (mw == 1 && m != mu) continue;   // wb[1][0], wb[1][mv] are zero
-                m_ = m_ + rmin(sb[mw], R(0)) * wb[mw][m];
-                p_ = p_ + rmax(sb[mw], R(0)) * wb[mw][m];
+                m_ = m_ + rneg(sb[mw]) * wb[mw][m];
+                p_ = p_ + rplus(sb[mw]) * wb[mw][m];
             }
             bm[m] = m_;
             bp[m] = p_;
@@ -408,6 +580,7 @@ struct RPEuler {
     static constexpr bool CONSERVATIVE = true;
     static constexpr bool RPT2_LINEAR = true;   // bm, bp linear in asdq
     static constexpr bool EXPLICIT_FMA = true;  // no contraction left to the compiler (mad)
+    static constexpr bool RANGED = sizeof(R) == 8;
     // u, v, a, enth, u2v2, g1a2, euv (and in FP32 1 / (2 a), which rpt2 then
     // takes from the normal solve)
     static constexpr int NROE = sizeof(R) == 4 ? 8 : 7;
@@ -459,6 +632,52 @@ struct RPEuler {
         c[5] = sq(dv(gamma * pn, q[0]));
     }
 
+    // (the momenta's squares are summed in one order for both directions: a sum
+    // of two rounds the same either way)
+    __device__ __forceinline__ static void cells(const double* q, const PhysParams& pp, bool fast, double cx[NCELL],
+                                                 double cy[NCELL]) {
+#pragma clang fp contract(off)
+        const double gamma1 = pp.gamma - 1.0;
+        const double k[1] = {0.5 * (q[1] * q[1] + q[2] * q[2])};
+        double rs, r[3], u[3];
+        auto values = [&](bool f) __attribute__((always_inline)) {
+            rs = f ? fast_root(q[0]) : sqrt(q[0]);
+            double d[1];
+            quotients(k, q[0], f, d);
+            const double p = gamma1 * (q[3] - d[0]);
+            const double nr[3] = {q[1], q[2], q[3] + p}, nu[3] = {q[1], q[2], pp.gamma * p};
+            quotients(nr, rs, f, r);
+            quotients(nu, q[0], f, u);
+        };
+        if (fast) values(true);
+        else values(false);
+        cx[0] = cy[0] = rs;
+        cx[1] = cy[2] = r[0];
+        cx[2] = cy[1] = r[1];
+        cx[3] = cy[3] = r[2];
+        cx[4] = u[0];
+        cy[4] = u[1];
+        cx[5] = cy[5] = sqrt(u[2]);
+    }
+
+    // Density, energy and gamma - 1 within 2^+-100, momenta zero or between
+    // 2^-300 and 2^200: their squares over the density are zero or above 2^-701,
+    // the pressures and enthalpies zero or above a sum's last place, 2^-860, and
+    // all below 2^520.
+    __device__ __forceinline__ static bool in_range(const double* q, const PhysParams& pp) {
+        return moderate(q[0]) && moderate(q[3]) && moderate(pp.gamma - 1.0) && exponent_within(q[1], -300, 200) &&
+               exponent_within(q[2], -300, 200);
+    }
+
+    // Whether the entropy fix has to look at the speed of an intermediate state:
+    // not if that is subsonic by a margin above all rounding,
+    // (rho u)^2 < 0.99 gamma p rho, with a pressure that is no small difference.
+    __device__ __forceinline__ static bool near_sonic(R rho, R rhou, R rhov, R en, R gamma, R gamma1) {
+#pragma clang fp contract(off)
+        const R e = en * rho, t = gamma * gamma1 * (e - R(0.5) * (rhou * rhou + rhov * rhov));
+        return !(rhou * rhou < R(0.99) * t && t > R(1e-6) * e && e > R(1e-200) && e < R(1e300) && rho > R(0));
+    }
+
     template <int IXY>
     __device__ __forceinline__ static void rpn2(const R* qL, const R* qR, const R* auxL,
                                                 const R* auxR, const PhysParams& pp,
@@ -476,7 +695,7 @@ struct RPEuler {
                                                  const R* cR, const R* /*auxL*/,
                                                  const R* /*auxR*/, const PhysParams& pp,
                                                  R wave[MWAVES][MEQN], R s[MWAVES], R amdq[MEQN],
-                                                 R apdq[MEQN], R roe[NROE]) {
+                                                 R apdq[MEQN], R roe[NROE], bool fast = false) {
 #pragma clang fp contract(off)
         constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
         const R gamma = (R) pp.gamma;
@@ -493,9 +712,10 @@ struct RPEuler {
             v = (cL[2] + cR[2]) * rh;
             enth = (cL[3] + cR[3]) * rh;
         } else {
-            u = dv(cL[1] + cR[1], rhsq2);
-            v = dv(cL[2] + cR[2], rhsq2);
-            enth = dv(cL[3] + cR[3], rhsq2);
+            const R n[3] = {cL[1] + cR[1], cL[2] + cR[2], cL[3] + cR[3]};
+            R r[3];
+            quotients(n, rhsq2, fast, r);
+            u = r[0]; v = r[1]; enth = r[2];
         }
         const R u2v2 = mad(v, v, u * u);
         const R a2s = gamma1 * mad(R(-.5), u2v2, enth);
@@ -540,13 +760,13 @@ struct RPEuler {
             const R rhou1 = qL[mu] + wave[0][mu];
             const R rhov1 = qL[mv] + wave[0][mv];
             const R en1 = qL[3] + wave[0][3];
-            const R p1 = gamma1 * (en1 - dv(R(0.5) * mad(rhov1, rhov1, rhou1 * rhou1), rho1));
-            const R c1 = sq(dv(gamma * p1, rho1));
-            const R s1 = dv(rhou1, rho1) - c1;
-            R sfract;
-            if (s0 < R(0) && s1 > R(0)) sfract = dv(s0 * (s1 - s[0]), s1 - s0);
-            else if (s[0] < R(0)) sfract = s[0];
-            else sfract = R(0);
+            R sfract = rneg(s[0]);
+            if (sizeof(R) == 4 || near_sonic(rho1, rhou1, rhov1, en1, gamma, gamma1)) {
+                const R p1 = gamma1 * (en1 - dv(R(0.5) * mad(rhov1, rhov1, rhou1 * rhou1), rho1));
+                const R c1 = sq(dv(gamma * p1, rho1));
+                const R s1 = dv(rhou1, rho1) - c1;
+                if (s0 < R(0) && s1 > R(0)) sfract = dv(s0 * (s1 - s[0]), s1 - s0);
+            }
 #pragma unroll
             for (int m = 0; m < 4; m++) amdq[m] = sfract * wave[0][m];
             if (!(s[1] >= R(0))) {
@@ -560,13 +780,17 @@ struct RPEuler {
                 const R rhou2 = qR[mu] - wave[3][mu];
                 const R rhov2 = qR[mv] - wave[3][mv];
                 const R en2 = qR[3] - wave[3][3];
-                const R p2 = gamma1 * (en2 - dv(R(0.5) * mad(rhov2, rhov2, rhou2 * rhou2), rho2));
-                const R c2 = sq(dv(gamma * p2, rho2));
-                const R s2 = dv(rhou2, rho2) + c2;
-                bool add = true;
-                if (s2 < R(0) && s3 > R(0)) sfract = dv(s2 * (s3 - s[3]), s3 - s2);
-                else if (s[3] < R(0)) sfract = s[3];
-                else add = false;
+                bool add = s[3] < R(0);
+                sfract = s[3];
+                if (sizeof(R) == 4 || near_sonic(rho2, rhou2, rhov2, en2, gamma, gamma1)) {
+                    const R p2 = gamma1 * (en2 - dv(R(0.5) * mad(rhov2, rhov2, rhou2 * rhou2), rho2));
+                    const R c2 = sq(dv(gamma * p2, rho2));
+                    const R s2 = dv(rhou2, rho2) + c2;
+                    if (s2 < R(0) && s3 > R(0)) {
+                        sfract = dv(s2 * (s3 - s[3]), s3 - s2);
+                        add = true;
+                    }
+                }
                 if (add) {
 #pragma unroll
                     for (int m = 0; m < 4; m++) amdq[m] = mad(sfract, wave[3][m], amdq[m]);
@@ -610,8 +834,8 @@ struct RPEuler {
                 b[mv] = mad(v, b[0], d);
                 b[3] = mad(enth, t, mad(v, d, mad(0.5f * u2v2, y3, u * y2)));
             };
-            split(rmin(v - a, 0.0f), rmin(v, 0.0f), rmin(v + a, 0.0f), bm);
-            split(rmax(v - a, 0.0f), rmax(v, 0.0f), rmax(v + a, 0.0f), bp);
+            split(rneg(v - a), rneg(v), rneg(v + a), bm);
+            split(rplus(v - a), rplus(v), rplus(v + a), bp);
             return;
         }
         const R a4 = dv(t4, R(2) * a);
@@ -625,15 +849,25 @@ struct RPEuler {
         wb[2][3] = a4 * (enth + v * a); sb[2] = v + a;
 #pragma unroll
         for (int m = 0; m < 4; m++) {
-            R m_ = rmin(sb[0], R(0)) * wb[0][m], p_ = rmax(sb[0], R(0)) * wb[0][m];
+            R m_ = rneg(sb[0]) * wb[0][m], p_ = rplus(sb[0]) * wb[0][m];
 #pragma unroll
             for (int mw = 1; mw < 3; mw++) {
-                m_ = m_ + rmin(sb[mw], R(0)) * wb[mw][m];
-                p_ = p_ + rmax(sb[mw], R(0)) * wb[mw][m];
+                m_ = m_ + rneg(sb[mw]) * wb[mw][m];
+                p_ = p_ + rplus(sb[mw]) * wb[mw][m];
             }
             bm[m] = m_;
             bp[m] = p_;
         }
+    }
+
+    // both fluctuations of an interface (one quotient each)
+    template <int IXY>
+    __device__ __forceinline__ static void rpt2_pair(const double roe[NROE], const double amdq[MEQN],
+                                                     const double apdq[MEQN], bool /*fast*/, double bmA[MEQN],
+                                                     double bpA[MEQN], double bmP[MEQN], double bpP[MEQN]) {
+        const PhysParams none{};
+        rpt2<IXY>(roe, amdq, nullptr, nullptr, nullptr, none, bmA, bpA);
+        rpt2<IXY>(roe, apdq, nullptr, nullptr, nullptr, none, bmP, bpP);
     }
 
     template <int IXY>
@@ -698,8 +932,8 @@ struct RPAdvection {
         const R delta = qR[0] - qL[0];
         wave[0][0] = delta;
         s[0] = auxR[IXY - 1];
-        amdq[0] = R(0) + rmin(s[0], R(0)) * wave[0][0];
-        apdq[0] = R(0) + rmax(s[0], R(0)) * wave[0][0];
+        amdq[0] = R(0) + rneg(s[0]) * wave[0][0];
+        apdq[0] = R(0) + rplus(s[0]) * wave[0][0];
         roe[0] = R(0);
     }
 
@@ -708,8 +942,8 @@ struct RPAdvection {
                                                 const R* /*aux1*/, const R* aux2, const R* aux3,
                                                 const PhysParams&, R bm[MEQN], R bp[MEQN]) {
         constexpr int kv = IXY == 1 ? 1 : 0;   // the transverse velocity component
-        bm[0] = rmin(aux2[kv], R(0)) * asdq[0];
-        bp[0] = rmax(aux3[kv], R(0)) * asdq[0];
+        bm[0] = rneg(aux2[kv]) * asdq[0];
+        bp[0] = rplus(aux3[kv]) * asdq[0];
     }
 
     template <int IXY>

@@ -117,7 +117,7 @@ __device__ __forceinline__ R philim(int mth, R r) {
     case 3: return dv(r + fabs(r), R(1) + fabs(r));
     case 4: {
         const R c = dv(R(1) + r, R(2));
-        return rmax(R(0), rmin(rmin(c, R(2)), R(2) * r));
+        return rpos0(rmin(rcap(c, R(2)), R(2) * r));
     }
     case 5: return r;
     case 6: {

@@ -52,13 +52,13 @@ __device__ __forceinline__ void limited_correction(const StepArgs& a, const R wa
 #pragma unroll
         for (int m = 0; m < MEQN; m++)
             if (!WZ::at(mw, m)) sum_term(wn, wave[mw][m], wave[mw][m], first);
-        const R d = s[mw] > R(0) ? +dotl[mw] : +dotr[mw];
+        const R d = pick(s[mw] > R(0), dotl[mw], dotr[mw]);
         if constexpr (sizeof(R) == 4) {
             const float r = d * __builtin_amdgcn_rcpf(rmax(wn, 1.17549435e-38f));
             phi[mw] = STD ? rmax(0.0f, rmin(rmin(mad(0.5f, r, 0.5f), 2.0f), 2.0f * r)) : philim<float>(mth, r);
         } else {
             const R rr = dv(d, wn);
-            phi[mw] = wave_nonzero(wn) ? philim<R>(mth, rr) : R(1);
+            phi[mw] = pick(wave_nonzero(wn), philim<R>(mth, rr), R(1));
         }
     }
     R c[MW];
@@ -134,6 +134,7 @@ step_strips(StepArgs a, StripShape sh) {
     constexpr int U = sizeof(R) == 4 && explicit_fma<RP>::value ? 2 : 1;
     // FP32 with a linear rpt2: the factor dt / (2 dx) goes on asdq
     constexpr bool PRE = sizeof(R) == 4 && rpt2_linear<RP>::value;
+    constexpr bool RANGED = ranged<RP>::value;
     using WZ1 = wave_zeros<RP, 1>;
     using WZ2 = wave_zeros<RP, 2>;
 
@@ -247,6 +248,7 @@ step_strips(StepArgs a, StripShape sh) {
     R tu[2][MEQN], fxm[2][MEQN], fxp[2][MEQN];
     R gPd[2][MEQN], gPu[2][MEQN], gpl[2][MEQN];
     double G[2][MEQN];
+    bool inA = false, inB = false, inC = false;   // every lane's cell of the row is in range (RP::RANGED)
     R smaxx = R(0), smaxy = R(0);         // largest |s| of every interface the lane solves
     const R halfx = R(0.5) * dtdx, halfy = R(0.5) * dtdy;
 
@@ -313,8 +315,13 @@ step_strips(StepArgs a, StripShape sh) {
                 R q[MEQN];
 #pragma unroll
                 for (int m = 0; m < MEQN; m++) q[m] = (R) qr[C][m];
-                RP::template cell<1>(q, a.pp, cx[P]);
-                RP::template cell<2>(q, a.pp, cy[P]);
+                if constexpr (RANGED) {
+                    inC = all_lanes(RP::in_range(q, a.pp));
+                    RP::cells(q, a.pp, inC, cx[P], cy[P]);
+                } else {
+                    RP::template cell<1>(q, a.pp, cx[P]);
+                    RP::template cell<2>(q, a.pp, cy[P]);
+                }
             }
 
             // ---- x sweep of row B (n - 1) ----
@@ -330,7 +337,10 @@ step_strips(StepArgs a, StripShape sh) {
                     R cL[NCD];
 #pragma unroll
                     for (int c = 0; c < NC; c++) cL[c] = prev_lane(cx[O][c]);
-                    RP::template rpn2c<1>(qL, qR, cL, cx[O], auxL, ar[B], a.pp, w, s, amdq, apdq, roe);
+                    if constexpr (RANGED)
+                        RP::template rpn2c<1>(qL, qR, cL, cx[O], auxL, ar[B], a.pp, w, s, amdq, apdq, roe, inB);
+                    else
+                        RP::template rpn2c<1>(qL, qR, cL, cx[O], auxL, ar[B], a.pp, w, s, amdq, apdq, roe);
                 } else {
                     RP::template rpn2<1>(qL, qR, auxL, ar[B], a.pp, w, s, amdq, apdq, roe);
                 }
@@ -377,8 +387,12 @@ step_strips(StepArgs a, StripShape sh) {
                         a1[m] = MAUX > 0 ? prev_lane(ar[A][m]) : R(0);
                         a3[m] = MAUX > 0 ? prev_lane(ar[C][m]) : R(0);
                     }
-                    RP::template rpt2<1>(roe, amdq, a1, auxL, a3, a.pp, bmA, bpA);
-                    RP::template rpt2<1>(roe, apdq, ar[A], ar[B], ar[C], a.pp, bmP, bpP);
+                    if constexpr (RANGED) {
+                        RP::template rpt2_pair<1>(roe, amdq, apdq, inB, bmA, bpA, bmP, bpP);
+                    } else {
+                        RP::template rpt2<1>(roe, amdq, a1, auxL, a3, a.pp, bmA, bpA);
+                        RP::template rpt2<1>(roe, apdq, ar[A], ar[B], ar[C], a.pp, bmP, bpP);
+                    }
 #pragma unroll
                     for (int m = 0; m < MEQN; m++) {
                         const R gAd = PRE ? bmA[m] : halfx * bmA[m], gAu = PRE ? bpA[m] : halfx * bpA[m];
@@ -399,7 +413,9 @@ step_strips(StepArgs a, StripShape sh) {
                 R qL[MEQN], qR[MEQN];
 #pragma unroll
                 for (int m = 0; m < MEQN; m++) { qL[m] = (R) qr[B][m]; qR[m] = (R) qr[C][m]; }
-                if constexpr (NC > 0)
+                if constexpr (RANGED)
+                    RP::template rpn2c<2>(qL, qR, cy[O], cy[P], ar[B], ar[C], a.pp, wv[P], sv[P], am[P], apq[P], ro[P], inB && inC);
+                else if constexpr (NC > 0)
                     RP::template rpn2c<2>(qL, qR, cy[O], cy[P], ar[B], ar[C], a.pp, wv[P], sv[P], am[P], apq[P], ro[P]);
                 else
                     RP::template rpn2<2>(qL, qR, ar[B], ar[C], a.pp, wv[P], sv[P], am[P], apq[P], ro[P]);
@@ -453,19 +469,21 @@ step_strips(StepArgs a, StripShape sh) {
 #pragma unroll
                         for (int m = 0; m < MEQN; m++) { amdq[m] = halfy * amdq[m]; apdq[m] = halfy * apdq[m]; }
                     }
-                    R a1[MAD], a3[MAD];
+                    // the rows below and above the interface, left and right of the cell
+                    R lA[MAD], rA[MAD], lB[MAD], rB[MAD];
 #pragma unroll
                     for (int m = 0; m < MAD; m++) {
-                        a1[m] = MAUX > 0 ? prev_lane(ar[A][m]) : R(0);
-                        a3[m] = MAUX > 0 ? next_lane(ar[A][m]) : R(0);
+                        lA[m] = MAUX > 0 ? prev_lane(ar[A][m]) : R(0);
+                        rA[m] = MAUX > 0 ? next_lane(ar[A][m]) : R(0);
+                        lB[m] = MAUX > 0 ? prev_lane(ar[B][m]) : R(0);
+                        rB[m] = MAUX > 0 ? next_lane(ar[B][m]) : R(0);
                     }
-                    RP::template rpt2<2>(ro[O], amdq, a1, ar[A], a3, a.pp, nAd, nAu);
-#pragma unroll
-                    for (int m = 0; m < MAD; m++) {
-                        a1[m] = MAUX > 0 ? prev_lane(ar[B][m]) : R(0);
-                        a3[m] = MAUX > 0 ? next_lane(ar[B][m]) : R(0);
+                    if constexpr (RANGED) {
+                        RP::template rpt2_pair<2>(ro[O], amdq, apdq, inA && inB, nAd, nAu, gPd[P], gPu[P]);
+                    } else {
+                        RP::template rpt2<2>(ro[O], amdq, lA, ar[A], rA, a.pp, nAd, nAu);
+                        RP::template rpt2<2>(ro[O], apdq, lB, ar[B], rB, a.pp, gPd[P], gPu[P]);
                     }
-                    RP::template rpt2<2>(ro[O], apdq, a1, ar[B], a3, a.pp, gPd[P], gPu[P]);
                     if constexpr (!PRE) {
 #pragma unroll
                         for (int m = 0; m < MEQN; m++) {
@@ -597,6 +615,8 @@ step_strips(StepArgs a, StripShape sh) {
                 }
                 qo += nxp;
             }
+            inA = inB;
+            inB = inC;
             j++;
         }
         if constexpr (U == 2) {
