@@ -82,12 +82,12 @@ struct FaceRel {
 };
 
 // One launch of the fused ghost fill and time-sync increments: ghost ops
-// [ncorner0, ncorner0 + nbig) of g.ops one wave each, the corner ops
-// [0, ncorner0) and [ncorner0 + nbig, ... + ncorner1) four to a wave, then
-// sync ops [0, nsync) of sops one wave each.
+// [ncorner0, ncorner0 + nbig) of g.ops `parts` waves each (set by the launch), the
+// corner ops [0, ncorner0) and [ncorner0 + nbig, ... + ncorner1) four to a wave,
+// then sync ops [0, nsync) of sops several to a wave.
 struct FlatArgs {
     GhostArgs g;
-    int ncorner0, nbig, ncorner1;
+    int ncorner0, nbig, ncorner1, parts;
     const FaceRel* frel;       // [slot][4]
     const int* sops;           // [nsync][8] as SyncArgs::ops
     int nsync;

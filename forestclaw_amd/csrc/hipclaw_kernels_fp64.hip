@@ -37,15 +37,23 @@ __device__ __forceinline__ void interp_cell(const double* qc, double* qf, int m,
     qf[QIX(fi + 1, fj + 1, m)] = c + gx * 0.25 + gy * 0.25;
 }
 
+// e / d of small numbers: e + 1/2 times the reciprocal is at least 1 / (2 d) off
+// every whole number, and its error stays below that for e < 2^21 (a general
+// 32-bit division is some 20 instructions).
+struct SmallDiv {
+    float r;
+    __device__ __forceinline__ explicit SmallDiv(int d) : r(__builtin_amdgcn_rcpf((float) d)) {}
+    __device__ __forceinline__ int operator()(int e) const { return (int) (((float) e + 0.5f) * r); }
+};
+
 // One wave per ghost op, OPW ops (waves) per workgroup.  Ops of one phase
 // write disjoint ghost cells and read only cells no op of the phase writes,
 // so each lane issues the loads of up to U elements before their stores: the
 // source and destination slabs are the same allocation, and without this the
 // compiler must wait for every store before the next load.
-// W lanes (t = 0..W-1) work on the op: a whole wave, or a quarter of one for
+// W lanes (t = 0..W-1) work on the op: a wave, several, or a quarter of one for
 // the corner ops of the fused launch.
-template <int W = 64>
-__device__ __forceinline__ void ghost_exchange_op(const GhostArgs& g, const GhostOp& op, int t) {
+__device__ __forceinline__ void ghost_exchange_op(const GhostArgs& g, const GhostOp& op, int t, int W = 64) {
     const int mx = g.mx, my = g.my, mbc = g.mbc, meqn = g.meqn;
     const int nxp = mx + 2 * mbc, nyp = my + 2 * mbc;
     const int TI = HIPCLAW_TIME_INTERP_SLOT;
@@ -59,6 +67,7 @@ __device__ __forceinline__ void ghost_exchange_op(const GhostArgs& g, const Ghos
         const bool face = op.type == GHOST_COPY_FACE;
         const int len = (op.which < 2) ? my : mx;
         const int n = face ? meqn * mbc * len : meqn * mbc * mbc;
+        const SmallDiv by_field(face ? mbc * len : mbc * mbc), by_mbc(mbc);
         for (int base = t; base < n; base += W * U) {
             double v[U];
             long long di[U];
@@ -69,16 +78,16 @@ __device__ __forceinline__ void ghost_exchange_op(const GhostArgs& g, const Ghos
                 if (e >= n) continue;
                 int m, i1, j1;
                 if (face) {
-                    m = e / (mbc * len);
-                    const int r = e - m * mbc * len, l = r / mbc, bb = r - l * mbc;  // ghost layer 0..mbc-1
+                    m = by_field(e);
+                    const int r = e - m * mbc * len, l = by_mbc(r), bb = r - l * mbc;  // ghost layer 0..mbc-1
                     if (op.which == 0) { i1 = 1 - mbc + bb; j1 = 1 + l; }
                     else if (op.which == 1) { i1 = mx + 1 + bb; j1 = 1 + l; }
                     else if (op.which == 2) { i1 = 1 + l; j1 = 1 - mbc + bb; }
                     else { i1 = 1 + l; j1 = my + 1 + bb; }
                 } else {
-                    m = e / (mbc * mbc);
-                    const int r = e - m * mbc * mbc;
-                    corner_cell(mx, my, op.which, r / mbc + 1, r % mbc + 1, i1, j1);
+                    m = by_field(e);
+                    const int r = e - m * mbc * mbc, l = by_mbc(r);
+                    corner_cell(mx, my, op.which, l + 1, r - l * mbc + 1, i1, j1);
                 }
                 v[u] = qs[QIX(i1 + op.ti, j1 + op.tj, m)];
                 di[u] = QIX(i1, j1, m);
@@ -94,6 +103,7 @@ __device__ __forceinline__ void ghost_exchange_op(const GhostArgs& g, const Ghos
         const bool face = op.type == GHOST_AVERAGE_FACE;
         const int len = (op.which < 2) ? my : mx;
         const int n = face ? meqn * mbc * len : meqn * mbc * mbc;
+        const SmallDiv by_field(face ? mbc * len : mbc * mbc), by_mbc(mbc);
         for (int base = t; base < n; base += W * U) {
             double v[U];
             long long di[U];
@@ -104,14 +114,14 @@ __device__ __forceinline__ void ghost_exchange_op(const GhostArgs& g, const Ghos
                 if (e >= n) continue;
                 int m, ic, jc;
                 if (face) {
-                    m = e / (mbc * len);
-                    const int r = e - m * mbc * len, l = r / mbc, bb = r - l * mbc + 1;  // ibc/jbc 1..mbc
+                    m = by_field(e);
+                    const int r = e - m * mbc * len, l = by_mbc(r), bb = r - l * mbc + 1;  // ibc/jbc 1..mbc
                     if (op.which < 2) { ic = (op.which == 0) ? 1 - bb : mx + bb; jc = 1 + l; }
                     else { ic = 1 + l; jc = (op.which == 2) ? 1 - bb : my + bb; }
                 } else {
-                    m = e / (mbc * mbc);
-                    const int r = e - m * mbc * mbc;
-                    corner_cell(mx, my, op.which, r / mbc + 1, r % mbc + 1, ic, jc);
+                    m = by_field(e);
+                    const int r = e - m * mbc * mbc, l = by_mbc(r);
+                    corner_cell(mx, my, op.which, l + 1, r - l * mbc + 1, ic, jc);
                 }
                 const int fi = 2 * ic - 1 + op.ti, fj = 2 * jc - 1 + op.tj;
                 // faces: only cells whose four children are interior to this fine grid
@@ -135,6 +145,7 @@ __device__ __forceinline__ void ghost_exchange_op(const GhostArgs& g, const Ghos
         const bool face = op.type == GHOST_INTERP_FACE;
         const int hb = mbc / 2;
         const int n = face ? meqn * hb * mx : meqn * hb * hb;  // the reference bounds the face loop by mx
+        const SmallDiv by_field(face ? hb * mx : hb * hb), by_hb(hb);
         constexpr int UI = 2;
         for (int base = t; base < n; base += W * UI) {
             double c[UI], gx[UI], gy[UI];
@@ -146,13 +157,13 @@ __device__ __forceinline__ void ghost_exchange_op(const GhostArgs& g, const Ghos
                 if (e >= n) continue;
                 int m, ic, jc;
                 if (face) {
-                    m = e / (hb * mx);
-                    const int r = e - m * hb * mx, l = r / hb, bb = r - l * hb + 1;
+                    m = by_field(e);
+                    const int r = e - m * hb * mx, l = by_hb(r), bb = r - l * hb + 1;
                     if (op.which < 2) { ic = (op.which == 0) ? bb : mx - bb + 1; jc = 1 + l; }
                     else { ic = 1 + l; jc = (op.which == 2) ? bb : my - bb + 1; }
                 } else {
-                    m = e / (hb * hb);
-                    const int r = e - m * hb * hb, ibc = r / hb + 1, jbc = r % hb + 1;
+                    m = by_field(e);
+                    const int r = e - m * hb * hb, l = by_hb(r), ibc = l + 1, jbc = r - l * hb + 1;
                     ic = (op.which & 1) ? mx - ibc + 1 : ibc;
                     jc = (op.which & 2) ? my - jbc + 1 : jbc;
                 }
@@ -207,6 +218,7 @@ __device__ __forceinline__ void physbc_op(const GhostArgs& g, const GhostOp& op)
         const int pair = pass & 1;
         const int len = pair == 0 ? my + 2 * mbc : mx + 2 * mbc;
         const int per = meqn * mbc * len, n = 2 * per;
+        const SmallDiv by_field(mbc * len), by_mbc(mbc);
         for (int base = threadIdx.x; base < n; base += PHYSBC_THREADS * U) {
             double v[U];
             long long di[U];
@@ -219,8 +231,8 @@ __device__ __forceinline__ void physbc_op(const GhostArgs& g, const GhostOp& op)
                 const int mth = (signed char) ((op.bc >> (8 * face)) & 0xff);
                 if (mth != 1 && mth != 3) continue;
                 const int f = e - (e >= per ? per : 0);
-                const int m = f / (mbc * len), r = f - m * mbc * len;
-                const int l = r / mbc, b = r - l * mbc + 1;
+                const int m = by_field(f), r = f - m * mbc * len;
+                const int l = by_mbc(r), b = r - l * mbc + 1;
                 int id, jd, is, js;
                 if (face < 2) {
                     jd = js = 1 - mbc + l;
@@ -273,115 +285,159 @@ __global__ void __launch_bounds__(PHYSBC_THREADS) ghost_groups(GhostArgs g, cons
 }
 
 // ---------------------------------------------------------------- fused ghost fill + sync
-// Cell (i, j) of patch `slot` as the ghost fill of this step leaves it, for an
-// interior cell or a face ghost cell that is not a corner and not filled by
-// interpolation: the neighbour's interior cell (same size), the average of the
-// fine child's four cells (fclaw2d_clawpatch46_average.f:61-174, the child
-// whose cells lie in its interior), or the physical BC of the patch's own
-// interior (clawpack46_bc2_default.f).  All of it reads interior cells only,
-// which no wave of the fused launch writes.
-__device__ double fused_cell_simple(const GhostArgs& g, const FaceRel* __restrict__ frel, int slot, int i,
-                                    int j, int m) {
+// The fused launch lasts as long as its longest chain of dependent loads, so
+// what an op reads is resolved in stages (the faces' relations, then all the
+// values), and an op's elements are spread over `parts` waves instead of being
+// taken in turn (flat_parts): shock-bubble FP64 on 2,740 patches of 16 x 16 16.4
+// -> 11.9 us per launch, dam break FP64 on 3,400 of 32 x 32 17.4 -> 13.8.
+
+// A face's relation; k: the face whose ghost strip holds (i, j), -1 for an
+// interior cell.
+__device__ __forceinline__ int strip_of(int mx, int my, int i, int j) {
+    return i < 1 ? 0 : i > mx ? 1 : j < 1 ? 2 : j > my ? 3 : -1;
+}
+__device__ __forceinline__ FaceRel load_rel(const FaceRel* __restrict__ frel, int slot, int k) {
+    const int4* p = (const int4*) (frel + 4 * (long long) slot + (k < 0 ? 0 : k));
+    const int4 a = p[0], b = p[1];
+    return FaceRel{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+}
+
+// Where cell (i, j) of patch `slot` comes from as the ghost fill of this step
+// leaves it, for an interior cell or a face ghost cell that is not a corner and
+// not filled by interpolation (r: the relation of its strip, k): the neighbour's
+// interior cell (same size), the average of the fine child's four cells
+// (fclaw2d_clawpatch46_average.f:61-174, the child whose cells lie in its
+// interior), or the physical BC of the patch's own interior
+// (clawpack46_bc2_default.f).  All of it reads interior cells only, which no wave
+// of the fused launch writes.
+struct CellRef {
+    const double* p;
+    enum Mode { value, negated, average, zero } mode;
+};
+__device__ __forceinline__ CellRef cell_ref(const GhostArgs& g, const FaceRel& r, int k, int slot, int i, int j, int m) {
     const int mx = g.mx, my = g.my, mbc = g.mbc;
     const int nxp = mx + 2 * mbc, nyp = my + 2 * mbc;
-    const double* qc = g.q + (long long) slot * g.pstride;
-    const int k = i < 1 ? 0 : i > mx ? 1 : j < 1 ? 2 : j > my ? 3 : -1;
-    if (k < 0) return qc[QIX(i, j, m)];
-    const FaceRel r = frel[4 * slot + k];
-    if (r.rel == FREL_SAME) return g.q[(long long) r.nb0 * g.pstride + QIX(i + r.ti0, j + r.tj0, m)];
-    if (r.rel == FREL_HALF) {
-        int fi = 2 * i - 1 + r.ti0, fj = 2 * j - 1 + r.tj0, nb = r.nb0;
-        if (fi < 1 || fi + 1 > mx || fj < 1 || fj + 1 > my) {
-            fi = 2 * i - 1 + r.ti1;
-            fj = 2 * j - 1 + r.tj1;
-            nb = r.nb1;
-            // one of the two children covers every cell of the face strip
-            if (fi < 1 || fi + 1 > mx || fj < 1 || fj + 1 > my) return 0.0;
-        }
-        const double* qs = g.q + (long long) nb * g.pstride;
-        double sum = 0;
-        sum = sum + qs[QIX(fi, fj, m)];
-        sum = sum + qs[QIX(fi + 1, fj, m)];
-        sum = sum + qs[QIX(fi, fj + 1, m)];
-        sum = sum + qs[QIX(fi + 1, fj + 1, m)];
-        return sum / 4.0;
-    }
-    // FREL_PHYS (the host admits nothing else where this is called): extrapolation
-    // copies the first interior cell, a wall mirrors the strip and negates the
-    // normal momentum
-    const int mth = r.bc;
-    int is = i, js = j, mn;
-    if (k == 0) { is = mth == 1 ? 1 : 1 - i; mn = 1; }
-    else if (k == 1) { is = mth == 1 ? mx : 2 * mx + 1 - i; mn = 1; }
-    else if (k == 2) { js = mth == 1 ? 1 : 1 - j; mn = 2; }
-    else { js = mth == 1 ? my : 2 * my + 1 - j; mn = 2; }
-    const double x = qc[QIX(is, js, m)];
-    return (mth == 3 && m == mn) ? -x : x;
-}
-
-// Interpolated value of coarse cell (ic, jc) of patch c at child (a, b) of its
-// 2 x 2 fine cells (fclaw2d_clawpatch46_interpolate.f:120-137), the coarse
-// neighbours read through fused_cell_simple.
-__device__ __forceinline__ double interp_child(const GhostArgs& g, const FaceRel* __restrict__ frel, int c,
-                                               int ic, int jc, int m, int a, int b) {
-    const double cc = fused_cell_simple(g, frel, c, ic, jc, m);
-    const double gx = amr_slope(cc - fused_cell_simple(g, frel, c, ic - 1, jc, m),
-                                fused_cell_simple(g, frel, c, ic + 1, jc, m) - cc);
-    const double gy = amr_slope(cc - fused_cell_simple(g, frel, c, ic, jc - 1, m),
-                                fused_cell_simple(g, frel, c, ic, jc + 1, m) - cc);
-    return cc + gx * (a ? 0.25 : -0.25) + gy * (b ? 0.25 : -0.25);
-}
-
-// fused_cell_simple, plus the face strips filled by interpolation from a coarser
-// patch (recomputed from the coarse patch's cells).
-__device__ double fused_cell(const GhostArgs& g, const FaceRel* __restrict__ frel, int slot, int i, int j,
-                             int m) {
-    const int mx = g.mx, my = g.my;
-    const int k = i < 1 ? 0 : i > mx ? 1 : j < 1 ? 2 : j > my ? 3 : -1;
+    CellRef c{nullptr, CellRef::value};
+    int from = slot, is = i, js = j;
     if (k >= 0) {
-        const FaceRel r = frel[4 * slot + k];
-        if (r.rel == FREL_DOUBLE) {
-            // fine cell (i, j) = child (a, b) of coarse cell (ic, jc):
-            // i = 2 ic - 1 + ti + a
-            const int u = i - r.ti0 + 1, v = j - r.tj0 + 1;
-            return interp_child(g, frel, r.nb0, u >> 1, v >> 1, m, u & 1, v & 1);
+        if (r.rel == FREL_SAME) {
+            from = r.nb0;
+            is = i + r.ti0;
+            js = j + r.tj0;
+        } else if (r.rel == FREL_HALF) {
+            c.mode = CellRef::average;
+            from = r.nb0;
+            is = 2 * i - 1 + r.ti0;
+            js = 2 * j - 1 + r.tj0;
+            if (is < 1 || is + 1 > mx || js < 1 || js + 1 > my) {
+                from = r.nb1;
+                is = 2 * i - 1 + r.ti1;
+                js = 2 * j - 1 + r.tj1;
+                // one of the two children covers every cell of the face strip
+                if (is < 1 || is + 1 > mx || js < 1 || js + 1 > my) c.mode = CellRef::zero;
+            }
+        } else {
+            // FREL_PHYS (the host admits nothing else where this is called):
+            // extrapolation copies the first interior cell, a wall mirrors the strip
+            // and negates the normal momentum
+            const int mth = r.bc;
+            if (k == 0) is = mth == 1 ? 1 : 1 - i;
+            else if (k == 1) is = mth == 1 ? mx : 2 * mx + 1 - i;
+            else if (k == 2) js = mth == 1 ? 1 : 1 - j;
+            else js = mth == 1 ? my : 2 * my + 1 - j;
+            if (mth == 3 && m == (k < 2 ? 1 : 2)) c.mode = CellRef::negated;
         }
     }
-    return fused_cell_simple(g, frel, slot, i, j, m);
+    c.p = g.q + (long long) from * g.pstride + QIX(is, js, m);
+    return c;
+}
+__device__ __forceinline__ void cell_loads(const CellRef& c, int nxp, double v[4]) {
+    v[0] = v[1] = v[2] = v[3] = 0.0;
+    if (c.mode != CellRef::zero) v[0] = c.p[0];
+    if (c.mode == CellRef::average) { v[1] = c.p[1]; v[2] = c.p[nxp]; v[3] = c.p[nxp + 1]; }
+}
+__device__ __forceinline__ double cell_value(const CellRef& c, const double v[4]) {
+    if (c.mode == CellRef::average) return ((((0.0 + v[0]) + v[1]) + v[2]) + v[3]) / 4.0;
+    return c.mode == CellRef::negated ? -v[0] : v[0];
+}
+
+// Interior coarse cell (ic, jc) of patch c and its slopes
+// (fclaw2d_clawpatch46_interpolate.f:120-137).
+__device__ __forceinline__ void coarse_cell(const GhostArgs& g, const FaceRel* __restrict__ frel, int c, int ic, int jc,
+                                            int m, double& cc, double& gx, double& gy) {
+    constexpr int DI[4] = {-1, 1, 0, 0}, DJ[4] = {0, 0, -1, 1};
+    const int nxp = g.mx + 2 * g.mbc, nyp = g.my + 2 * g.mbc, mbc = g.mbc;
+    FaceRel r[4];
+    int k[4];
+#pragma unroll
+    for (int d = 0; d < 4; d++) {
+        k[d] = strip_of(g.mx, g.my, ic + DI[d], jc + DJ[d]);
+        r[d] = FaceRel{};
+        if (k[d] >= 0) r[d] = load_rel(frel, c, k[d]);
+    }
+    cc = g.q[(long long) c * g.pstride + QIX(ic, jc, m)];
+    CellRef n[4];
+    double v[4][4], x[4];
+#pragma unroll
+    for (int d = 0; d < 4; d++) {
+        n[d] = cell_ref(g, r[d], k[d], c, ic + DI[d], jc + DJ[d], m);
+        cell_loads(n[d], nxp, v[d]);
+    }
+#pragma unroll
+    for (int d = 0; d < 4; d++) x[d] = cell_value(n[d], v[d]);
+    gx = amr_slope(cc - x[0], x[1] - cc);
+    gy = amr_slope(cc - x[2], x[3] - cc);
+}
+
+// A cell as cell_ref's, or of a face strip that is filled by interpolation from a
+// coarser patch (recomputed from the coarse patch's cells).
+__device__ __forceinline__ double fused_cell(const GhostArgs& g, const FaceRel* __restrict__ frel, int slot, int i,
+                                             int j, int m) {
+    const int k = strip_of(g.mx, g.my, i, j);
+    FaceRel r{};
+    if (k >= 0) r = load_rel(frel, slot, k);
+    if (k >= 0 && r.rel == FREL_DOUBLE) {
+        // fine cell (i, j) = child (a, b) of coarse cell (ic, jc):
+        // i = 2 ic - 1 + ti + a
+        const int u = i - r.ti0 + 1, v = j - r.tj0 + 1;
+        double cc, gx, gy;
+        coarse_cell(g, frel, r.nb0, u >> 1, v >> 1, m, cc, gx, gy);
+        return cc + gx * (u & 1 ? 0.25 : -0.25) + gy * (v & 1 ? 0.25 : -0.25);
+    }
+    const CellRef c = cell_ref(g, r, k, slot, i, j, m);
+    double v[4];
+    cell_loads(c, g.mx + 2 * g.mbc, v);
+    return cell_value(c, v);
 }
 
 // Interpolation op (dst = fine, src = coarse) as in ghost_exchange_op, its
-// coarse-side reads through fused_cell_simple.
-template <int W = 64>
-__device__ void fused_interp_op(const GhostArgs& g, const FaceRel* __restrict__ frel, const GhostOp& op,
-                                int t) {
+// coarse-side reads resolved by cell_ref.
+__device__ __forceinline__ void fused_interp_op(const GhostArgs& g, const FaceRel* __restrict__ frel, const GhostOp& op,
+                                                int t, int W) {
     const int mx = g.mx, my = g.my, mbc = g.mbc, meqn = g.meqn;
     const int nxp = mx + 2 * mbc, nyp = my + 2 * mbc;
     double* qd = g.q + (long long) op.dst * g.pstride;
     const bool face = op.type == GHOST_INTERP_FACE;
     const int hb = mbc / 2;
     const int n = face ? meqn * hb * mx : meqn * hb * hb;
+    const SmallDiv by_field(face ? hb * mx : hb * hb), by_hb(hb);
     for (int e = t; e < n; e += W) {
         int m, ic, jc;
         if (face) {
-            m = e / (hb * mx);
-            const int r = e - m * hb * mx, l = r / hb, bb = r - l * hb + 1;
+            m = by_field(e);
+            const int r = e - m * hb * mx, l = by_hb(r), bb = r - l * hb + 1;
             if (op.which < 2) { ic = (op.which == 0) ? bb : mx - bb + 1; jc = 1 + l; }
             else { ic = 1 + l; jc = (op.which == 2) ? bb : my - bb + 1; }
         } else {
-            m = e / (hb * hb);
-            const int r = e - m * hb * hb, ibc = r / hb + 1, jbc = r % hb + 1;
+            m = by_field(e);
+            const int r = e - m * hb * hb, l = by_hb(r), ibc = l + 1, jbc = r - l * hb + 1;
             ic = (op.which & 1) ? mx - ibc + 1 : ibc;
             jc = (op.which & 2) ? my - jbc + 1 : jbc;
         }
         const int fi = 2 * ic - 1 + op.ti, fj = 2 * jc - 1 + op.tj;
         if (face && (fi < 1 - mbc || fi + 1 > mx + mbc || fj < 1 - mbc || fj + 1 > my + mbc)) continue;
-        const int c = op.src;
-        const double cc = fused_cell_simple(g, frel, c, ic, jc, m);
-        const double gx = amr_slope(cc - fused_cell_simple(g, frel, c, ic - 1, jc, m),
-                                    fused_cell_simple(g, frel, c, ic + 1, jc, m) - cc);
-        const double gy = amr_slope(cc - fused_cell_simple(g, frel, c, ic, jc - 1, m),
-                                    fused_cell_simple(g, frel, c, ic, jc + 1, m) - cc);
+        double cc, gx, gy;
+        coarse_cell(g, frel, op.src, ic, jc, m, cc, gx, gy);
         const long long d0 = QIX(fi, fj, m);
         qd[d0] = cc + gx * -0.25 + gy * -0.25;
         qd[d0 + 1] = cc + gx * 0.25 + gy * -0.25;
@@ -390,12 +446,13 @@ __device__ void fused_interp_op(const GhostArgs& g, const FaceRel* __restrict__ 
     }
 }
 
-// Physical BC of one patch by one wave (clawpack46_bc2_default.f), each ghost
+// Physical BC of one patch (clawpack46_bc2_default.f), each ghost
 // cell written once with its final value: the sources are interior cells or
 // ghost cells of a neighbouring face strip, recomputed through fused_cell, and
 // a corner both of whose faces are physical takes the y-face's value (the
 // reference applies faces 2 and 3 after faces 0 and 1).
-__device__ void fused_physbc_op(const GhostArgs& g, const FaceRel* __restrict__ frel, const GhostOp& op, int t) {
+__device__ __forceinline__ void fused_physbc_op(const GhostArgs& g, const FaceRel* __restrict__ frel, const GhostOp& op, int t,
+                                                int W) {
     const int mx = g.mx, my = g.my, mbc = g.mbc, meqn = g.meqn;
     const int nxp = mx + 2 * mbc, nyp = my + 2 * mbc;
     double* qd = g.q + (long long) op.dst * g.pstride;
@@ -407,9 +464,10 @@ __device__ void fused_physbc_op(const GhostArgs& g, const FaceRel* __restrict__ 
         const int mth = code(face);
         const int len = face < 2 ? my + 2 * mbc : mx + 2 * mbc;
         const int n = meqn * mbc * len;
-        for (int e = t; e < n; e += 64) {
-            const int m = e / (mbc * len), r = e - m * mbc * len;
-            const int l = r / mbc, b = r - l * mbc + 1;
+        const SmallDiv by_field(mbc * len), by_mbc(mbc);
+        for (int e = t; e < n; e += W) {
+            const int m = by_field(e), r = e - m * mbc * len;
+            const int l = by_mbc(r), b = r - l * mbc + 1;
             int id, jd, is, js;
             if (face < 2) {
                 jd = js = 1 - mbc + l;
@@ -429,57 +487,86 @@ __device__ void fused_physbc_op(const GhostArgs& g, const FaceRel* __restrict__ 
     }
 }
 
-// Time-sync increments of one op (as time_sync_cells): a same-size op writes
-// every position of its face, a coarse/fine op the positions its fine patch
-// covers (the other child's op writes the rest; the reference adds zero for
-// the positions a child does not cover).
-__device__ void fused_sync_op(const FlatArgs& f, const int* __restrict__ op, int t) {
-    const int mx = f.g.mx, meqn = f.g.meqn;
-    const int type = op[0], dst = op[1], src = op[2], face = op[3], ti = op[4], tj = op[5];
-    const double area = f.dxs[dst] * f.dys[dst];
-    const double* __restrict__ rt = f.reg + (long long) dst * f.rstride;
-    const double* __restrict__ rn = f.reg + (long long) src * f.rstride;
-    double* __restrict__ qo = f.qinc + (long long) dst * f.cstride;
+// Time-sync increments (as time_sync_cells): a same-size op writes every
+// position of its face, a coarse/fine op the positions its fine patch covers
+// (the other child's op writes the rest; the reference adds zero for the
+// positions a child does not cover).  A wave takes the positions of `ops`
+// consecutive ops, up to SYNC_ITEMS per lane, in two stages of loads: the ops,
+// then sizes and registers.  An op at a time is a chain of memory latencies for
+// little more than one load per lane (whole launch, dam break FP32 on 11,296
+// patches of 32 x 32, items 1, 2, 3, 4: 37, 35, 32, 35 us, of which the
+// registers' and increments' 70 MB need 14; ensemble of 64 runs 61, 62, 58, 66).
+constexpr int SYNC_ITEMS = 3;
+__device__ void fused_sync_ops(const FlatArgs& f, int op0, int ops, int t) {
+    const int mx = f.g.mx, meqn = f.g.meqn, per = meqn * mx;
+    const int n = min(ops, f.nsync - op0) * per;
     const int kout = f.fluxreg ? REG_EFIN : REG_EFOUT;
-    const int kn = face ^ 1;
-    const int kfl = (face == 0 || face == 2) ? REG_FP : REG_FM;
-    for (int e = t; e < meqn * mx; e += 64) {
-        const int m = e / mx, c = e - m * mx + 1;
-        auto R = [&](const double* rr, int kk, int kind, int pos) -> double {
-            return rr[((kk * 4 + kind) * meqn + m) * mx + pos];
-        };
-        const double ein = R(rt, face, REG_EFIN, c - 1);
-        const double ft = f.fluxreg ? 0.0 : R(rt, face, kfl, c - 1);
-        double v;
-        if (type != SYNC_F2C) {
-            const double ef = R(rn, kn, kout, c - 1);
-            const double fn = f.fluxreg ? 0.0 : R(rn, kn, kfl, c - 1);
-            const double delta = (face == 0 || face == 2) ? (ef - ein) - (fn - ft) : (ein - ef) - (fn - ft);
-            v = 0.5 * delta / area;
+    const SmallDiv by_per(per), by_mx(mx);
+    for (int base = t; base < n; base += 64 * SYNC_ITEMS) {
+        int type[SYNC_ITEMS], dst[SYNC_ITEMS], src[SYNC_ITEMS], face[SYNC_ITEMS], m[SYNC_ITEMS], c[SYNC_ITEMS], f0[SYNC_ITEMS];
+        bool on[SYNC_ITEMS];
+        int4 lo[SYNC_ITEMS];
+        int2 hi[SYNC_ITEMS];
+#pragma unroll
+        for (int u = 0; u < SYNC_ITEMS; u++) {
+            const int e = min(base + 64 * u, n - 1);
+            const int o = by_per(e), r = e - o * per;
+            m[u] = by_mx(r);
+            c[u] = r - m[u] * mx;
+            const int* op = f.sops + 8 * (long long) (op0 + o);
+            lo[u] = *(const int4*) op;
+            hi[u] = *(const int2*) (op + 4);
+        }
+        double ein[SYNC_ITEMS], ft[SYNC_ITEMS], ef[SYNC_ITEMS], ef2[SYNC_ITEMS], fn[SYNC_ITEMS], fn2[SYNC_ITEMS];
+        double area[SYNC_ITEMS], area_src[SYNC_ITEMS];
+#pragma unroll
+        for (int u = 0; u < SYNC_ITEMS; u++) {
+            type[u] = lo[u].x; dst[u] = lo[u].y; src[u] = lo[u].z; face[u] = lo[u].w;
+            const bool f2c = type[u] == SYNC_F2C;
+            f0[u] = f2c ? 2 * c[u] + (face[u] < 2 ? hi[u].y : hi[u].x) : c[u];   // 0-based position on src
+            on[u] = base + 64 * u < n && (!f2c || (f0[u] >= 0 && f0[u] + 1 < mx));
+            ein[u] = ft[u] = ef[u] = ef2[u] = fn[u] = fn2[u] = 0.0;
+            area[u] = area_src[u] = 1.0;
+            if (on[u]) {
+                const int kfl = (face[u] == 0 || face[u] == 2) ? REG_FP : REG_FM;
+                const double* __restrict__ rt = f.reg + (long long) dst[u] * f.rstride + (face[u] * 4 * meqn + m[u]) * mx + c[u];
+                const double* __restrict__ rn = f.reg + (long long) src[u] * f.rstride + ((face[u] ^ 1) * 4 * meqn + m[u]) * mx + f0[u];
+                area[u] = f.dxs[dst[u]] * f.dys[dst[u]];
+                ein[u] = rt[REG_EFIN * per];
+                ef[u] = rn[kout * per];
+                if (f2c) ef2[u] = rn[kout * per + 1];
+                if (!f.fluxreg) {
+                    ft[u] = rt[kfl * per];
+                    fn[u] = rn[kfl * per];
+                    if (f2c) fn2[u] = rn[kfl * per + 1];
+                }
+                if (type[u] == SYNC_SAMESIZE_PAIR) area_src[u] = f.dxs[src[u]] * f.dys[src[u]];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < SYNC_ITEMS; u++) {
+            if (!on[u]) continue;
+            const bool f2c = type[u] == SYNC_F2C;
+            if (f2c) { ef[u] = ef[u] + ef2[u]; fn[u] = fn[u] + fn2[u]; }
+            const double delta = (face[u] == 0 || face[u] == 2) ? (ef[u] - ein[u]) - (fn[u] - ft[u])
+                                                                : (ein[u] - ef[u]) - (fn[u] - ft[u]);
+            const double v = (f2c ? delta : 0.5 * delta) / area[u];
+            const int pos = m[u] * mx + c[u];
+            f.qinc[(long long) dst[u] * f.cstride + face[u] * per + pos] = 0.0 + v;
             // the partner's op (dst and src swapped, face ^ 1) would compute the
             // same delta: it reads these two registers and takes their
             // difference in the same order (the FP32 flux form stores no
             // fluctuations, fn = ft = 0)
-            if (type == SYNC_SAMESIZE_PAIR) {
-                const double area_src = f.dxs[src] * f.dys[src];
-                f.qinc[(long long) src * f.cstride + (kn * meqn + m) * mx + c - 1] = 0.0 + 0.5 * delta / area_src;
-            }
-        } else {
-            const int f0 = 2 * c - 1 + (face < 2 ? tj : ti);
-            if (f0 < 1 || f0 + 1 > mx) continue;
-            const double ef = R(rn, kn, kout, f0 - 1) + R(rn, kn, kout, f0);
-            const double flu = f.fluxreg ? 0.0 : R(rn, kn, kfl, f0 - 1) + R(rn, kn, kfl, f0);
-            const double deltac = (face == 0 || face == 2) ? (ef - ein) - (flu - ft) : (ein - ef) - (flu - ft);
-            v = deltac / area;
+            if (type[u] == SYNC_SAMESIZE_PAIR)
+                f.qinc[(long long) src[u] * f.cstride + (face[u] ^ 1) * per + pos] = 0.0 + 0.5 * delta / area_src[u];
         }
-        qo[(face * meqn + m) * mx + c - 1] = 0.0 + v;
     }
 }
 
 // The fused launch, no op depending on another: ghost ops (copies and
 // averages read interior cells; interpolations and physical BCs recompute the
-// ghost cells they read), then time-sync increments.  A face, physical-BC or
-// sync op takes a wave; the corner ops, a few cells each, take a quarter of
+// ghost cells they read), then time-sync increments.  A face or physical-BC op
+// takes a wave or several; the corner ops, a few cells each, take a quarter of
 // one.  The interior cells keep their values before the time sync, which
 // every ghost op reads (the reference fills ghost cells before it
 // synchronises, src/fclaw2d_advance.c:330-341); the next update adds the
@@ -488,19 +575,30 @@ constexpr int FLAT_OPW = 4;           // waves per workgroup
 constexpr int FLAT_CORNER_LANES = 16; // lanes of one corner op
 constexpr int FLAT_CORNERS = 64 / FLAT_CORNER_LANES;
 
-__device__ __forceinline__ int flat_corner_waves(int n) { return (n + FLAT_CORNERS - 1) / FLAT_CORNERS; }
+// Waves of one face or physical-BC op: one for every 64 ghost cells of a face and
+// field, so that no lane takes two.
+static int flat_parts(const GhostArgs& g) {
+    const int n = g.meqn * g.mbc * (std::max(g.mx, g.my) + 2 * g.mbc);
+    return std::min(4, (n + 63) / 64);
+}
+__host__ __device__ __forceinline__ int flat_corner_waves(int n) { return (n + FLAT_CORNERS - 1) / FLAT_CORNERS; }
+// Time-sync ops of one wave, per positions each: as many as its lanes take at once.
+__host__ __device__ __forceinline__ int flat_sync_ops(int per) {
+    return per < 64 * SYNC_ITEMS ? 64 * SYNC_ITEMS / per : 1;
+}
 
 __global__ void __launch_bounds__(64 * FLAT_OPW) ghost_flat(FlatArgs f) {
-    int w = blockIdx.x * FLAT_OPW + (int) (threadIdx.x >> 6);
+    int w = blockIdx.x * FLAT_OPW + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    if (w < f.nbig) {
-        const GhostOp op = f.g.ops[f.ncorner0 + w];
-        if (op.type == GHOST_INTERP_FACE || op.type == GHOST_INTERP_CORNER) fused_interp_op(f.g, f.frel, op, lane);
-        else if (op.type == GHOST_PHYSBC) fused_physbc_op(f.g, f.frel, op, lane);
-        else ghost_exchange_op(f.g, op, lane);
+    if (w < f.nbig * f.parts) {
+        const int o = w / f.parts, t = (w - o * f.parts) * 64 + lane, W = 64 * f.parts;
+        const GhostOp op = f.g.ops[f.ncorner0 + o];
+        if (op.type == GHOST_INTERP_FACE || op.type == GHOST_INTERP_CORNER) fused_interp_op(f.g, f.frel, op, t, W);
+        else if (op.type == GHOST_PHYSBC) fused_physbc_op(f.g, f.frel, op, t, W);
+        else ghost_exchange_op(f.g, op, t, W);
         return;
     }
-    w -= f.nbig;
+    w -= f.nbig * f.parts;
     const int nw0 = flat_corner_waves(f.ncorner0), nw1 = flat_corner_waves(f.ncorner1);
     if (w < nw0 + nw1) {
         // corner ops [0, ncorner0) and [ncorner0 + nbig, ... + ncorner1)
@@ -509,54 +607,55 @@ __global__ void __launch_bounds__(64 * FLAT_OPW) ghost_flat(FlatArgs f) {
         if (k < (first ? f.ncorner0 : f.ncorner1)) {
             const GhostOp op = f.g.ops[(first ? 0 : f.ncorner0 + f.nbig) + k];
             const int t = lane % FLAT_CORNER_LANES;
-            if (op.type == GHOST_INTERP_CORNER) fused_interp_op<FLAT_CORNER_LANES>(f.g, f.frel, op, t);
-            else ghost_exchange_op<FLAT_CORNER_LANES>(f.g, op, t);
+            if (op.type == GHOST_INTERP_CORNER) fused_interp_op(f.g, f.frel, op, t, FLAT_CORNER_LANES);
+            else ghost_exchange_op(f.g, op, t, FLAT_CORNER_LANES);
         }
         return;
     }
     w -= nw0 + nw1;
-    if (w < f.nsync) fused_sync_op(f, f.sops + 8 * w, lane);
+    const int ops = flat_sync_ops(f.g.meqn * f.g.mx);
+    if (w * ops < f.nsync) fused_sync_ops(f, w * ops, ops, lane);
 }
 
 // The pending increments added into the slab (after the last step of an
-// advance, so the state is the synchronised one), one thread per edge cell of
-// the patches listed in slots (those with a corrected face), in the update's
+// advance, so the state is the synchronised one), one workgroup per patch listed
+// in slots (those with a corrected face), in the update's
 // order: a corner cell belongs to its x-face when that face is
 // corrected, and takes both faces' increments in the reference's order.
 __global__ void apply_qcorr(double* __restrict__ q, const double* __restrict__ qcorr,
-                            const int* __restrict__ cmask, const int* __restrict__ slots, int n,
+                            const int* __restrict__ cmask, const int* __restrict__ slots,
                             long long pstride, long long cstride, int mx, int my, int mbc, int meqn) {
-    const int per = 4 * meqn * mx;
-    const long long e = (long long) blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (long long) n * per) return;
-    const int k = (int) (e / per), r = (int) (e - (long long) k * per);
-    const int slot = slots[k];
-    const int fc = r / (meqn * mx), r2 = r - fc * meqn * mx, m = r2 / mx, c = r2 - m * mx + 1;
-    const int mask = cmask[slot];
-    if (!((mask >> fc) & 1)) return;
-    const int len = fc < 2 ? my : mx;
-    const int other = (c == 1 || c == len) ? (fc < 2 ? (c == 1 ? 2 : 3) : (c == 1 ? 0 : 1)) : -1;
-    const bool other_on = other >= 0 && ((mask >> other) & 1);
-    if (fc >= 2 && other_on) return;
+    const int slot = slots[blockIdx.x], mask = cmask[slot];
+    const SmallDiv by_face(meqn * mx), by_mx(mx);
     const int nxp = mx + 2 * mbc, nyp = my + 2 * mbc;
-    const int i = fc == 0 ? 1 : fc == 1 ? mx : c, j = fc == 2 ? 1 : fc == 3 ? my : c;
     const double* qc = qcorr + (long long) slot * cstride;
-    const double v = qc[(fc * meqn + m) * len + c - 1];
-    double* cell = q + (long long) slot * pstride + QIX(i, j, m);
-    double x = *cell;
-    if (other_on) {
-        const double w = qc[(other * meqn + m) * mx + (fc == 0 ? 0 : mx - 1)];
-        if (sync_y_first(mask, fc, other)) { x = x + w; x = x + v; }
-        else { x = x + v; x = x + w; }
-    } else {
-        x = x + v;
+    for (int r = threadIdx.x; r < 4 * meqn * mx; r += blockDim.x) {
+        const int fc = by_face(r), r2 = r - fc * meqn * mx, m = by_mx(r2), c = r2 - m * mx + 1;
+        if (!((mask >> fc) & 1)) continue;
+        const int len = fc < 2 ? my : mx;
+        const int other = (c == 1 || c == len) ? (fc < 2 ? (c == 1 ? 2 : 3) : (c == 1 ? 0 : 1)) : -1;
+        const bool other_on = other >= 0 && ((mask >> other) & 1);
+        if (fc >= 2 && other_on) continue;
+        const int i = fc == 0 ? 1 : fc == 1 ? mx : c, j = fc == 2 ? 1 : fc == 3 ? my : c;
+        const double v = qc[(fc * meqn + m) * len + c - 1];
+        double* cell = q + (long long) slot * pstride + QIX(i, j, m);
+        double x = *cell;
+        if (other_on) {
+            const double w = qc[(other * meqn + m) * mx + (fc == 0 ? 0 : mx - 1)];
+            if (sync_y_first(mask, fc, other)) { x = x + w; x = x + v; }
+            else { x = x + v; x = x + w; }
+        } else {
+            x = x + v;
+        }
+        *cell = x;
     }
-    *cell = x;
 }
 
-int launch_ghost_flat(const FlatArgs& f, hipStream_t st) {
-    const int n = f.nbig + (f.ncorner0 + FLAT_CORNERS - 1) / FLAT_CORNERS +
-                  (f.ncorner1 + FLAT_CORNERS - 1) / FLAT_CORNERS + f.nsync;
+int launch_ghost_flat(const FlatArgs& args, hipStream_t st) {
+    FlatArgs f = args;
+    f.parts = flat_parts(f.g);
+    const int ops = flat_sync_ops(f.g.meqn * f.g.mx);
+    const int n = f.nbig * f.parts + flat_corner_waves(f.ncorner0) + flat_corner_waves(f.ncorner1) + (f.nsync + ops - 1) / ops;
     if (n <= 0) return 0;
     hipLaunchKernelGGL(ghost_flat, dim3((n + FLAT_OPW - 1) / FLAT_OPW), dim3(64 * FLAT_OPW), 0, st, f);
     return (int) hipGetLastError();
@@ -565,10 +664,9 @@ int launch_ghost_flat(const FlatArgs& f, hipStream_t st) {
 int launch_apply_qcorr(double* q, const double* qcorr, const int* cmask, const int* slots, int n,
                        long long pstride, long long cstride, int mx, int my, int mbc, int meqn,
                        hipStream_t st) {
-    const long long total = (long long) n * 4 * meqn * mx;
-    if (total <= 0) return 0;
-    hipLaunchKernelGGL(apply_qcorr, dim3((unsigned) ((total + 255) / 256)), dim3(256), 0, st, q, qcorr, cmask,
-                       slots, n, pstride, cstride, mx, my, mbc, meqn);
+    if (n <= 0) return 0;
+    hipLaunchKernelGGL(apply_qcorr, dim3(n), dim3(256), 0, st, q, qcorr, cmask,
+                       slots, pstride, cstride, mx, my, mbc, meqn);
     return (int) hipGetLastError();
 }
 
