@@ -2221,34 +2221,19 @@ int hipclaw_timing(hipclaw_state_t* s, int nsteps, double* total_ms, double* ste
     return HIPCLAW_OK;
 }
 
-static void two_sum_host(double a, double b, double& s, double& e) {
-    s = a + b;
-    const double bb = s - a;
-    e = (a - (s - bb)) + (b - bb);
-}
-
 int hipclaw_mass(hipclaw_state_t* s, double* sum_hi, double* sum_lo) {
     if (!s || !sum_hi) return fail(HIPCLAW_EINVAL, "hipclaw_mass: bad arguments%s");
     const int meqn = s->cfg.meqn;
+    char* host = nullptr;
+    if (int rc = stage_reserve(s, sizeof(double) * 2 * (size_t) meqn, &host)) return rc;
+    const double* sums = (const double*) host;
     int e = hipclaw::launch_mass(s->q[s->cur], s->all_slots, s->npatch, s->dxs, s->dys, s->pstride,
-                                 s->cfg.mx, s->cfg.my, s->cfg.mbc, meqn, s->mass_buf, s->st);
-    if (e) return hipfail((hipError_t) e, "patch_mass launch");
-    std::vector<double> buf(2 * (size_t) meqn * s->npatch);
-    if (!buf.empty())
-        HIP_TRY(hipMemcpyAsync(buf.data(), s->mass_buf, sizeof(double) * buf.size(), hipMemcpyDeviceToHost, s->st));
+                                 s->cfg.mx, s->cfg.my, s->cfg.mbc, meqn, s->mass_buf, (double*) host, s->st);
+    if (e) return hipfail((hipError_t) e, "mass launch");
     HIP_TRY(hipStreamSynchronize(s->st));
     for (int m = 0; m < meqn; m++) {
-        double hi = 0.0, lo = 0.0;
-        for (int p = 0; p < s->npatch; p++) {
-            double t, err;
-            two_sum_host(hi, buf[((size_t) p * meqn + m) * 2], t, err);
-            hi = t;
-            lo += err + buf[((size_t) p * meqn + m) * 2 + 1];
-        }
-        double t, err;
-        two_sum_host(hi, lo, t, err);
-        sum_hi[m] = t;
-        if (sum_lo) sum_lo[m] = err;
+        sum_hi[m] = sums[2 * m];
+        if (sum_lo) sum_lo[m] = sums[2 * m + 1];
     }
     return HIPCLAW_OK;
 }
@@ -2273,16 +2258,15 @@ int hipclaw_tag_patches(hipclaw_state_t* s, int ivar, double refine_threshold,
         return fail(HIPCLAW_EINVAL, "hipclaw_tag_patches: bad arguments%s");
     const int n = s->npatch;
     if (n == 0) return HIPCLAW_OK;
-    if (int rc = ensure_iwork(s, 2 * (size_t) n)) return rc;
-    int* dev = s->iwork;
+    // two ints per patch, straight into host memory
+    char* host = nullptr;
+    if (int rc = stage_reserve(s, sizeof(int) * 2 * (size_t) n, &host)) return rc;
+    const int* out = (const int*) host;
     int e = hipclaw::launch_tag_patches(s->q[s->cur], s->all_slots, n, s->dxs, s->dys, s->pstride,
                                         s->cfg.mx, s->cfg.my, s->cfg.mbc, ivar, refine_threshold,
-                                        coarsen_threshold, dev, s->st);
-    std::vector<int> out(2 * (size_t) n);
-    hipError_t he = e ? (hipError_t) e
-                      : hipMemcpyAsync(out.data(), dev, sizeof(int) * 2 * (size_t) n, hipMemcpyDeviceToHost, s->st);
-    if (he == hipSuccess) he = hipStreamSynchronize(s->st);
-    if (he != hipSuccess) return hipfail(he, "tag_patches");
+                                        coarsen_threshold, (int*) host, s->st);
+    if (e) return hipfail((hipError_t) e, "tag_patches launch");
+    HIP_TRY(hipStreamSynchronize(s->st));
     for (int p = 0; p < n; p++) {
         exceeds_refine[p] = out[2 * p];
         exceeds_coarsen[p] = out[2 * p + 1];

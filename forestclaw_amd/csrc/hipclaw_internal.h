@@ -104,6 +104,7 @@ struct FlatArgs {
 enum { REGRID_SAME = 0, REGRID_CHILD = 1, REGRID_PARENT = 2 };
 
 // Launchers (return hipError_t as int).
+// out[w]: whether patch w exceeds the refine, the coarsen threshold; host memory.
 int launch_tag_patches(const double* q, const int* slots, int n, const double* dxs,
                        const double* dys, long long pstride, int mx, int my, int mbc, int ivar,
                        double thr_refine, double thr_coarsen, int* out, hipStream_t st);
@@ -151,9 +152,10 @@ int launch_timeinterp(const double* q, const double* qlast, double* qti, const i
 int launch_copy_interior(const double* src, double* dst, const int* slots, int n,
                          long long pstride, int mx, int my, int mbc, int meqn,
                          hipStream_t st);
-// Per-slot compensated FP64 sums of q*dx*dy over interior cells: out[slot][m] = (hi, lo)
+// Compensated FP64 sums of q*dx*dy over the interior cells of the n patches:
+// out[m] = (hi, lo), host memory; parts: room for 2 meqn doubles per patch.
 int launch_mass(const double* q, const int* slots, int n, const double* dxs, const double* dys,
-                long long pstride, int mx, int my, int mbc, int meqn, double* out,
+                long long pstride, int mx, int my, int mbc, int meqn, double* parts, double* out,
                 hipStream_t st);
 
 // Largest tile the FP64 / FP32 kernels are instantiated for, per solver.
