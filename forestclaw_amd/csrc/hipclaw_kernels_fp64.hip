@@ -1023,67 +1023,107 @@ int launch_copy_patches(const double* src, double* dst, const int* slots, int n,
 // Ghost-patch message of each listed slot (the data a rank sends another for
 // a patch bordering it): the q band of mbc ghost and refratio*mbc interior
 // layers in the order of fclaw2d_clawpatch46_fort_local_ghost_pack
-// (src/patches/clawpatch/fort_4.6/fclaw2d_clawpatch46_local_ghost_pack.f:38-84;
-// band[] holds the slab offsets of one field in that order), then, with time
-// sync, the registers in the order of fclaw2d_clawpatch_time_sync_pack_registers
+// (src/patches/clawpatch/fort_4.6/fclaw2d_clawpatch46_local_ghost_pack.f:38-84),
+// then, with time sync, the registers in the order of fclaw2d_clawpatch_time_sync_pack_registers
 // (src/patches/clawpatch/fclaw2d_clawpatch_conservation.c:112-195): per face
 // meqn*len quadruples (fm, fp, edge flux 0, edge flux 1), then len pairs
 // (edge length, area).  unpack = 1 writes q and the registers back (edge
 // lengths and areas follow from dx, dy and are not read).
+//
+// A thread takes MESSAGE_ITEMS values, all loaded before they are stored, and
+// finds their places by arithmetic: looking them up in a table is one more memory
+// latency in a launch that lasts a few of them.
+constexpr int MESSAGE_ITEMS = 4;
+
+// slab offset of value e of the band, in the order of the reference's four loops
+struct Band {
+    int ng, mint, mx, my, nxp, n0, n1, n2;
+    SmallDiv narrow, bottom, top;
+    __device__ __forceinline__ Band(int mx, int my, int mbc)
+        : ng(mbc), mint(2 * mbc), mx(mx), my(my), nxp(mx + 2 * mbc), n0((my - mint + ng) * (mint + ng)),
+          n1(n0 + (mint + ng) * (mx + ng - mint)), n2(n1 + (my + ng - mint) * (mint + ng)), narrow(mint + ng),
+          bottom(mx + ng - mint), top(mx - mint + ng) {}
+    __device__ __forceinline__ int operator()(int e) const {
+        int i, j;
+        if (e < n0) {                    // left, up to the top strip
+            const int r = narrow(e);
+            j = 1 - ng + r;
+            i = 1 - ng + e - r * narrow.d;
+        } else if (e < n1) {             // bottom
+            e -= n0;
+            const int r = bottom(e);
+            j = 1 - ng + r;
+            i = mint + 1 + e - r * bottom.d;
+        } else if (e < n2) {             // right
+            e -= n1;
+            const int r = narrow(e);
+            j = mint + 1 + r;
+            i = mx - mint + 1 + e - r * narrow.d;
+        } else {                         // top
+            e -= n2;
+            const int r = top(e);
+            j = my - mint + 1 + r;
+            i = 1 - ng + e - r * top.d;
+        }
+        return (j + ng - 1) * nxp + i + ng - 1;
+    }
+};
+
 __global__ void __launch_bounds__(256)
 ghost_message(double* __restrict__ q, double* __restrict__ reg, const int* __restrict__ slots,
-              int n, const int* __restrict__ band, int nband, long long pstride, long long rstride,
+              int nband, long long pstride, long long rstride,
               int mx, int my, int mbc, int meqn, const double* __restrict__ dxs,
-              const double* __restrict__ dys, double* __restrict__ buf, long long elems,
-              int unpack) {
-    const int p = blockIdx.y;
-    if (p >= n) return;
-    const int slot = slots[p];
+              const double* __restrict__ dys, double* __restrict__ buf, int elems, int unpack) {
+    const int p = blockIdx.x, slot = slots[p];
     double* qp = q + (long long) slot * pstride;
-    double* b = buf + (long long) p * elems;
-    const long long plane = (long long) (mx + 2 * mbc) * (my + 2 * mbc);
-    const int nq = meqn * nband;
-    const int stride = gridDim.x * blockDim.x;
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nq; k += stride) {
-        const int m = k / nband, e = k - m * nband;
-        double* c = qp + m * plane + band[e];
-        if (unpack) *c = b[k];
-        else b[k] = *c;
-    }
-    if (!reg) return;
     double* rp = reg + (long long) slot * rstride;
-    double* rb = b + nq;
+    double* b = buf + (long long) p * elems;
+    const int plane = (mx + 2 * mbc) * (my + 2 * mbc), nq = meqn * nband;
     const double dx = dxs[slot], dy = dys[slot];
-    const int nreg = 2 * (4 * meqn + 2) * (mx + my);
-    for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < nreg; r += stride) {
-        int f = 0, t = r;
-        for (; f < 3; f++) {
-            const int len = f < 2 ? my : mx, blk = (4 * meqn + 2) * len;
-            if (t < blk) break;
-            t -= blk;
+    const Band band(mx, my, mbc);
+    const SmallDiv by_field(nband), by_my(my), by_mx(mx);
+    double v[MESSAGE_ITEMS];
+    double* c[MESSAGE_ITEMS];            // the value's place in the patch; a length or an area has none
+#pragma unroll
+    for (int u = 0; u < MESSAGE_ITEMS; u++) {
+        const int k = (blockIdx.y * MESSAGE_ITEMS + u) * 256 + threadIdx.x;
+        c[u] = nullptr;
+        v[u] = 0.0;
+        if (k >= elems) continue;
+        if (k < nq) {
+            const int m = by_field(k);
+            c[u] = qp + (long long) m * plane + band(k - m * nband);
+        } else {
+            const int per = 4 * meqn + 2, r = k - nq;
+            const bool xface = r < 2 * per * my;
+            const int len = xface ? my : mx, t2 = xface ? r : r - 2 * per * my, second = t2 >= per * len;
+            const int f = (xface ? 0 : 2) + second, t = t2 - second * per * len;
+            if (t < 4 * meqn * len) {
+                const int j = t >> 2, kind = t & 3;        // kinds FM, FP, EFIN, EFOUT in order
+                const int m = xface ? by_my(j) : by_mx(j), pos = j - m * len;
+                c[u] = rp + ((f * 4 + kind) * meqn + m) * mx + pos;
+            } else {
+                v[u] = ((t - 4 * meqn * len) & 1) ? dx * dy : xface ? dy : dx;
+            }
         }
-        const int len = f < 2 ? my : mx;
-        if (t < 4 * meqn * len) {
-            const int j = t >> 2, kind = t & 3;        // kinds FM, FP, EFIN, EFOUT in order
-            const int m = j / len, pos = j - m * len;
-            double* c = rp + ((f * 4 + kind) * meqn + m) * mx + pos;
-            if (unpack) *c = rb[r];
-            else rb[r] = *c;
-        } else if (!unpack) {
-            const int w = (t - 4 * meqn * len) & 1;
-            rb[r] = w == 0 ? (f < 2 ? dy : dx) : dx * dy;
-        }
+        if (unpack) v[u] = b[k];
+        else if (c[u]) v[u] = *c[u];
+    }
+#pragma unroll
+    for (int u = 0; u < MESSAGE_ITEMS; u++) {
+        const int k = (blockIdx.y * MESSAGE_ITEMS + u) * 256 + threadIdx.x;
+        if (k >= elems) continue;
+        if (!unpack) b[k] = v[u];
+        else if (c[u]) *c[u] = v[u];
     }
 }
 
-int launch_ghost_message(double* q, double* reg, const int* slots, int n, const int* band,
-                         int nband, long long pstride, long long rstride, int mx, int my, int mbc,
-                         int meqn, const double* dxs, const double* dys, double* buf,
-                         long long elems, int unpack, hipStream_t st) {
+int launch_ghost_message(double* q, double* reg, const int* slots, int n, int nband, long long pstride,
+                         long long rstride, int mx, int my, int mbc, int meqn, const double* dxs, const double* dys,
+                         double* buf, int elems, int unpack, hipStream_t st) {
     if (n <= 0) return 0;
-    const long long per = elems;
-    dim3 grid((unsigned) std::min<long long>((per + 255) / 256, 64), n);
-    hipLaunchKernelGGL(ghost_message, grid, dim3(256), 0, st, q, reg, slots, n, band, nband,
+    const int chunk = 256 * MESSAGE_ITEMS;
+    hipLaunchKernelGGL(ghost_message, dim3(n, (elems + chunk - 1) / chunk), dim3(256), 0, st, q, reg, slots, nband,
                        pstride, rstride, mx, my, mbc, meqn, dxs, dys, buf, elems, unpack);
     return (int) hipGetLastError();
 }
