@@ -1310,7 +1310,27 @@ int hipclaw_set_sync_program(hipclaw_state_t* s, const int* ops, int nops) {
     return hipclaw_set_sync_program_k(s, 0, ops, nops, nullptr, 0);
 }
 
-static int time_sync_async(hipclaw_state_t* s, int k) {
+// The registers that program k's synchronisation zeroes once every correction of
+// it has read them.
+static hipclaw::Resets resets_of(const hipclaw_state_t* s, int k) {
+    hipclaw::Resets z;
+    if (!s->reg) return z;
+    z.reg = s->reg;
+    z.list = s->sp[k].resets;
+    z.n = s->sp[k].nresets;
+    z.rstride = s->rstride;
+    z.per_face = 4 * s->cfg.meqn * s->cfg.mx;
+    return z;
+}
+
+static int reset_registers(hipclaw_state_t* s, const hipclaw::Resets& z) {
+    if (int e = hipclaw::launch_copy_patches(nullptr, nullptr, nullptr, 0, s->pstride, z, s->st))
+        return hipfail((hipError_t) e, "register reset launch");
+    return HIPCLAW_OK;
+}
+
+// resets = false leaves the registers to a later launch (resets_of).
+static int time_sync_async(hipclaw_state_t* s, int k, bool resets = true) {
     const SyncProgram& y = s->sp[k];
     if (!s->reg || (y.ngroups == 0 && y.nresets == 0)) return HIPCLAW_OK;
     hipclaw::SyncArgs a;
@@ -1318,8 +1338,6 @@ static int time_sync_async(hipclaw_state_t* s, int k) {
     a.start = y.start;
     a.ngroups = y.ngroups;
     a.maxgroup = y.maxgroup;
-    a.resets = y.resets;
-    a.nresets = y.nresets;
     a.q = s->q[s->cur];
     a.reg = s->reg;
     a.dxs = s->dxs;
@@ -1329,7 +1347,7 @@ static int time_sync_async(hipclaw_state_t* s, int k) {
     a.mx = s->cfg.mx; a.mbc = s->cfg.mbc; a.meqn = s->cfg.meqn;
     a.fluxreg = s->cfg.precision == HIPCLAW_FP32_BULK && s->conservative;
     if (int e = hipclaw::launch_time_sync(a, s->st)) return hipfail((hipError_t) e, "time_sync launch");
-    return HIPCLAW_OK;
+    return resets ? reset_registers(s, resets_of(s, k)) : HIPCLAW_OK;
 }
 
 int hipclaw_time_sync_k(hipclaw_state_t* s, int k) {
@@ -1785,7 +1803,7 @@ int hipclaw_step_batch(hipclaw_state_t* s, const int* slots, int nslots, double 
     if (int rc = clear_cfl(s)) return rc;
     if (s->qlast) {  // fclaw2d_clawpatch_save_current_step before every update
         int e = hipclaw::launch_copy_patches(s->q[s->cur], s->qlast, s->batch_slots, nslots,
-                                             s->pstride, s->st);
+                                             s->pstride, hipclaw::Resets{}, s->st);
         if (e) return hipfail((hipError_t) e, "copy_patches launch");
     }
     double* src = s->q[s->cur];
@@ -1944,13 +1962,15 @@ static int advance_launches(hipclaw_state_t* s, double dt, int nsteps, StepTimer
 // copied whole into qlast, then the step reading that copy and writing the
 // new interiors straight into the current slab, which the other levels keep
 // reading (the same values as stepping the slab itself: qlast holds its
-// every cell).
-static int subcycle_update(hipclaw_state_t* s, int level, double dt) {
+// every cell).  `due`: the registers of the last synchronisation, still to be
+// zeroed before this update adds to them.
+static int subcycle_update(hipclaw_state_t* s, int level, double dt, hipclaw::Resets& due) {
     const int l = level - s->lmin, n = s->loff[l + 1] - s->loff[l];
-    if (n == 0) return HIPCLAW_OK;
     const int* slots = s->lslots + s->loff[l];
-    int e = hipclaw::launch_copy_patches(s->q[s->cur], s->qlast, slots, n, s->pstride, s->st);
+    int e = hipclaw::launch_copy_patches(s->q[s->cur], s->qlast, slots, n, s->pstride, due, s->st);
     if (e) return hipfail((hipError_t) e, "copy_patches launch");
+    due.n = 0;
+    if (n == 0) return HIPCLAW_OK;
     return launch_step(s, step_args(s, s->qlast, s->q[s->cur], slots, n, dt));
 }
 
@@ -1975,14 +1995,14 @@ struct LevelCounter {
 // advance_level (src/fclaw2d_advance.c:112-150, 152-170): the level's step,
 // then, when the coarser level is due, its step and its time-interpolated
 // copies at the finer level's new time.
-static int subcycle_level(hipclaw_state_t* s, int level, int curr_fine_step, LevelCounter* tc) {
+static int subcycle_level(hipclaw_state_t* s, int level, int curr_fine_step, LevelCounter* tc, hipclaw::Resets& due) {
     LevelCounter& c = tc[level - s->lmin];
-    if (int rc = subcycle_update(s, level, c.dt_step)) return rc;
+    if (int rc = subcycle_update(s, level, c.dt_step, due)) return rc;
     c.last_step += c.step_inc;
     if (level > s->lmin) {
         LevelCounter& cc = tc[level - 1 - s->lmin];
         if (cc.last_step == curr_fine_step) {
-            if (int rc = subcycle_level(s, level - 1, cc.last_step, tc)) return rc;
+            if (int rc = subcycle_level(s, level - 1, cc.last_step, tc, due)) return rc;
             const double alpha = ((double) (c.last_step % cc.step_inc)) / cc.step_inc;
             if (int rc = subcycle_timeinterp(s, level - 1, alpha)) return rc;
         }
@@ -1992,6 +2012,7 @@ static int subcycle_level(hipclaw_state_t* s, int level, int curr_fine_step, Lev
 
 static int subcycle_launches(hipclaw_state_t* s, double dt, int ncoarse) {
     const int lmin = s->lmin, lmax = s->lmax, nl = lmax - lmin + 1;
+    hipclaw::Resets due;
     for (int c = 0; c < ncoarse; c++) {
         LevelCounter tc[HIPCLAW_MAX_PROGRAMS];
         for (int l = 0; l < nl; l++) {   // initialize_timestep_counters (:54-110)
@@ -2001,22 +2022,26 @@ static int subcycle_launches(hipclaw_state_t* s, double dt, int ncoarse) {
         }
         const int total = tc[nl - 1].total_steps;
         for (int nf = 0; nf < total; nf++) {
-            if (int rc = subcycle_level(s, lmax, nf, tc)) return rc;
+            if (int rc = subcycle_level(s, lmax, nf, tc, due)) return rc;
             const int last_step = tc[nl - 1].last_step;
             if (last_step < total) {
                 int ti = lmax - 1;
                 while (last_step % tc[ti - lmin].step_inc == 0) ti--;
                 const int k = 1 + ti - lmin;   // levels ti + 1 .. lmax, ti time-interpolated
                 if (int rc = ghost_fill_async(s, k)) return rc;
-                if (s->reg)
-                    if (int rc = time_sync_async(s, k)) return rc;
+                if (s->reg) {
+                    if (int rc = time_sync_async(s, k, false)) return rc;
+                    due = resets_of(s, k);
+                }
             }
         }
         if (int rc = ghost_fill_async(s, 0)) return rc;
-        if (s->reg)
-            if (int rc = time_sync_async(s, 0)) return rc;
+        if (s->reg) {
+            if (int rc = time_sync_async(s, 0, false)) return rc;
+            due = resets_of(s, 0);
+        }
     }
-    return HIPCLAW_OK;
+    return reset_registers(s, due);
 }
 
 // What the subcycled advance needs: subcycle state, levels, and the programs
@@ -2149,7 +2174,8 @@ int hipclaw_capture_graph(hipclaw_state_t* s, double dt, int nsteps) {
     HIP_TRY(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
     int rc = advance_launches(s, dt, nsteps, StepTimer::none);
     if (!rc && s->cur != cur0) {   // an odd number of steps: the result back into the slab the next replay starts from
-        if (int c = hipclaw::launch_copy_patches(s->q[s->cur], s->q[cur0], s->all_slots, s->npatch, s->pstride, s->st))
+        if (int c = hipclaw::launch_copy_patches(s->q[s->cur], s->q[cur0], s->all_slots, s->npatch, s->pstride,
+                                                hipclaw::Resets{}, s->st))
             rc = hipfail((hipError_t) c, "copy_patches launch");
     }
     hipGraph_t g = nullptr;
@@ -2171,7 +2197,7 @@ int hipclaw_replay_graph(hipclaw_state_t* s) {
     if (int rc = guard_save(s)) return rc;
     if (s->cur != s->graph_cur) {   // (any number of steps where a tile covers a patch)
         if (int e = hipclaw::launch_copy_patches(s->q[s->cur], s->q[s->graph_cur], s->all_slots, s->npatch,
-                                                 s->pstride, s->st))
+                                                 s->pstride, hipclaw::Resets{}, s->st))
             return hipfail((hipError_t) e, "copy_patches launch");
         s->cur = s->graph_cur;
     }

@@ -61,8 +61,6 @@ struct SyncArgs {
     const double* dxs;
     const double* dys;
     long long pstride, rstride;
-    const int* resets;   // [nresets][2]: (slot, face) registers zeroed after the corrections
-    int nresets;
     int mx, mbc, meqn;   // mx == my
     int fluxreg;         // registers hold one shared edge flux (FP32 flux form)
 };
@@ -136,8 +134,15 @@ int launch_reset_cfl(unsigned long long* p, int blocks, unsigned long long* sum,
 constexpr int STEP_BLOCKS = 64, STEP_SUMS = 5;
 int launch_collect_steps(unsigned long long* cfl, int blocks, unsigned long long* sum, unsigned long long* out,
                          hipStream_t st);
-// Whole patch slabs src[slot] -> dst[slot].
-int launch_copy_patches(const double* src, double* dst, const int* slots, int n, long long pstride,
+// Whole patch slabs src[slot] -> dst[slot], and registers to zero.
+struct Resets {
+    double* reg = nullptr;
+    const int* list = nullptr;   // [n][2]: (slot, face)
+    int n = 0;
+    long long rstride = 0;
+    int per_face = 0;
+};
+int launch_copy_patches(const double* src, double* dst, const int* slots, int n, long long pstride, const Resets& z,
                         hipStream_t st);
 int launch_ghost_message(double* q, double* reg, const int* slots, int n, int nband, long long pstride,
                          long long rstride, int mx, int my, int mbc, int meqn, const double* dxs, const double* dys,
