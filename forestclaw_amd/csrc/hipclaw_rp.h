@@ -564,12 +564,21 @@ struct RPShallow {
     template <int IXY>
     __device__ __forceinline__ static void consflux(const double* q, const double* /*aux*/,
                                                     const PhysParams& pp, double* f) {
+        consflux_of<IXY>(q, q[IXY == 1 ? 1 : 2] / q[0], pp, f);
+    }
+    template <int IXY>
+    __device__ __forceinline__ static void consflux_of(const double* q, double un, const PhysParams& pp, double* f) {
         constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
         const double hun = q[mu], hut = q[mv], h = q[0];
-        const double un = hun / h;
         f[0] = hun;
         f[mu] = (hun * hun) / h + (0.5 * pp.grav) * (h * h);
         f[mv] = un * hut;
+    }
+    // the same from the cell's values in both directions (`cells`)
+    template <int IXY>
+    __device__ __forceinline__ static void consflux_cells(const double* q, const double cx[NCELL], const double cy[NCELL],
+                                                          const PhysParams& pp, double* f) {
+        consflux_of<IXY>(q, IXY == 1 ? cx[3] : cy[3], pp, f);
     }
 };
 
@@ -900,12 +909,25 @@ struct RPEuler {
     __device__ __forceinline__ static void consflux(const double* q, const double* /*aux*/,
                                                     const PhysParams& pp, double* f) {
         constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
-        const double rho = q[0], un = q[mu] / rho, ut = q[mv] / rho, en = q[3];
+        consflux_of<IXY>(q, q[mu] / q[0], q[mv] / q[0], pp, f);
+    }
+    template <int IXY>
+    __device__ __forceinline__ static void consflux_of(const double* q, double un, double ut, const PhysParams& pp,
+                                                       double* f) {
+        constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
+        const double rho = q[0], en = q[3];
         const double p = (pp.gamma - 1.0) * (en - 0.5 * rho * (un * un + ut * ut));
         f[0] = q[mu];
         f[mu] = q[mu] * un + p;
         f[mv] = q[mu] * ut;
         f[3] = un * (en + p);
+    }
+    // the same from the cell's values in both directions (`cells`)
+    template <int IXY>
+    __device__ __forceinline__ static void consflux_cells(const double* q, const double cx[NCELL], const double cy[NCELL],
+                                                          const PhysParams& pp, double* f) {
+        if constexpr (IXY == 1) consflux_of<IXY>(q, cx[4], cy[4], pp, f);
+        else consflux_of<IXY>(q, cy[4], cx[4], pp, f);
     }
 };
 

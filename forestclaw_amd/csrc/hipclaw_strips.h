@@ -280,6 +280,18 @@ step_strips(StepArgs a, StripShape sh) {
                 }
                 qp += nxp;
             }
+            if constexpr (NC > 0) {
+                R q[MEQN];
+#pragma unroll
+                for (int m = 0; m < MEQN; m++) q[m] = (R) qr[C][m];
+                if constexpr (RANGED) {
+                    inC = all_lanes(RP::in_range(q, a.pp));
+                    RP::cells(q, a.pp, inC, cx[P], cy[P]);
+                } else {
+                    RP::template cell<1>(q, a.pp, cx[P]);
+                    RP::template cell<2>(q, a.pp, cy[P]);
+                }
+            }
             if constexpr (REGS && !FLUXFORM) {
                 // FP64 form: conservative flux of the pre-step state at the first
                 // interior and first ghost cell of every patch edge
@@ -289,14 +301,16 @@ step_strips(StepArgs a, StripShape sh) {
                 for (int m = 0; m < MAD; m++) ac[m] = MAUX > 0 ? (double) ar[C][m] : 0.0;
                 const int b = n - 2;          // interior row of the strip
                 if (byface && b >= own_y && b >= 0 && b < H) {
-                    RP::template consflux<1>(qr[C], ac, a.pp, fl);
+                    if constexpr (RANGED) RP::template consflux_cells<1>(qr[C], cx[P], cy[P], a.pp, fl);
+                    else RP::template consflux<1>(qr[C], ac, a.pp, fl);
                     double* r = rx + b + (i == 0 || i == mx + 1 ? REG_EFOUT : REG_EFIN) * MEQN * mx;
 #pragma unroll
                     for (int m = 0; m < MEQN; m++) reg_put<ACC>(r + m * mx, dtdy_el * fl[m]);
                 }
                 const bool below = bottom && (b == -1 || b == 0), above = top && (b == H - 1 || b == H);
                 if ((below || above) && incol) {
-                    RP::template consflux<2>(qr[C], ac, a.pp, fl);
+                    if constexpr (RANGED) RP::template consflux_cells<2>(qr[C], cx[P], cy[P], a.pp, fl);
+                    else RP::template consflux<2>(qr[C], ac, a.pp, fl);
                     double el;
                     // (a strip of one row has both faces, one after the other)
                     if (below) {
@@ -309,18 +323,6 @@ step_strips(StepArgs a, StripShape sh) {
 #pragma unroll
                         for (int m = 0; m < MEQN; m++) reg_put<ACC>(r + m * mx, el * fl[m]);
                     }
-                }
-            }
-            if constexpr (NC > 0) {
-                R q[MEQN];
-#pragma unroll
-                for (int m = 0; m < MEQN; m++) q[m] = (R) qr[C][m];
-                if constexpr (RANGED) {
-                    inC = all_lanes(RP::in_range(q, a.pp));
-                    RP::cells(q, a.pp, inC, cx[P], cy[P]);
-                } else {
-                    RP::template cell<1>(q, a.pp, cx[P]);
-                    RP::template cell<2>(q, a.pp, cy[P]);
                 }
             }
 
