@@ -168,11 +168,12 @@ struct hipclaw_state {
     // which the next update adds (deferred through qcorr)
     bool fused_ok = false;
     // ops: corners of every step (averages, interpolations) [0, fc0), the
-    // other ops of every step [fc0, fc0 + fbig), same-size face copies
+    // other ops of every step [fc0, fc0 + fbig) (the last fphys of them physical
+    // BCs), same-size face copies
     // [.., + fcopy), corner copies [.., + fc1) (copies only in an advance's
     // last step)
     GhostOp* fops = nullptr;
-    int fops_cap = 0, fc0 = 0, fbig = 0, fcopy = 0, fc1 = 0;
+    int fops_cap = 0, fc0 = 0, fbig = 0, fphys = 0, fcopy = 0, fc1 = 0;
     int* pull = nullptr;          // [slot][8] offsets of same-size ghost strips (StepArgs::pull)
     int pull_cap = 0;
     bool pull_ok = false;
@@ -1171,7 +1172,7 @@ static int fused_finish(hipclaw_state_t* s, const int* ops, int nops, FusedBuild
     int* pull = reinterpret_cast<int*>(b.stage + b.off_pull);
     const bool pull_ok = (double) s->pstride * s->max_patches < 2.0e9;
     if (pull_ok) std::fill(pull, pull + 8 * (size_t) np, 0);
-    int nc = 0, nl = b.ncorner, nf = b.nlite, nfc = b.nlite + b.ncopy;
+    int nc = 0, nl = b.ncorner, nphys = b.nlite, nf = b.nlite, nfc = b.nlite + b.ncopy;
     for (int o = 0; o < nops; o++) {
         const int* op = ops + 8 * o;
         const int type = op[0];
@@ -1204,9 +1205,9 @@ static int fused_finish(hipclaw_state_t* s, const int* ops, int nops, FusedBuild
             if (b.bcop[op[1]] != o) continue;   // once per patch
         }
         const bool corner = type == hipclaw::GHOST_AVERAGE_CORNER || type == hipclaw::GHOST_INTERP_CORNER;
-        fops[corner ? nc++ : nl++] = to_op(op);
+        fops[corner ? nc++ : type == hipclaw::GHOST_PHYSBC ? --nphys : nl++] = to_op(op);
     }
-    if (nc != b.ncorner || nl != b.nlite || nf != b.nlite + b.ncopy || nfc != nf + b.ncopyc)
+    if (nc != b.ncorner || nl != nphys || nf != b.nlite + b.ncopy || nfc != nf + b.ncopyc)
         return fail(HIPCLAW_EINVAL, "internal: fused ghost op count mismatch%s");
     if (int rc = stage_copy(s, s->fops, s->fops_cap, fops, nfc, "fused ghost ops")) return rc;
     if (pull_ok)
@@ -1215,6 +1216,7 @@ static int fused_finish(hipclaw_state_t* s, const int* ops, int nops, FusedBuild
     // buffer waits for them; launches on the stream come after them)
     s->fc0 = b.ncorner;
     s->fbig = b.nlite - b.ncorner;
+    s->fphys = b.nlite - nphys;
     s->fcopy = b.ncopy;
     s->fc1 = b.ncopyc;
     s->pull_ok = pull_ok;
@@ -1373,6 +1375,8 @@ static int ghost_flat_async(hipclaw_state_t* s, bool full, bool sync) {
     f.g.mx = s->cfg.mx; f.g.my = s->cfg.my; f.g.mbc = s->cfg.mbc; f.g.meqn = s->cfg.meqn;
     f.ncorner0 = s->fc0;
     f.nbig = full ? s->fbig + s->fcopy : s->fbig;
+    f.nphys = s->fphys;
+    f.phys0 = s->fbig - s->fphys;
     f.ncorner1 = full ? s->fc1 : 0;
     f.frel = s->frel;
     f.sops = !sync ? nullptr : s->fpaired ? s->fsops : s->sp[0].ops;

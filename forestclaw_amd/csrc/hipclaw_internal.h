@@ -80,12 +80,13 @@ struct FaceRel {
 };
 
 // One launch of the fused ghost fill and time-sync increments: ghost ops
-// [ncorner0, ncorner0 + nbig) of g.ops `parts` waves each (set by the launch), the
-// corner ops [0, ncorner0) and [ncorner0 + nbig, ... + ncorner1) four to a wave,
+// [ncorner0, ncorner0 + nbig) of g.ops one wave or several each, the corner ops [0, ncorner0) and [ncorner0 + nbig, ... + ncorner1) four to a wave,
 // then sync ops [0, nsync) of sops several to a wave.
 struct FlatArgs {
     GhostArgs g;
-    int ncorner0, nbig, ncorner1, parts;
+    int ncorner0, nbig, ncorner1;
+    int phys0, nphys;          // the physical BCs among the nbig
+    int parts, phys_parts;     // set by the launch
     const FaceRel* frel;       // [slot][4]
     const int* sops;           // [nsync][8] as SyncArgs::ops
     int nsync;

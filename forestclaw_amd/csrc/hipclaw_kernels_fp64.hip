@@ -290,8 +290,8 @@ __global__ void __launch_bounds__(PHYSBC_THREADS) ghost_groups(GhostArgs g, cons
 // ---------------------------------------------------------------- fused ghost fill + sync
 // The fused launch lasts as long as its longest chain of dependent loads, so
 // what an op reads is resolved in stages (the faces' relations, then all the
-// values), and an op's elements are spread over `parts` waves instead of being
-// taken in turn (flat_parts): shock-bubble FP64 on 2,740 patches of 16 x 16 16.4
+// values), and an op's elements are spread over several waves instead of being
+// taken in turn (flat_waves): shock-bubble FP64 on 2,740 patches of 16 x 16 16.4
 // -> 11.9 us per launch, dam break FP64 on 3,400 of 32 x 32 17.4 -> 13.8.
 
 // A face's relation; k: the face whose ghost strip holds (i, j), -1 for an
@@ -578,12 +578,12 @@ constexpr int FLAT_OPW = 4;           // waves per workgroup
 constexpr int FLAT_CORNER_LANES = 16; // lanes of one corner op
 constexpr int FLAT_CORNERS = 64 / FLAT_CORNER_LANES;
 
-// Waves of one face or physical-BC op: one for every 64 ghost cells of a face and
-// field, so that no lane takes two.
-static int flat_parts(const GhostArgs& g) {
-    const int n = g.meqn * g.mbc * (std::max(g.mx, g.my) + 2 * g.mbc);
-    return std::min(4, (n + 63) / 64);
-}
+// Waves of one op, so that no lane takes two elements in turn whose chains are
+// long: a physical BC's are the ghost cells of a face, an interpolation's its
+// coarse cells (copies and averages load several elements at once anyway, and
+// waves without work are not free: ensemble of 64 runs, 22,436 patches of 16 x 16,
+// 58 us with two waves for every op, 56 with one).
+static int flat_waves(int n) { return std::min(4, (n + 63) / 64); }
 __host__ __device__ __forceinline__ int flat_corner_waves(int n) { return (n + FLAT_CORNERS - 1) / FLAT_CORNERS; }
 // Time-sync ops of one wave, per positions each: as many as its lanes take at once.
 __host__ __device__ __forceinline__ int flat_sync_ops(int per) {
@@ -593,15 +593,20 @@ __host__ __device__ __forceinline__ int flat_sync_ops(int per) {
 __global__ void __launch_bounds__(64 * FLAT_OPW) ghost_flat(FlatArgs f) {
     int w = blockIdx.x * FLAT_OPW + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    if (w < f.nbig * f.parts) {
-        const int o = w / f.parts, t = (w - o * f.parts) * 64 + lane, W = 64 * f.parts;
-        const GhostOp op = f.g.ops[f.ncorner0 + o];
+    if (w < f.nphys * f.phys_parts) {
+        const int o = w / f.phys_parts, t = (w - o * f.phys_parts) * 64 + lane;
+        fused_physbc_op(f.g, f.frel, f.g.ops[f.ncorner0 + f.phys0 + o], t, 64 * f.phys_parts);
+        return;
+    }
+    w -= f.nphys * f.phys_parts;
+    if (w < (f.nbig - f.nphys) * f.parts) {
+        const int k = w / f.parts, t = (w - k * f.parts) * 64 + lane, W = 64 * f.parts;
+        const GhostOp op = f.g.ops[f.ncorner0 + k + (k < f.phys0 ? 0 : f.nphys)];
         if (op.type == GHOST_INTERP_FACE || op.type == GHOST_INTERP_CORNER) fused_interp_op(f.g, f.frel, op, t, W);
-        else if (op.type == GHOST_PHYSBC) fused_physbc_op(f.g, f.frel, op, t, W);
         else ghost_exchange_op(f.g, op, t, W);
         return;
     }
-    w -= f.nbig * f.parts;
+    w -= (f.nbig - f.nphys) * f.parts;
     const int nw0 = flat_corner_waves(f.ncorner0), nw1 = flat_corner_waves(f.ncorner1);
     if (w < nw0 + nw1) {
         // corner ops [0, ncorner0) and [ncorner0 + nbig, ... + ncorner1)
@@ -656,9 +661,11 @@ __global__ void apply_qcorr(double* __restrict__ q, const double* __restrict__ q
 
 int launch_ghost_flat(const FlatArgs& args, hipStream_t st) {
     FlatArgs f = args;
-    f.parts = flat_parts(f.g);
+    const int side = std::max(f.g.mx, f.g.my);
+    f.parts = flat_waves(f.g.meqn * (f.g.mbc / 2) * side);
+    f.phys_parts = flat_waves(f.g.meqn * f.g.mbc * (side + 2 * f.g.mbc));
     const int ops = flat_sync_ops(f.g.meqn * f.g.mx);
-    const int n = f.nbig * f.parts + flat_corner_waves(f.ncorner0) + flat_corner_waves(f.ncorner1) + (f.nsync + ops - 1) / ops;
+    const int n = f.nphys * f.phys_parts + (f.nbig - f.nphys) * f.parts + flat_corner_waves(f.ncorner0) + flat_corner_waves(f.ncorner1) + (f.nsync + ops - 1) / ops;
     if (n <= 0) return 0;
     hipLaunchKernelGGL(ghost_flat, dim3((n + FLAT_OPW - 1) / FLAT_OPW), dim3(64 * FLAT_OPW), 0, st, f);
     return (int) hipGetLastError();
