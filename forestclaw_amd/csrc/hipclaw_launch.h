@@ -132,10 +132,12 @@ inline int device_simds() {
     return n;
 }
 
-// pairs: two waves of the kernel fit a SIMD.  nw: waves per workgroup.  The
-// waves share nothing; one per workgroup lets the dispatcher place each by itself.
+// pairs: two waves of the kernel fit a SIMD.  lds: its bytes per wave (one wave per
+// workgroup then).  nw: waves per workgroup.  The waves share nothing; one per
+// workgroup lets the dispatcher place each by itself.
 template <typename K>
-inline int launch_strips(K kernel, bool pairs, int nw, const StepArgs& a, const StepLaunch& L) {
+inline int launch_strips(K kernel, bool pairs, int lds, int nw, const StepArgs& a, const StepLaunch& L) {
+    if (lds > 0) nw = 1;
     if (a.nwork <= 0) return 0;
     const bool inplace = a.qsrc == a.qdst;
     const int simds = device_simds();
@@ -146,9 +148,9 @@ inline int launch_strips(K kernel, bool pairs, int nw, const StepArgs& a, const 
     const long long blocks = ((waves + nw - 1) / nw + 7) / 8 * 8;   // a multiple of the 8 XCDs
     if (waves * 64 > 0x7fffffffLL) return (int) hipErrorInvalidConfiguration;
     if (L.start || L.stop)
-        hipExtLaunchKernelGGL(kernel, dim3((unsigned) blocks), dim3(64 * nw), 0, L.st, L.start, L.stop, 0, a, sh);
+        hipExtLaunchKernelGGL(kernel, dim3((unsigned) blocks), dim3(64 * nw), lds, L.st, L.start, L.stop, 0, a, sh);
     else
-        hipLaunchKernelGGL(kernel, dim3((unsigned) blocks), dim3(64 * nw), 0, L.st, a, sh);
+        hipLaunchKernelGGL(kernel, dim3((unsigned) blocks), dim3(64 * nw), lds, L.st, a, sh);
     return (int) hipGetLastError();
 }
 
@@ -158,19 +160,20 @@ inline int launch_strips(K kernel, bool pairs, int nw, const StepArgs& a, const 
 template <class RP, typename R, bool WITH_REGS>
 inline int launch_step_strips(int nw, const StepArgs& a, const StepLaunch& st) {
     constexpr bool FF = sizeof(R) == 4 && RP::CONSERVATIVE, pairs = strip_waves_per_eu<RP, R>() > 1;
+    constexpr int lds = strip_lds<RP, R>();
     const bool std = all_mc_limiter<RP>(a) && a.order2 && a.transverse == 2;
     if (a.reg) {
         if constexpr (WITH_REGS) {
             if (a.reg_accumulate)
-                return std ? launch_strips(step_strips<RP, R, FF, 2, true>, pairs, nw, a, st)
-                           : launch_strips(step_strips<RP, R, FF, 2, false>, pairs, nw, a, st);
-            return std ? launch_strips(step_strips<RP, R, FF, 1, true>, pairs, nw, a, st)
-                       : launch_strips(step_strips<RP, R, FF, 1, false>, pairs, nw, a, st);
+                return std ? launch_strips(step_strips<RP, R, FF, 2, true>, pairs, lds, nw, a, st)
+                           : launch_strips(step_strips<RP, R, FF, 2, false>, pairs, lds, nw, a, st);
+            return std ? launch_strips(step_strips<RP, R, FF, 1, true>, pairs, lds, nw, a, st)
+                       : launch_strips(step_strips<RP, R, FF, 1, false>, pairs, lds, nw, a, st);
         }
         return (int) hipErrorInvalidValue;
     }
-    return std ? launch_strips(step_strips<RP, R, FF, 0, true>, pairs, nw, a, st)
-               : launch_strips(step_strips<RP, R, FF, 0, false>, pairs, nw, a, st);
+    return std ? launch_strips(step_strips<RP, R, FF, 0, true>, pairs, lds, nw, a, st)
+               : launch_strips(step_strips<RP, R, FF, 0, false>, pairs, lds, nw, a, st);
 }
 
 // Waves per workgroup by default.  Strips: one.  16 x 16 tiles: four for FP64,

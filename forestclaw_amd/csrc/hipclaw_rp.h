@@ -181,8 +181,9 @@ __device__ __forceinline__ bool exponent_within(double x, int lo, int hi) {
 // 100 shock-bubble steps 12.5 -> 11.7 ms, batched 24 x 20 shallow water 134 -> 125
 // us): RP::in_range(q,
 // pp) says whether a cell's values allow the fast forms above, RP::cells gives
-// `cell` in both directions, rpn2c takes whether both cells are in range, and
-// rpt2_pair splits both fluctuations of an interface.
+// `cell` in both directions, rpn2c takes whether both cells are in range, rpt2_pair
+// splits both fluctuations of an interface, and right_going gives apdq once more
+// from the waves, their speeds and amdq, so that it need not be kept beside them.
 template <class RP, class = void>
 struct ranged : std::false_type {};
 template <class RP>
@@ -453,12 +454,20 @@ struct RPShallow {
                 }
             }
         }
+        right_going<IXY>(wave, s, amdq, apdq);
+    }
+
+    // apdq: what amdq leaves of the waves' sum (FP64)
+    template <int IXY>
+    __device__ __forceinline__ static void right_going(const R wave[MWAVES][MEQN], const R s[MWAVES], const R amdq[MEQN],
+                                                       R apdq[MEQN]) {
+#pragma clang fp contract(off)
 #pragma unroll
-        for (int m = 0; m < 3; m++) {
+        for (int m = 0; m < MEQN; m++) {
             R df = R(0);
             bool first = true;
 #pragma unroll
-            for (int mw = 0; mw < 3; mw++)
+            for (int mw = 0; mw < MWAVES; mw++)
                 if (!wave_zero<IXY>(mw, m)) sum_term(df, s[mw], wave[mw][m], first);
             apdq[m] = df - amdq[m];
         }
@@ -590,9 +599,9 @@ struct RPEuler {
     static constexpr bool RPT2_LINEAR = true;   // bm, bp linear in asdq
     static constexpr bool EXPLICIT_FMA = true;  // no contraction left to the compiler (mad)
     static constexpr bool RANGED = sizeof(R) == 8;
-    // u, v, a, enth, u2v2, g1a2, euv (and in FP32 1 / (2 a), which rpt2 then
-    // takes from the normal solve)
-    static constexpr int NROE = sizeof(R) == 4 ? 8 : 7;
+    // u, v, a, enth, g1a2, and in FP32 u2v2, euv and 1 / (2 a) of the normal solve
+    // (FP64 has no registers for the first two of them, which rpt2 computes again)
+    static constexpr int NROE = sizeof(R) == 4 ? 8 : 5;
 
     __device__ __forceinline__ static void speeds(const R roe[NROE], R s[MWAVES]) {
         s[0] = roe[0] - roe[2]; s[1] = s[2] = roe[0]; s[3] = roe[0] + roe[2];
@@ -739,7 +748,8 @@ struct RPEuler {
             g1a2 = dv(gamma1, a2s);
         }
         const R euv = enth - u2v2;
-        roe[0] = u; roe[1] = v; roe[2] = a; roe[3] = enth; roe[4] = u2v2; roe[5] = g1a2; roe[6] = euv;
+        roe[0] = u; roe[1] = v; roe[2] = a; roe[3] = enth; roe[4] = g1a2;
+        if constexpr (sizeof(R) == 4) { roe[5] = u2v2; roe[6] = euv; }
 
         const R d0 = qR[0] - qL[0], d1 = qR[mu] - qL[mu], d2 = qR[mv] - qL[mv], d3 = qR[3] - qL[3];
         const R a3 = g1a2 * (mad(v, d2, mad(u, d1, euv * d0)) - d3);
@@ -806,12 +816,20 @@ struct RPEuler {
                 }
             }
         }
+        right_going<IXY>(wave, s, amdq, apdq);
+    }
+
+    // apdq: what amdq leaves of the waves' sum (FP64)
+    template <int IXY>
+    __device__ __forceinline__ static void right_going(const R wave[MWAVES][MEQN], const R s[MWAVES], const R amdq[MEQN],
+                                                       R apdq[MEQN]) {
+#pragma clang fp contract(off)
 #pragma unroll
-        for (int m = 0; m < 4; m++) {
+        for (int m = 0; m < MEQN; m++) {
             R df = R(0);
             bool first = true;
 #pragma unroll
-            for (int mw = 0; mw < 4; mw++)
+            for (int mw = 0; mw < MWAVES; mw++)
                 if (!wave_zero<IXY>(mw, m)) sum_term(df, s[mw], wave[mw][m], first);
             apdq[m] = df - amdq[m];
         }
@@ -824,8 +842,9 @@ struct RPEuler {
                                                 R bp[MEQN]) {
 #pragma clang fp contract(off)
         constexpr int mu = IXY == 1 ? 1 : 2, mv = IXY == 1 ? 2 : 1;
-        const R u = roe[0], v = roe[1], a = roe[2], enth = roe[3], u2v2 = roe[4];
-        const R g1a2 = roe[5], euv = roe[6];
+        const R u = roe[0], v = roe[1], a = roe[2], enth = roe[3], g1a2 = roe[4];
+        const R u2v2 = sizeof(R) == 4 ? roe[NROE - 3] : mad(v, v, u * u);
+        const R euv = sizeof(R) == 4 ? roe[NROE - 2] : enth - u2v2;
         const R a3 = g1a2 * (mad(v, asdq[mv], mad(u, asdq[mu], euv * asdq[0])) - asdq[3]);
         const R a2 = mad(-u, asdq[0], asdq[mu]);
         const R t4 = mad(-a, a3, mad(a - v, asdq[0], asdq[mv]));

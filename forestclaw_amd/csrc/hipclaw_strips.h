@@ -109,14 +109,28 @@ __device__ __forceinline__ int opaque(int x) {
     return x;
 }
 
-// Waves per SIMD the register allocation aims for.  The FP64 Euler form keeps
-// more than the 256 registers of two waves and gets all 512; the others run
-// with two waves and nothing in scratch (three waves of 168 registers spill,
-// and a reload waits for the stores in flight: shallow water FP32 on 11,296
-// patches of 32 x 32 0.412 ms with 3 waves and 6 spills against 0.331 with 2).
+// Where the registers of two waves do not hold what a step leaves to the next
+// (Euler FP64, 324 registers of 256), it stands in LDS, each lane its own column:
+// sets of MEQN values, of which the last three are kept for the two latest rows,
+// then MWAVES products.  Euler's 40 values are 20 KiB per wave, eight waves all of
+// a CU's 160.  (100 shock-bubble steps on 2,740 patches of 16 x 16 11.1 ms with one
+// wave per SIMD and the rest in accumulation registers, 9.8 ms with two.)
+template <class RP, typename R>
+constexpr bool strip_carry() { return sizeof(R) == 8 && RP::MEQN * RP::MWAVES > 9 && ranged<RP>::value; }
+enum { CARRY_TU = 0, CARRY_PD, CARRY_PU, CARRY_FXM, CARRY_FXP = CARRY_FXM + 2, CARRY_GPL = CARRY_FXP + 2,
+       CARRY_DL = CARRY_GPL + 2 };
+template <class RP, typename R>
+constexpr int strip_lds() { return strip_carry<RP, R>() ? (CARRY_DL * RP::MEQN + RP::MWAVES) * 64 * (int) sizeof(R) : 0; }
+
+// Waves per SIMD the register allocation aims for.  Two, and nothing in scratch
+// (three waves of 168 registers spill, and a reload waits for the stores in
+// flight: shallow water FP32 on 11,296 patches of 32 x 32 0.412 ms with 3 waves
+// and 6 spills against 0.331 with 2); advection has room for three; a registered
+// FP64 solver of more wave components than shallow water gets all 512 registers.
 template <class RP, typename R>
 constexpr int strip_waves_per_eu() {
-    return RP::MEQN * RP::MWAVES == 1 ? 3 : (sizeof(R) == 8 && RP::MEQN * RP::MWAVES > 9) ? 1 : 2;
+    return RP::MEQN * RP::MWAVES == 1 ? 3
+           : sizeof(R) == 8 && RP::MEQN * RP::MWAVES > 9 && !strip_carry<RP, R>() ? 1 : 2;
 }
 
 template <class RP, typename R, bool FLUXFORM, int KEEP, bool STD>
@@ -135,6 +149,8 @@ step_strips(StepArgs a, StripShape sh) {
     // FP32 with a linear rpt2: the factor dt / (2 dx) goes on asdq
     constexpr bool PRE = sizeof(R) == 4 && rpt2_linear<RP>::value;
     constexpr bool RANGED = ranged<RP>::value;
+    constexpr bool CARRY = strip_carry<RP, R>();
+    extern __shared__ double carry_mem[];
     using WZ1 = wave_zeros<RP, 1>;
     using WZ2 = wave_zeros<RP, 2>;
 
@@ -251,6 +267,7 @@ step_strips(StepArgs a, StripShape sh) {
     bool inA = false, inB = false, inC = false;   // every lane's cell of the row is in range (RP::RANGED)
     R smaxx = R(0), smaxy = R(0);         // largest |s| of every interface the lane solves
     const R halfx = R(0.5) * dtdx, halfy = R(0.5) * dtdy;
+    R* const carry = (R*) carry_mem + (threadIdx.x >> 6) * ((CARRY_DL * MEQN + MW) * 64) + lane;
 
 
     // Step n: row C is row n.  Every stage is entered as the rows it needs are
@@ -264,6 +281,8 @@ step_strips(StepArgs a, StripShape sh) {
             const int n = n0 + e;
             const int P = e, O = 1 - e, A = e, B = e + 1, C = e + 2, N = (e + 3) & 3;
             if (U > 1 && n > H + 3) break;
+            R* const kept = carry + (n & 1) * (MEQN * 64);          // this row's and
+            R* const last = carry + (1 - (n & 1)) * (MEQN * 64);    // the last row's sets of the two latest rows
             // ---- row n + 1 under way ----
             if (n < H + 3) {
                 const double* p = qp + (j < 1 ? dlo : j > my ? dhi : dmid);
@@ -372,6 +391,10 @@ step_strips(StepArgs a, StripShape sh) {
                 for (int m = 0; m < MEQN; m++) {
                     fxm[P][m] = mad(R(0.5), cq[m], zadd(amdq[m]));
                     if constexpr (!FLUXFORM) fxp[P][m] = mad(R(0.5), cq[m], -apdq[m]);
+                    if constexpr (CARRY) {
+                        kept[(CARRY_FXM * MEQN + m) * 64] = fxm[P][m];
+                        kept[(CARRY_FXP * MEQN + m) * 64] = fxp[P][m];
+                    }
                 }
                 if (STD || a.transverse) {
                     if (STD || (a.order2 && a.transverse == 2)) {
@@ -399,18 +422,25 @@ step_strips(StepArgs a, StripShape sh) {
                     for (int m = 0; m < MEQN; m++) {
                         const R gAd = PRE ? bmA[m] : halfx * bmA[m], gAu = PRE ? bpA[m] : halfx * bpA[m];
                         const R gBd = PRE ? bmP[m] : halfx * bmP[m], gBu = PRE ? bpP[m] : halfx * bpP[m];
-                        gt[m] = tu[O][m] + (-next_lane(gAd) - gBd);
+                        const R below = CARRY ? carry[(CARRY_TU * MEQN + m) * 64] : tu[O][m];
+                        gt[m] = below + (-next_lane(gAd) - gBd);
                         tu[P][m] = -next_lane(gAu) - gBu;
+                        if constexpr (CARRY) carry[(CARRY_TU * MEQN + m) * 64] = tu[P][m];
                     }
                 } else {
 #pragma unroll
-                    for (int m = 0; m < MEQN; m++) { gt[m] = R(0); tu[P][m] = R(0); }
+                    for (int m = 0; m < MEQN; m++) {
+                        gt[m] = R(0);
+                        tu[P][m] = R(0);
+                        if constexpr (CARRY) carry[(CARRY_TU * MEQN + m) * 64] = R(0);
+                    }
                 }
             } else {
                 unset(gt); unset(tu[P]); unset(fxm[P]); unset(fxp[P]);
             }
 
             // ---- the y-interface between rows B and C, as solved ----
+            R dlo[MW];                        // the products of the interface below
             if (n >= 1) {
                 R qL[MEQN], qR[MEQN];
 #pragma unroll
@@ -428,12 +458,18 @@ step_strips(StepArgs a, StripShape sh) {
 #pragma unroll
                     for (int m = 0; m < MEQN; m++)
                         if (!WZ2::at(mw, m)) sum_term(d, wv[O][mw][m], wv[P][mw][m], first);
+                    if constexpr (CARRY) {
+                        dlo[mw] = carry[(CARRY_DL * MEQN + mw) * 64];
+                        carry[(CARRY_DL * MEQN + mw) * 64] = d;
+                    } else {
+                        dlo[mw] = dl[O][mw];
+                    }
                     dl[P][mw] = d;
                 }
             } else {
 #pragma unroll
                 for (int mw = 0; mw < MW; mw++) unset(wv[P][mw]);
-                unset(sv[P]); unset(am[P]); unset(apq[P]); unset(ro[P]); unset(dl[P]);
+                unset(sv[P]); unset(am[P]); unset(apq[P]); unset(ro[P]); unset(dl[P]); unset(dlo);
             }
 
             double out[MEQN], Fx[MEQN];       // row A's new values; x-flux left of the cell
@@ -447,22 +483,30 @@ step_strips(StepArgs a, StripShape sh) {
 #pragma unroll
                     for (int mw = 0; mw < MW; mw++) so[mw] = sv[O][mw];
                 }
+                R ap[MEQN];
+                if constexpr (RANGED) {
+                    RP::template right_going<2>(wv[O], so, am[O], ap);
+                } else {
+#pragma unroll
+                    for (int m = 0; m < MEQN; m++) ap[m] = apq[O][m];
+                }
 #pragma unroll
                 for (int mw = 0; mw < MW; mw++) smaxy = fmax(smaxy, fabs(so[mw]));
                 R cq[MEQN];
 #pragma unroll
                 for (int m = 0; m < MEQN; m++) cq[m] = R(0);
-                if (STD || a.order2) limited_correction<RP, R, 2, STD>(a, wv[O], so, dl[O], dl[P], dtdy, cq);
+                if (STD || a.order2) limited_correction<RP, R, 2, STD>(a, wv[O], so, dlo, dl[P], dtdy, cq);
 #pragma unroll
                 for (int m = 0; m < MEQN; m++) {
                     gm[m] = gt[m] + mad(R(0.5), cq[m], zadd(am[O][m]));
-                    if constexpr (!FLUXFORM) gpl[P][m] = gt[m] + mad(R(0.5), cq[m], -apq[O][m]);
+                    if constexpr (!FLUXFORM) gpl[P][m] = gt[m] + mad(R(0.5), cq[m], -ap[m]);
+                    if constexpr (CARRY) kept[(CARRY_GPL * MEQN + m) * 64] = gpl[P][m];
                 }
                 R nAd[MEQN], nAu[MEQN];
                 if (STD || a.transverse) {
                     R amdq[MEQN], apdq[MEQN];
 #pragma unroll
-                    for (int m = 0; m < MEQN; m++) { amdq[m] = am[O][m]; apdq[m] = apq[O][m]; }
+                    for (int m = 0; m < MEQN; m++) { amdq[m] = am[O][m]; apdq[m] = ap[m]; }
                     if (STD || (a.order2 && a.transverse == 2)) {
 #pragma unroll
                         for (int m = 0; m < MEQN; m++) { amdq[m] = amdq[m] + cq[m]; apdq[m] = apdq[m] - cq[m]; }
@@ -500,11 +544,20 @@ step_strips(StepArgs a, StripShape sh) {
                 // ---- row A: x-fluxes with the transverse parts of its two y-interfaces, update ----
 #pragma unroll
                 for (int m = 0; m < MEQN; m++) {
-                    const R t1 = -nAd[m] - gPd[O][m];      // into the x-face left of the cell
-                    const R t2 = -nAu[m] - gPu[O][m];      // into the one right of it
+                    R pd = gPd[O][m], pu = gPu[O][m], xm = fxm[O][m], xp = fxp[O][m];
+                    if constexpr (CARRY) {
+                        pd = carry[(CARRY_PD * MEQN + m) * 64];
+                        pu = carry[(CARRY_PU * MEQN + m) * 64];
+                        xm = last[(CARRY_FXM * MEQN + m) * 64];
+                        xp = last[(CARRY_FXP * MEQN + m) * 64];
+                        carry[(CARRY_PD * MEQN + m) * 64] = gPd[P][m];
+                        carry[(CARRY_PU * MEQN + m) * 64] = gPu[P][m];
+                    }
+                    const R t1 = -nAd[m] - pd;             // into the x-face left of the cell
+                    const R t2 = -nAu[m] - pu;             // into the one right of it
                     const R t2l = prev_lane(t2);
-                    fm[m] = (fxm[O][m] + t2l) + t1;
-                    if constexpr (!FLUXFORM) fp[m] = (fxp[O][m] + t2l) + t1;
+                    fm[m] = (xm + t2l) + t1;
+                    if constexpr (!FLUXFORM) fp[m] = (xp + t2l) + t1;
                 }
                 if constexpr (FLUXFORM) {
                     // FP64 fluxes f and g of the row's cells, each evaluated once: the
@@ -525,7 +578,7 @@ step_strips(StepArgs a, StripShape sh) {
 #pragma unroll
                     for (int m = 0; m < MEQN; m++) {
                         const R Dx = next_lane(fm[m]) - fp[m];
-                        const R Dy = gm[m] - gpl[O][m];
+                        const R Dy = gm[m] - (CARRY ? last[(CARRY_GPL * MEQN + m) * 64] : gpl[O][m]);
                         if constexpr (sizeof(R) == sizeof(double)) out[m] = (qr[A][m] - dtdx * Dx) - dtdy * Dy;
                         else out[m] = fmad64(-dtdy64, (double) Dy, fmad64(-dtdx64, (double) Dx, qr[A][m]));
                     }
