@@ -109,27 +109,32 @@ __device__ __forceinline__ int opaque(int x) {
     return x;
 }
 
-// Where the registers of two waves do not hold what a step leaves to the next
-// (Euler FP64, 324 registers of 256), it stands in LDS, each lane its own column:
-// sets of MEQN values, of which the last three are kept for the two latest rows,
-// then MWAVES products.  Euler's 40 values are 20 KiB per wave, eight waves all of
-// a CU's 160.  (100 shock-bubble steps on 2,740 patches of 16 x 16 11.1 ms with one
-// wave per SIMD and the rest in accumulation registers, 9.8 ms with two.)
+// What a step leaves to the next stands in LDS, each lane its own column, where
+// that gains a wave per SIMD: sets of MEQN values, of which the last three are kept
+// for the two latest rows, then MWAVES products.
+//   * Euler FP64, 324 registers: two waves instead of one (100 shock-bubble steps on
+//     2,740 patches of 16 x 16 11.1 -> 9.8 ms).  Its 40 values are 20 KiB per wave,
+//     eight waves all of a CU's 160.
+//   * Shallow water FP32, 186 registers: three instead of two (200 dam break steps
+//     on 11,296 patches of 32 x 32 64.1 -> 63.0 ms, 100 ensemble steps 26.4 -> 26.1).
 template <class RP, typename R>
-constexpr bool strip_carry() { return sizeof(R) == 8 && RP::MEQN * RP::MWAVES > 9 && ranged<RP>::value; }
+constexpr bool strip_carry() {
+    return sizeof(R) == 8 ? RP::MEQN * RP::MWAVES > 9 && ranged<RP>::value
+                          : RP::MEQN * RP::MWAVES == 9 && explicit_fma<RP>::value;
+}
 enum { CARRY_TU = 0, CARRY_PD, CARRY_PU, CARRY_FXM, CARRY_FXP = CARRY_FXM + 2, CARRY_GPL = CARRY_FXP + 2,
        CARRY_DL = CARRY_GPL + 2 };
 template <class RP, typename R>
 constexpr int strip_lds() { return strip_carry<RP, R>() ? (CARRY_DL * RP::MEQN + RP::MWAVES) * 64 * (int) sizeof(R) : 0; }
 
-// Waves per SIMD the register allocation aims for.  Two, and nothing in scratch
-// (three waves of 168 registers spill, and a reload waits for the stores in
-// flight: shallow water FP32 on 11,296 patches of 32 x 32 0.412 ms with 3 waves
-// and 6 spills against 0.331 with 2); advection has room for three; a registered
-// FP64 solver of more wave components than shallow water gets all 512 registers.
+// Waves per SIMD the register allocation aims for, with nothing in scratch: a
+// reload waits for the stores in flight (shallow water FP32 with three waves and 6
+// spills, before the values above stood in LDS, 0.412 ms on 11,296 patches of
+// 32 x 32, with two waves and none 0.331).  A registered FP64 solver of more wave
+// components than shallow water gets all 512 registers.
 template <class RP, typename R>
 constexpr int strip_waves_per_eu() {
-    return RP::MEQN * RP::MWAVES == 1 ? 3
+    return RP::MEQN * RP::MWAVES == 1 || (sizeof(R) == 4 && strip_carry<RP, R>()) ? 3
            : sizeof(R) == 8 && RP::MEQN * RP::MWAVES > 9 && !strip_carry<RP, R>() ? 1 : 2;
 }
 
@@ -393,7 +398,7 @@ step_strips(StepArgs a, StripShape sh) {
                     if constexpr (!FLUXFORM) fxp[P][m] = mad(R(0.5), cq[m], -apdq[m]);
                     if constexpr (CARRY) {
                         kept[(CARRY_FXM * MEQN + m) * 64] = fxm[P][m];
-                        kept[(CARRY_FXP * MEQN + m) * 64] = fxp[P][m];
+                        if constexpr (!FLUXFORM) kept[(CARRY_FXP * MEQN + m) * 64] = fxp[P][m];
                     }
                 }
                 if (STD || a.transverse) {
@@ -500,7 +505,7 @@ step_strips(StepArgs a, StripShape sh) {
                 for (int m = 0; m < MEQN; m++) {
                     gm[m] = gt[m] + mad(R(0.5), cq[m], zadd(am[O][m]));
                     if constexpr (!FLUXFORM) gpl[P][m] = gt[m] + mad(R(0.5), cq[m], -ap[m]);
-                    if constexpr (CARRY) kept[(CARRY_GPL * MEQN + m) * 64] = gpl[P][m];
+                    if constexpr (CARRY && !FLUXFORM) kept[(CARRY_GPL * MEQN + m) * 64] = gpl[P][m];
                 }
                 R nAd[MEQN], nAu[MEQN];
                 if (STD || a.transverse) {
@@ -549,7 +554,7 @@ step_strips(StepArgs a, StripShape sh) {
                         pd = carry[(CARRY_PD * MEQN + m) * 64];
                         pu = carry[(CARRY_PU * MEQN + m) * 64];
                         xm = last[(CARRY_FXM * MEQN + m) * 64];
-                        xp = last[(CARRY_FXP * MEQN + m) * 64];
+                        if constexpr (!FLUXFORM) xp = last[(CARRY_FXP * MEQN + m) * 64];
                         carry[(CARRY_PD * MEQN + m) * 64] = gPd[P][m];
                         carry[(CARRY_PU * MEQN + m) * 64] = gPu[P][m];
                     }
