@@ -1850,8 +1850,10 @@ int hipclaw_step_batch_noalloc(const hipclaw_config_t* cfg, int npatch, const do
     unsigned long long* dcfl = reinterpret_cast<unsigned long long*>(base);
     int* dslots = reinterpret_cast<int*>(base + NOALLOC_CFL_BYTES);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    HIP_TRY(hipMemcpyAsync(dslots, slots, sizeof(int) * (size_t) nslots, hipMemcpyHostToDevice, st));
-    if (int e = hipclaw::launch_reset_cfl(dcfl, 1, nullptr, st)) return hipfail((hipError_t) e, "reset");
+    // the cleared CFL words and the slot list behind them in one copy
+    std::vector<unsigned char> upload(NOALLOC_CFL_BYTES + sizeof(int) * (size_t) nslots);
+    std::memcpy(upload.data() + NOALLOC_CFL_BYTES, slots, sizeof(int) * (size_t) nslots);
+    HIP_TRY(hipMemcpyAsync(base, upload.data(), upload.size(), hipMemcpyHostToDevice, st));
     hipclaw::StepArgs a;
     a.qsrc = q_in;
     a.qdst = q_out;
@@ -1873,8 +1875,10 @@ int hipclaw_step_batch_noalloc(const hipclaw_config_t* cfg, int npatch, const do
     a.reg_accumulate = 0;
     a.dtscale = nullptr;
     const hipclaw::StepLaunch L(st);
-    int e = launch_solver_step(cfg->solver, cfg->precision, tile, 0, a, L);
-    if (e) return hipfail((hipError_t) e, "step launch");
+    if (int e = launch_solver_step(cfg->solver, cfg->precision, tile, 0, a, L)) {
+        (void) hipStreamSynchronize(st);   // (the copy may still read `upload`)
+        return hipfail((hipError_t) e, "step launch");
+    }
     unsigned long long words[CFL_BYTES / sizeof(unsigned long long)];
     HIP_TRY(hipMemcpyAsync(words, dcfl, CFL_BYTES, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
