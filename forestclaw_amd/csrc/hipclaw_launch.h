@@ -133,8 +133,7 @@ inline int device_simds() {
 }
 
 // pairs: two waves of the kernel fit a SIMD.  lds: its bytes per wave (one wave per
-// workgroup then).  nw: waves per workgroup.  The waves share nothing; one per
-// workgroup lets the dispatcher place each by itself.
+// workgroup then).  nw: waves per workgroup.
 template <typename K>
 inline int launch_strips(K kernel, bool pairs, int lds, int nw, const StepArgs& a, const StepLaunch& L) {
     if (lds > 0) nw = 1;
@@ -176,20 +175,24 @@ inline int launch_step_strips(int nw, const StepArgs& a, const StepLaunch& st) {
                : launch_strips(step_strips<RP, R, FF, 0, false>, pairs, lds, nw, a, st);
 }
 
-// Waves per workgroup by default.  Strips: one.  16 x 16 tiles: four for FP64,
-// two for the FP32-bulk form (a sweep's 18 rows, three per wave, are three
-// groups for each of two waves, where four take two, two, one and one and wait
-// at the barrier; FP64 tiles need the latency hiding of four).
+// Waves per workgroup by default.  Strips: four, which share nothing but lie on the
+// four SIMDs of one CU, beside each other in its cache (one and four, subcycled dam
+// break FP64 9.80 and 9.62 ms, dam break FP64 22.53 and 22.46, shock-bubble FP32
+// 5.20 and 5.16, advection 567 and 565 us; three leave a SIMD of every CU idle).
+// 16 x 16 tiles: four for FP64, two for the FP32-bulk form (a sweep's 18 rows, three
+// per wave, are three groups for each of two waves, where four take two, two, one
+// and one and wait at the barrier; FP64 tiles need the latency hiding of four).
 // hipclaw_set_waves and the autotuner choose 2, 3 or 4.
+constexpr int STRIP_WAVES = 4;
 inline int default_waves(bool strips, bool fp64, int tile) {
-    return tile != 16 ? 0 : strips ? 1 : fp64 ? 4 : 2;   // (0: one choice)
+    return tile != 16 ? 0 : strips ? STRIP_WAVES : fp64 ? 4 : 2;   // (0: one choice)
 }
 
 // waves = 0: the default; 2, 3 or 4 select the variant.
 template <class RP, typename R, bool WITH_REGS>
 inline int launch_step_tile(int tile, int waves, const StepArgs& a, const StepLaunch& st) {
     if constexpr (uses_strips<RP>()) {
-        return launch_step_strips<RP, R, WITH_REGS>(waves > 0 ? waves : 1, a, st);
+        return launch_step_strips<RP, R, WITH_REGS>(waves > 0 ? waves : STRIP_WAVES, a, st);
     } else {
         if (waves == 0) waves = default_waves(false, sizeof(R) == 8, tile);
         switch (tile) {
