@@ -73,7 +73,8 @@ struct SyncProgram {
     int* ops = nullptr;       // [nops][8], grouped by destination
     int* start = nullptr;     // [ngroups + 1]
     int* resets = nullptr;    // [nresets][2] (slot, face)
-    int ngroups = 0, nresets = 0, ops_cap = 0, groups_cap = 0, resets_cap = 0;
+    int* fresh = nullptr;     // [slot] the reset faces as bits (subcycling)
+    int ngroups = 0, nresets = 0, ops_cap = 0, groups_cap = 0, resets_cap = 0, fresh_cap = 0;
     int maxgroup = 0;         // most ops of one destination
     bool set = false;         // installed since the last regrid
 };
@@ -632,6 +633,7 @@ void hipclaw_destroy(hipclaw_state_t* s) {
         hipFree(y.ops);
         hipFree(y.start);
         hipFree(y.resets);
+        hipFree(y.fresh);
     }
     hipFree(s->qlast);
     hipFree(s->qti);
@@ -1048,6 +1050,11 @@ int hipclaw_set_sync_program_k(hipclaw_state_t* s, int k, const int* ops, int no
     if (int rc = upload(s, y.ops, y.ops_cap, ops, 8 * nops, "sync ops")) return rc;
     if (int rc = upload(s, y.start, y.groups_cap, start.data(), ngroups + 1, "sync groups")) return rc;
     if (int rc = upload(s, y.resets, y.resets_cap, resets, 2 * nresets, "register resets")) return rc;
+    std::vector<int> fresh(s->reg_accumulate ? s->npatch : 0, 0);
+    if (s->reg_accumulate) {
+        for (int r = 0; r < nresets; r++) fresh[resets[2 * r]] |= 1 << resets[2 * r + 1];
+        if (int rc = upload(s, y.fresh, y.fresh_cap, fresh.data(), s->npatch, "reset faces")) return rc;
+    }
     HIP_TRY(hipStreamSynchronize(s->st));
     y.ngroups = ngroups;
     y.nresets = nresets;
@@ -1970,16 +1977,27 @@ static int advance_launches(hipclaw_state_t* s, double dt, int nsteps, StepTimer
 // copied whole into qlast, then the step reading that copy and writing the
 // new interiors straight into the current slab, which the other levels keep
 // reading (the same values as stepping the slab itself: qlast holds its
-// every cell).  `due`: the registers of the last synchronisation, still to be
-// zeroed before this update adds to them.
-static int subcycle_update(hipclaw_state_t* s, int level, double dt, hipclaw::Resets& due) {
+// every cell).
+//
+// What a synchronisation leaves to the updates after it: the registers still to be
+// zeroed, with the first update's copy, and which faces those are.  Their first
+// update after it may write instead of add; `stepped` holds the levels that had it.
+struct SyncDue {
+    hipclaw::Resets resets;
+    const int* fresh = nullptr;
+    unsigned long long stepped = 0;
+};
+static int subcycle_update(hipclaw_state_t* s, int level, double dt, SyncDue& due) {
     const int l = level - s->lmin, n = s->loff[l + 1] - s->loff[l];
     const int* slots = s->lslots + s->loff[l];
-    int e = hipclaw::launch_copy_patches(s->q[s->cur], s->qlast, slots, n, s->pstride, due, s->st);
+    int e = hipclaw::launch_copy_patches(s->q[s->cur], s->qlast, slots, n, s->pstride, due.resets, s->st);
     if (e) return hipfail((hipError_t) e, "copy_patches launch");
-    due.n = 0;
+    due.resets.n = 0;
     if (n == 0) return HIPCLAW_OK;
-    return launch_step(s, step_args(s, s->qlast, s->q[s->cur], slots, n, dt));
+    hipclaw::StepArgs a = step_args(s, s->qlast, s->q[s->cur], slots, n, dt);
+    if (!(due.stepped >> l & 1)) a.cmask = due.fresh;
+    due.stepped |= 1ull << l;
+    return launch_step(s, a);
 }
 
 // The time-interpolated copies of a level (fclaw2d_timeinterp).
@@ -2003,7 +2021,7 @@ struct LevelCounter {
 // advance_level (src/fclaw2d_advance.c:112-150, 152-170): the level's step,
 // then, when the coarser level is due, its step and its time-interpolated
 // copies at the finer level's new time.
-static int subcycle_level(hipclaw_state_t* s, int level, int curr_fine_step, LevelCounter* tc, hipclaw::Resets& due) {
+static int subcycle_level(hipclaw_state_t* s, int level, int curr_fine_step, LevelCounter* tc, SyncDue& due) {
     LevelCounter& c = tc[level - s->lmin];
     if (int rc = subcycle_update(s, level, c.dt_step, due)) return rc;
     c.last_step += c.step_inc;
@@ -2020,7 +2038,7 @@ static int subcycle_level(hipclaw_state_t* s, int level, int curr_fine_step, Lev
 
 static int subcycle_launches(hipclaw_state_t* s, double dt, int ncoarse) {
     const int lmin = s->lmin, lmax = s->lmax, nl = lmax - lmin + 1;
-    hipclaw::Resets due;
+    SyncDue due;
     for (int c = 0; c < ncoarse; c++) {
         LevelCounter tc[HIPCLAW_MAX_PROGRAMS];
         for (int l = 0; l < nl; l++) {   // initialize_timestep_counters (:54-110)
@@ -2039,17 +2057,17 @@ static int subcycle_launches(hipclaw_state_t* s, double dt, int ncoarse) {
                 if (int rc = ghost_fill_async(s, k)) return rc;
                 if (s->reg) {
                     if (int rc = time_sync_async(s, k, false)) return rc;
-                    due = resets_of(s, k);
+                    due = SyncDue{resets_of(s, k), s->sp[k].fresh, 0};
                 }
             }
         }
         if (int rc = ghost_fill_async(s, 0)) return rc;
         if (s->reg) {
             if (int rc = time_sync_async(s, 0, false)) return rc;
-            due = resets_of(s, 0);
+            due = SyncDue{resets_of(s, 0), s->sp[0].fresh, 0};
         }
     }
-    return reset_registers(s, due);
+    return reset_registers(s, due.resets);
 }
 
 // What the subcycled advance needs: subcycle state, levels, and the programs

@@ -79,6 +79,9 @@ struct StepArgs {
     // comes from a coarse/fine op); qsrc still holds the values before the
     // fix-up, and staging adds the increments (sync_corner_order).
     const double* qcorr = nullptr;
+    // With reg_accumulate, when there is no fix-up: the faces (bits 0-3 of
+    // cmask[slot]) whose registers are zero, so that a first term may be written
+    // instead of added (nullptr: none known).
     const int* cmask = nullptr;
     long long cstride = 0;
     // Ghost strips staged straight from a same-size neighbour (null: every halo
