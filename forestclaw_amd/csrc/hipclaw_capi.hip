@@ -523,12 +523,13 @@ static int check_config(const hipclaw_config_t* cfg, int* tile_out) {
 // place; with two slabs its patches may be cut into strips of any height, and
 // the update reads same-size ghost strips from the neighbours instead of having
 // them copied first.  Without memory to spare (as much again stays free) the
-// state keeps one slab.
+// state keeps one slab, and so does a subcycling one, whose updates read the copy
+// of the state before them.
 static void second_slab(hipclaw_state_t* s) {
     const size_t bytes = sizeof(double) * (size_t) s->pstride * (size_t) s->max_patches;
     size_t free_bytes = 0, total = 0;
     s->inplace = true;
-    if (hipMemGetInfo(&free_bytes, &total) == hipSuccess && free_bytes / 2 >= bytes &&
+    if (!s->cfg.subcycle && hipMemGetInfo(&free_bytes, &total) == hipSuccess && free_bytes / 2 >= bytes &&
         hipMalloc((void**) &s->q[1], bytes) == hipSuccess)
         s->inplace = false;
     else
