@@ -12,7 +12,9 @@
 #include <cstdio>
 #include <cstring>
 #include <cmath>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <unordered_map>
 #include <vector>
 
@@ -1859,9 +1861,12 @@ int hipclaw_step_batch_noalloc(const hipclaw_config_t* cfg, int npatch, const do
     int* dslots = reinterpret_cast<int*>(base + NOALLOC_CFL_BYTES);
     hipStream_t st = static_cast<hipStream_t>(stream);
     // the cleared CFL words and the slot list behind them in one copy
-    std::vector<unsigned char> upload(NOALLOC_CFL_BYTES + sizeof(int) * (size_t) nslots);
-    std::memcpy(upload.data() + NOALLOC_CFL_BYTES, slots, sizeof(int) * (size_t) nslots);
-    HIP_TRY(hipMemcpyAsync(base, upload.data(), upload.size(), hipMemcpyHostToDevice, st));
+    const size_t nupload = NOALLOC_CFL_BYTES + sizeof(int) * (size_t) nslots;
+    std::unique_ptr<unsigned char[]> upload(new (std::nothrow) unsigned char[nupload]);
+    if (!upload) return fail(HIPCLAW_ENOMEM, "hipclaw_step_batch_noalloc: host allocation failed%s");
+    std::memset(upload.get(), 0, NOALLOC_CFL_BYTES);
+    std::memcpy(upload.get() + NOALLOC_CFL_BYTES, slots, sizeof(int) * (size_t) nslots);
+    HIP_TRY(hipMemcpyAsync(base, upload.get(), nupload, hipMemcpyHostToDevice, st));
     hipclaw::StepArgs a;
     a.qsrc = q_in;
     a.qdst = q_out;
