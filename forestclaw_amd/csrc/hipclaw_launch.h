@@ -113,9 +113,9 @@ inline int launch_step_shape(const StepArgs& a, const StepLaunch& st) {
 // components (Euler's 4 x 4) at most; a solver with more of them runs on tiles.
 // Below that strips are faster wherever a launch has a few hundred waves'
 // work, and no slower than 1.2 times the tiles where it has less (kernel times
-// with tiles and with strips, us: shallow water FP64 16 x 16, 16 patches 12.4 /
-// 13.7, 256 15.7 / 18.0, 2800 77 / 65; 32 x 32, 6000 patches FP64 534 / 371,
-// FP32-bulk 194 / 144; Euler FP64 899 / 630; advection FP64 142 / 67).
+// with tiles and with strips, us: shallow water FP64 16 x 16, 16 patches 14.7 /
+// 16.4, 256 25.6 / 20.1, 2800 82 / 63; 32 x 32, 6000 patches FP64 569 / 346,
+// FP32-bulk 206 / 145; Euler FP64 856 / 502; advection FP64 140 / 69).
 template <class RP>
 constexpr bool uses_strips() { return RP::MEQN * RP::MWAVES <= 16; }
 

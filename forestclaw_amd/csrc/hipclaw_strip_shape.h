@@ -71,9 +71,9 @@ inline bool strip_pattern(int mx, bool whole, StripShape& sh) {
 // H + 3 row steps each (three rows lead in).  Alone on its SIMD a wave waits for
 // its own results a sixth of the time, which a second one would use (`pairs`:
 // the kernel's registers leave room for it).  Kernel times, us: shallow water
-// FP64, 700 patches of 32 x 32 (420 waves of columns), H = 4, 8, 16, 32: 72, 61,
-// 63, 111; 256 of 16 x 16 (86), H = 1, 2, 4, 8, 16: 22, 18, 24, 35, 59; Euler
-// FP32-bulk, 2800 of 16 x 16 (934), H = 4, 8, 16: 54, 42, 44.
+// FP64, 700 patches of 32 x 32 (420 waves of columns), H = 4, 8, 16, 32: 71, 62,
+// 66, 110; 256 of 16 x 16 (86), H = 1, 2, 4, 8, 16: 23, 20, 25, 36, 59; Euler
+// FP32-bulk, 2800 of 16 x 16 (934), H = 4, 8, 16: 50, 42, 45.
 inline void strip_rows(int my, int nwork, int simds, bool pairs, bool whole, StripShape& sh) {
     const double cols = (double) nwork * sh.waves / sh.patches;
     double best = 0.0;

@@ -1,10 +1,10 @@
 // Batched patch update, one wave per group of column strips.
 //
-// The same step as step_tiles (hipclaw_step.h), organised without LDS and
-// without barriers: a wave holds S strips of W interior columns, one staged
-// column (W + 4 of them, with the halo) per lane, and marches up the rows.
-// Rows and the y-interfaces between them live in registers; the x-direction
-// goes across lanes with DPP shifts.  With row n loaded the wave
+// The same step as step_tiles (hipclaw_step.h), organised without barriers: a
+// wave holds S strips of W interior columns, one staged column (W + 4 of them,
+// with the halo) per lane, and marches up the rows.  Rows and the y-interfaces
+// between them live in registers (some in the lane's own LDS words where that
+// gains a wave per SIMD); the x-direction goes across lanes with DPP shifts.  With row n loaded the wave
 //
 //   * sweeps row n - 1 in x (normal and transverse solves);
 //   * solves the y-interface between rows n - 1 and n;
