@@ -61,9 +61,9 @@ __device__ __forceinline__ float pick(bool c, float a, float b) { return c ? a :
 // select); FP32 uses the hardware v_min_f32 / v_max_f32, which differ only
 // for NaN operands.
 template <typename R>
-__device__ __forceinline__ R rmin(R a, R b) { return pick(a < b, a, b); }
+__device__ __forceinline__ R rmin(R a, R b) { return a < b ? a : b; }
 template <typename R>
-__device__ __forceinline__ R rmax(R a, R b) { return pick(a > b, a, b); }
+__device__ __forceinline__ R rmax(R a, R b) { return a > b ? a : b; }
 template <>
 __device__ __forceinline__ float rmin<float>(float a, float b) { return __builtin_fminf(a, b); }
 template <>

@@ -58,7 +58,7 @@ __device__ __forceinline__ void limited_correction(const StepArgs& a, const R wa
             phi[mw] = STD ? rmax(0.0f, rmin(rmin(mad(0.5f, r, 0.5f), 2.0f), 2.0f * r)) : philim<float>(mth, r);
         } else {
             const R rr = dv(d, wn);
-            phi[mw] = pick(wave_nonzero(wn), philim<R>(mth, rr), R(1));
+            phi[mw] = pick(wave_nonzero(wn), philim<R, true>(mth, rr), R(1));
         }
     }
     R c[MW];
