@@ -26,8 +26,10 @@ extern "C" {
 #endif
 
 /* Version of the descriptor and of the kernel argument block its launchers
- * take; a descriptor built against another version is refused. */
-#define HIPCLAW_SOLVER_ABI 1
+ * take, the memory it points to included; a descriptor built against another
+ * version is refused.  1: the Courant number is one word.  2: it is a block of
+ * words (StepArgs::cfl). */
+#define HIPCLAW_SOLVER_ABI 2
 
 /* Registered solvers get numbers from HIPCLAW_RP_USER on. */
 #define HIPCLAW_RP_USER 16
