@@ -1759,6 +1759,7 @@ static hipclaw::StepArgs step_args(hipclaw_state_t* s, const double* src, double
     a.cfl = s->cfl;
     a.pstride = s->pstride;
     a.astride = s->astride;
+    a.clock = 0;
     a.nwork = n;
     a.mx = s->cfg.mx; a.my = s->cfg.my; a.mbc = s->cfg.mbc;
     a.ntx = s->ntx; a.nty = s->nty;
@@ -1878,6 +1879,7 @@ int hipclaw_step_batch_noalloc(const hipclaw_config_t* cfg, int npatch, const do
     const long long cells = (long long) (cfg->mx + 2 * cfg->mbc) * (cfg->my + 2 * cfg->mbc);
     a.pstride = cells * cfg->meqn;
     a.astride = cells * cfg->maux;
+    a.clock = 0;
     a.nwork = nslots;
     a.mx = cfg->mx; a.my = cfg->my; a.mbc = cfg->mbc;
     a.ntx = ntx; a.nty = nty;
@@ -1911,6 +1913,7 @@ static int advance_step(hipclaw_state_t* s, hipclaw::StepArgs& a, int step, Step
             if (int e = hipclaw::launch_collect_steps(s->cfl, hipclaw::STEP_BLOCKS, s->sum, nullptr, s->st))
                 return hipfail((hipError_t) e, "collect_steps launch");
         a.cfl = s->cfl + (size_t) block * hipclaw::CFL_BLOCK;
+        a.clock = 1;
     }
     return launch_step(s, a);
 }

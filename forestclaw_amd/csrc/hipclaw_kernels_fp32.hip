@@ -8,8 +8,8 @@ namespace hipclaw {
 
 int launch_step_fp32(int solver, int tile, int waves, const StepArgs& a, const StepLaunch& st) {
     switch (solver) {
-    case 0: return launch_step_tile<RPAdvection<float>, float, true>(tile, waves, a, st);
-    case 1: return launch_step_tile<RPShallow<float>, float, true>(tile, waves, a, st);
+    case 0: return launch_step_tile<RPAdvection<float>, float, true, true>(tile, waves, a, st);
+    case 1: return launch_step_tile<RPShallow<float>, float, true, true>(tile, waves, a, st);
     case 2: return launch_step_tile<RPEuler<float>, float, true>(tile, waves, a, st);
     default: return (int) hipErrorInvalidValue;
     }

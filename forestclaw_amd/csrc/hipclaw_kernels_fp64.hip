@@ -1396,7 +1396,7 @@ int launch_time_sync(const SyncArgs& a, hipStream_t st) {
 int launch_step_fp64(int solver, int tile, int waves, const StepArgs& a, const StepLaunch& st) {
     switch (solver) {
     case 0: return launch_step_tile<RPAdvection<double>, double, true>(tile, waves, a, st);
-    case 1: return launch_step_tile<RPShallow<double>, double, true>(tile, waves, a, st);
+    case 1: return launch_step_tile<RPShallow<double>, double, true, true>(tile, waves, a, st);
     case 2: return launch_step_tile<RPEuler<double>, double, true>(tile, waves, a, st);
     default: return (int) hipErrorInvalidValue;
     }

@@ -1,7 +1,7 @@
 // Launch dispatch of the step kernel for one Riemann functor: the strip kernel
-// (step_strips), or for solvers with more wave components than a lane can keep
-// the LDS tile kernel (step_tiles); time-sync registers and the compile-time
-// method pick the instantiation.  Shared by the built-in solvers' two
+// (step_strips), or for small launches and for solvers with more wave components
+// than a lane can keep the LDS tile kernel (step_tiles); time-sync registers and the
+// compile-time method pick the instantiation.  Shared by the built-in solvers' two
 // translation units (FP64 compiled without FMA contraction, FP32-bulk with it)
 // and by solvers an application compiles itself (hipclaw_user_solver.h); the
 // instantiations take the contraction mode of the unit that includes this.
@@ -109,15 +109,15 @@ inline int launch_step_shape(const StepArgs& a, const StepLaunch& st) {
     }
 }
 
-// Strips keep one interface's waves of three rows in registers, 16 wave
-// components (Euler's 4 x 4) at most; a solver with more of them runs on tiles.
-// Below that strips are faster wherever a launch has a few hundred waves'
-// work, and no slower than 1.2 times the tiles where it has less (kernel times
-// with tiles and with strips, us: shallow water FP64 16 x 16, 16 patches 14.7 /
-// 16.4, 256 25.6 / 20.1, 2800 82 / 63; 32 x 32, 6000 patches FP64 569 / 346,
+// Whether a launch of a solver that uses strips goes to the tile kernel all the same
+// (tiles_pay).  Larger launches are faster in strips (tiles and strips, us: shallow
+// water FP64 16 x 16, 2800 patches 82 / 63; 32 x 32, 6000 patches FP64 569 / 346,
 // FP32-bulk 206 / 145; Euler FP64 856 / 502; advection FP64 140 / 69).
-template <class RP>
-constexpr bool uses_strips() { return RP::MEQN * RP::MWAVES <= 16; }
+inline bool launches_tiles(const StepArgs& a, int tile, int wave_bytes, int simds) {
+    const bool inplace = a.qsrc == a.qdst;
+    if (inplace && a.ntx * a.nty != 1) return false;
+    return tiles_pay(wave_bytes, tile, a.mx, a.my, a.nwork, a.ntx * a.nty, simds, a.reg != nullptr, inplace);
+}
 
 inline int device_simds() {
     static std::atomic<int> simds{0};
@@ -188,22 +188,42 @@ inline int default_waves(bool strips, bool fp64, int tile) {
     return tile != 16 ? 0 : strips ? STRIP_WAVES : fp64 ? 4 : 2;   // (0: one choice)
 }
 
+// Whether the tile kernel is instantiated for a tile (T = 32 only WITH32).
+template <class RP, typename R, bool WITH_REGS, bool WITH32>
+constexpr bool has_tile(int tile, bool regs) {
+    constexpr bool FF = sizeof(R) == 4 && RP::CONSERVATIVE;
+    if (regs && !WITH_REGS) return false;
+    return tile == 8    ? (regs ? step_fits<RP, R, 8, FF, true>() : step_fits<RP, R, 8, FF, false>())
+           : tile == 16 ? (regs ? step_fits<RP, R, 16, FF, true>() : step_fits<RP, R, 16, FF, false>())
+                        : WITH32 && tile == 32 &&
+                              (regs ? step_fits<RP, R, 32, FF, true>() : step_fits<RP, R, 32, FF, false>());
+}
+
+template <class RP, typename R, bool WITH_REGS, bool WITH32>
+inline int launch_step_tiles(int tile, int waves, const StepArgs& a, const StepLaunch& st) {
+    if (waves == 0) waves = default_waves(false, sizeof(R) == 8, tile);
+    switch (tile) {
+    case 8: return launch_step_shape<RP, R, 8, 2, WITH_REGS>(a, st);
+    case 16:
+        return waves == 2 ? launch_step_shape<RP, R, 16, 2, WITH_REGS>(a, st)
+             : waves == 3 ? launch_step_shape<RP, R, 16, 3, WITH_REGS>(a, st)
+                          : launch_step_shape<RP, R, 16, 4, WITH_REGS>(a, st);
+    case 32:
+        if constexpr (WITH32) return launch_step_shape<RP, R, 32, 16, WITH_REGS>(a, st);
+        return (int) hipErrorInvalidValue;
+    default: return (int) hipErrorInvalidValue;
+    }
+}
+
 // waves = 0: the default; 2, 3 or 4 select the variant.
-template <class RP, typename R, bool WITH_REGS>
+template <class RP, typename R, bool WITH_REGS, bool WITH32 = false>
 inline int launch_step_tile(int tile, int waves, const StepArgs& a, const StepLaunch& st) {
     if constexpr (uses_strips<RP>()) {
-        return launch_step_strips<RP, R, WITH_REGS>(waves > 0 ? waves : STRIP_WAVES, a, st);
-    } else {
-        if (waves == 0) waves = default_waves(false, sizeof(R) == 8, tile);
-        switch (tile) {
-        case 8: return launch_step_shape<RP, R, 8, 2, WITH_REGS>(a, st);
-        case 16:
-            return waves == 2 ? launch_step_shape<RP, R, 16, 2, WITH_REGS>(a, st)
-                 : waves == 3 ? launch_step_shape<RP, R, 16, 3, WITH_REGS>(a, st)
-                              : launch_step_shape<RP, R, 16, 4, WITH_REGS>(a, st);
-        default: return (int) hipErrorInvalidValue;
-        }
+        if (!has_tile<RP, R, WITH_REGS, WITH32>(tile, a.reg != nullptr) ||
+            !launches_tiles(a, tile, RP::MEQN * RP::MWAVES * (int) sizeof(R), device_simds()))
+            return launch_step_strips<RP, R, WITH_REGS>(waves > 0 ? waves : STRIP_WAVES, a, st);
     }
+    return launch_step_tiles<RP, R, WITH_REGS, WITH32>(tile, waves, a, st);
 }
 
 }  // namespace hipclaw

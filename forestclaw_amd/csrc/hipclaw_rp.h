@@ -970,6 +970,7 @@ struct RPAdvection {
                                                 const PhysParams&, R wave[MWAVES][MEQN],
                                                 R s[MWAVES], R amdq[MEQN], R apdq[MEQN],
                                                 R roe[NROE]) {
+#pragma clang fp contract(off)
         const R delta = qR[0] - qL[0];
         wave[0][0] = delta;
         s[0] = auxR[IXY - 1];
@@ -982,6 +983,7 @@ struct RPAdvection {
     __device__ __forceinline__ static void rpt2(const R* /*roe*/, const R asdq[MEQN],
                                                 const R* /*aux1*/, const R* aux2, const R* aux3,
                                                 const PhysParams&, R bm[MEQN], R bp[MEQN]) {
+#pragma clang fp contract(off)
         constexpr int kv = IXY == 1 ? 1 : 0;   // the transverse velocity component
         bm[0] = rneg(aux2[kv]) * asdq[0];
         bp[0] = rplus(aux3[kv]) * asdq[0];

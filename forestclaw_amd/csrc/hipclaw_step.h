@@ -51,10 +51,12 @@ struct StepArgs {
     // of them: atomics on one word are served one after another, ~11 ns each.
     // Beside each of them stands a clock word, the largest of which is when the
     // launch's last wave ended, and beside that, in the first, when the launch
-    // began (step_strips; wall clock ticks).
+    // began (wall clock ticks); the tile kernel's small launches, 0.2 us of 8, keep
+    // them only with `clock`.
     unsigned long long* cfl;
     long long pstride;         // doubles per patch in q
     long long astride;         // doubles per patch in aux
+    int clock;
     int nwork;
     int mx, my, mbc;
     int ntx, nty;              // tiles per patch in x and y
@@ -107,9 +109,11 @@ enum { REG_FM = 0, REG_FP = 1, REG_EFIN = 2, REG_EFOUT = 3 };
 // every register is reset at every synchronisation (no subcycling) the
 // previous value is zero and need not be read.
 __device__ __forceinline__ void reg_add(double* r, double v, int accumulate) {
+#pragma clang fp contract(off)
     *r = (accumulate ? *r : 0.0) + v;
 }
 __device__ __forceinline__ void reg_sub(double* r, double v, int accumulate) {
+#pragma clang fp contract(off)
     *r = (accumulate ? *r : 0.0) - v;
 }
 
@@ -229,9 +233,142 @@ __device__ __forceinline__ void riemann(const R* qL, const R* qR, const R* auxL,
     }
 }
 
-// The tile kernel serves the solvers with more wave components per interface
-// (meqn x mwaves > 16) than the strip kernel's lanes can keep; the allocator
-// sizes it without a target for the waves per SIMD.
+// Limiter and second-order correction of one interface (clawpack46_inlinelimiter.f,
+// clawpack46_flux2.f:139-153).  dotl, dotr: the waves' products with those of
+// the interface before and after.  FP64 limits the waves and sums them in the
+// reference's order; FP32 puts the limiter into the sum's coefficients, and a
+// wave whose norm is below the smallest normal number has the limiter of a
+// slightly larger one (its terms are below 1e-19 either way, save those of the
+// Beam-Warming limiter, which lie between zero and the neighbour's wave, FP64's).
+// PICK: as philim's.
+template <class RP, typename R, int IXY, bool STD, bool PICK>
+__device__ __forceinline__ void limited_correction(const StepArgs& a, const R wave[RP::MWAVES][RP::MEQN],
+                                                   const R s[RP::MWAVES], const R dotl[RP::MWAVES],
+                                                   const R dotr[RP::MWAVES], R dtd, R cqxx[RP::MEQN]) {
+#pragma clang fp contract(off)
+    constexpr int MEQN = RP::MEQN, MW = RP::MWAVES;
+    using WZ = wave_zeros<RP, IXY>;
+    R phi[MW];
+#pragma unroll
+    for (int mw = 0; mw < MW; mw++) {
+        phi[mw] = R(1);
+        const int mth = STD ? 4 : a.mthlim[mw];
+        if (mth == 0) continue;
+        R wn = R(0);
+        bool first = true;
+#pragma unroll
+        for (int m = 0; m < MEQN; m++)
+            if (!WZ::at(mw, m)) sum_term(wn, wave[mw][m], wave[mw][m], first);
+        const bool up = s[mw] > R(0);
+        const R d = PICK ? pick(up, dotl[mw], dotr[mw]) : up ? dotl[mw] : dotr[mw];
+        if constexpr (sizeof(R) == 4) {
+            const float r = d * __builtin_amdgcn_rcpf(rmax(wn, 1.17549435e-38f));
+            phi[mw] = STD ? rmax(0.0f, rmin(rmin(mad(0.5f, r, 0.5f), 2.0f), 2.0f * r)) : philim<float>(mth, r);
+        } else {
+            const R rr = dv(d, wn);
+            const R lim = philim<R, PICK>(mth, rr);
+            phi[mw] = PICK ? pick(wave_nonzero(wn), lim, R(1)) : wave_nonzero(wn) ? lim : R(1);
+        }
+    }
+    R c[MW];
+#pragma unroll
+    for (int mw = 0; mw < MW; mw++) {
+        const R as = fabs(s[mw]);
+        if constexpr (sizeof(R) == 4) c[mw] = mad(-(as * dtd), as, as) * phi[mw];
+        else c[mw] = as * (R(1) - as * dtd);
+    }
+#pragma unroll
+    for (int m = 0; m < MEQN; m++) {
+        R sum = R(0);
+        bool first = true;
+#pragma unroll
+        for (int mw = 0; mw < MW; mw++) {
+            if (WZ::at(mw, m)) continue;
+            if constexpr (sizeof(R) == 4) sum_term(sum, c[mw], wave[mw][m], first);
+            else sum_term(sum, c[mw], phi[mw] * wave[mw][m], first);
+        }
+        cqxx[m] = sum;
+    }
+}
+
+// a b + c in one rounding: the FP32-bulk form's FP64 state update
+__device__ __forceinline__ double fmad64(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// Solvers the strip kernel (hipclaw_strips.h) serves: it keeps one interface's
+// waves of three rows in registers, 16 wave components (Euler's 4 x 4) at most.
+template <class RP>
+constexpr bool uses_strips() { return RP::MEQN * RP::MWAVES <= 16; }
+
+// The tile kernel's second-order correction of the interface of each lane, the
+// one before it on the lane before.  Solvers of the strip kernel take that one's
+// operations, so that both give the same bits.  `used`: some cell of the tile
+// reads the interface's flux.
+template <class RP, typename R, int IXY, int LIM>
+__device__ __forceinline__ void tile_correction(const StepArgs& a, R wave[RP::MWAVES][RP::MEQN],
+                                                const R s[RP::MWAVES], R dtd, bool used, R cqxx[RP::MEQN]) {
+    constexpr int MEQN = RP::MEQN, MW = RP::MWAVES;
+    using WZ = wave_zeros<RP, IXY>;
+#pragma unroll
+    for (int m = 0; m < MEQN; m++) cqxx[m] = R(0);
+    if (!a.order2) return;
+    if constexpr (uses_strips<RP>()) {
+        R dotl[MW], dotr[MW];
+#pragma unroll
+        for (int mw = 0; mw < MW; mw++) {
+            dotl[mw] = R(0);
+            bool first = true;
+#pragma unroll
+            for (int m = 0; m < MEQN; m++) {
+                if (WZ::at(mw, m)) continue;
+                const R wl = prev_lane(wave[mw][m]);
+                sum_term(dotl[mw], wl, wave[mw][m], first);
+            }
+            dotr[mw] = next_lane(dotl[mw]);
+        }
+        limited_correction<RP, R, IXY, LIM == 4, false>(a, wave, s, dotl, dotr, dtd, cqxx);
+    } else {
+#pragma unroll
+        for (int mw = 0; mw < MW; mw++) {
+            const int mth = LIM > 0 ? LIM : a.mthlim[mw];
+            if (mth == 0) continue;
+            R wn = R(0), dotl = R(0);
+#pragma unroll
+            for (int m = 0; m < MEQN; m++)
+                if (!WZ::at(mw, m)) wn = wn + wave[mw][m] * wave[mw][m];
+#pragma unroll
+            for (int m = 0; m < MEQN; m++) {
+                if (WZ::at(mw, m)) continue;
+                const R wl = prev_lane(wave[mw][m]);
+                dotl = dotl + wl * wave[mw][m];
+            }
+            const R dotr = next_lane(dotl);
+            // phi = 1 where the reference leaves the wave as it is (zero norm, or an
+            // interface whose flux no cell of the tile reads): phi * w = w bit for bit
+            const R rr = dv(s[mw] > R(0) ? dotl : dotr, wn);
+            const R phi = used && wave_nonzero(wn) ? philim<R>(mth, rr) : R(1);
+#pragma unroll
+            for (int m = 0; m < MEQN; m++)
+                if (!WZ::at(mw, m)) wave[mw][m] = phi * wave[mw][m];
+        }
+#pragma unroll
+        for (int m = 0; m < MEQN; m++) {
+            R c = R(0);
+#pragma unroll
+            for (int mw = 0; mw < MW; mw++)
+                if (!WZ::at(mw, m)) c = c + fabs(s[mw]) * (R(1) - fabs(s[mw]) * dtd) * wave[mw][m];
+            cqxx[m] = c;
+        }
+    }
+}
+
+// The tile kernel serves the solvers with more wave components, and the small
+// launches of the others (tiles_pay).
+//
+// Waves per SIMD the register allocation aims for: 4, except FP64 16 x 16
+// tiles, which need more than the 128 VGPRs of 4 waves and are held to the 168
+// of 3 (without the target the allocator let them grow to 2 waves).  A solver
+// with more than 16 wave components cannot keep them in the registers of 4
+// waves; it gets no target and the allocator sizes the kernel itself.
 //
 // LIM = 0 reads each wave family's limiter from a.mthlim at run time; LIM > 0
 // is that limiter for every family, fixed at compile time.  The run-time
@@ -239,8 +376,13 @@ __device__ __forceinline__ void riemann(const R* qL, const R* qR, const R* auxL,
 // sweeps and, with the kernel's other uniform values, spills scalar
 // registers into vector lanes; the fixed form has neither (about 40 % fewer
 // vector instructions in each sweep for the MC limiter).
+template <class RP, typename R, int T>
+constexpr int step_waves_per_eu() {
+    return !uses_strips<RP>() ? 1 : sizeof(R) == 8 && T == 16 ? 3 : 4;
+}
+
 template <class RP, typename R, int T, int NW, bool FLUXFORM, bool REGS, int LIM = 0>
-__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1)))
+__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(step_waves_per_eu<RP, R, T>())))
 step_tiles(StepArgs a) {
     constexpr int MEQN = RP::MEQN, MW = RP::MWAVES, MAUX = RP::MAUX, NROE = RP::NROE;
     // wave components zero by construction, skipped in the sums over waves
@@ -263,6 +405,7 @@ step_tiles(StepArgs a) {
     R* const s_gt = sm.gt();
     R* const s_ab = sm.ab();
 
+    if (a.clock && blockIdx.x == 0 && threadIdx.x == 0) a.cfl[2] = __builtin_amdgcn_s_memrealtime();
     const int ntiles = a.nwork * a.ntx * a.nty;
     const int mx = a.mx, my = a.my, mbc = a.mbc;
     const int nxp = mx + 2 * mbc, nyp = my + 2 * mbc;
@@ -547,42 +690,7 @@ step_tiles(StepArgs a) {
                 for (int mw = 0; mw < MW; mw++) smax = fmax(smax, fabs(s[mw]));
             }
             R cqxx[MEQN];
-#pragma unroll
-            for (int m = 0; m < MEQN; m++) cqxx[m] = R(0);
-            if (a.order2) {
-#pragma unroll
-                for (int mw = 0; mw < MW; mw++) {
-                    const int mth = LIM > 0 ? LIM : a.mthlim[mw];
-                    if (mth == 0) continue;
-                    R wn = R(0), dotl = R(0);
-#pragma unroll
-                    for (int m = 0; m < MEQN; m++)
-                        if (!WZ1::at(mw, m)) wn = wn + wave_[mw][m] * wave_[mw][m];
-#pragma unroll
-                    for (int m = 0; m < MEQN; m++) {
-                        if (WZ1::at(mw, m)) continue;
-                        const R wl = prev_lane(wave_[mw][m]);
-                        dotl = dotl + wl * wave_[mw][m];
-                    }
-                    const R dotr = next_lane(dotl);
-                    // phi = 1 where the reference leaves the wave as it is (zero
-                    // norm, or an interface whose flux no cell of the tile reads):
-                    // phi * w = w bit for bit
-                    const R rr = dv(s[mw] > R(0) ? dotl : dotr, wn);
-                    const R phi = (k >= 1 && k <= T + 1 && wave_nonzero(wn)) ? philim<R>(mth, rr) : R(1);
-#pragma unroll
-                    for (int m = 0; m < MEQN; m++)
-                        if (!WZ1::at(mw, m)) wave_[mw][m] = phi * wave_[mw][m];
-                }
-#pragma unroll
-                for (int m = 0; m < MEQN; m++) {
-                    R c = R(0);
-#pragma unroll
-                    for (int mw = 0; mw < MW; mw++)
-                        if (!WZ1::at(mw, m)) c = c + fabs(s[mw]) * (R(1) - fabs(s[mw]) * dtdx) * wave_[mw][m];
-                    cqxx[m] = c;
-                }
-            }
+            tile_correction<RP, R, 1, LIM>(a, wave_, s, dtdx, k >= 1 && k <= T + 1, cqxx);
             if (act && r >= 1 && r <= T && k >= 1 && k <= T + 1) {
 #pragma unroll
                 for (int m = 0; m < MEQN; m++) {
@@ -672,42 +780,7 @@ step_tiles(StepArgs a) {
                 for (int mw = 0; mw < MW; mw++) smax = fmax(smax, fabs(s[mw]));
             }
             R cqxx[MEQN];
-#pragma unroll
-            for (int m = 0; m < MEQN; m++) cqxx[m] = R(0);
-            if (a.order2) {
-#pragma unroll
-                for (int mw = 0; mw < MW; mw++) {
-                    const int mth = LIM > 0 ? LIM : a.mthlim[mw];
-                    if (mth == 0) continue;
-                    R wn = R(0), dotl = R(0);
-#pragma unroll
-                    for (int m = 0; m < MEQN; m++)
-                        if (!WZ2::at(mw, m)) wn = wn + wave_[mw][m] * wave_[mw][m];
-#pragma unroll
-                    for (int m = 0; m < MEQN; m++) {
-                        if (WZ2::at(mw, m)) continue;
-                        const R wl = prev_lane(wave_[mw][m]);
-                        dotl = dotl + wl * wave_[mw][m];
-                    }
-                    const R dotr = next_lane(dotl);
-                    // phi = 1 where the reference leaves the wave as it is (zero
-                    // norm, or an interface whose flux no cell of the tile reads):
-                    // phi * w = w bit for bit
-                    const R rr = dv(s[mw] > R(0) ? dotl : dotr, wn);
-                    const R phi = (k >= 1 && k <= T + 1 && wave_nonzero(wn)) ? philim<R>(mth, rr) : R(1);
-#pragma unroll
-                    for (int m = 0; m < MEQN; m++)
-                        if (!WZ2::at(mw, m)) wave_[mw][m] = phi * wave_[mw][m];
-                }
-#pragma unroll
-                for (int m = 0; m < MEQN; m++) {
-                    R cq = R(0);
-#pragma unroll
-                    for (int mw = 0; mw < MW; mw++)
-                        if (!WZ2::at(mw, m)) cq = cq + fabs(s[mw]) * (R(1) - fabs(s[mw]) * dtdy) * wave_[mw][m];
-                    cqxx[m] = cq;
-                }
-            }
+            tile_correction<RP, R, 2, LIM>(a, wave_, s, dtdy, k >= 1 && k <= T + 1, cqxx);
             // normal y-fluxes: gm = gt + faddm, gp = gt + faddp
             const bool own_col = c >= 1 && c <= T;
             if constexpr (FLUXFORM) {
@@ -804,7 +877,7 @@ step_tiles(StepArgs a) {
                 if constexpr (sizeof(R) == sizeof(double))
                     qo[off] = (qc - dtdx * Dx) - dtdy * Dy;
                 else  // FP32 fluctuations, FP64 state: q never passes through FP32
-                    qo[off] = (qc - dtdx64 * (double) Dx) - dtdy64 * (double) Dy;
+                    qo[off] = fmad64(-dtdy64, (double) Dy, fmad64(-dtdx64, (double) Dx, qc));
             }
             if constexpr (REGS) {
                 double* __restrict__ rg = a.reg + (long long) slot * a.rstride;
@@ -890,7 +963,7 @@ step_tiles(StepArgs a) {
                     const double qc = SQD(m, c + 2, b + 2);
                     const double dfx = xflux(c + 1, b, m, fc[m]) - xflux(c, b, m, fl[m]);
                     const double dgy = yflux(b + 1, c, m, gc[m]) - yflux(b, c, m, gb[m]);
-                    qo[off] = (qc - dtdx64 * dfx) - dtdy64 * dgy;
+                    qo[off] = fmad64(-dtdy64, dgy, fmad64(-dtdx64, dfx, qc));
                 }
             }
         }
@@ -900,7 +973,11 @@ step_tiles(StepArgs a) {
     // ---- CFL: wave64 max over all tiles of this workgroup, one atomic per wave ----
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) cfl = fmax(cfl, __shfl_xor(cfl, off, 64));
-    if (lane == 0 && cfl > 0.0) atomicMax(a.cfl, (unsigned long long) __double_as_longlong(cfl));
+    if (lane == 0) {
+        unsigned long long* w = a.cfl + ((blockIdx.x * NW + wave) & (CFL_WORDS - 1)) * CFL_STRIDE;
+        if (cfl > 0.0) atomicMax(w, (unsigned long long) __double_as_longlong(cfl));
+        if (a.clock) atomicMax(w + 1, (unsigned long long) __builtin_amdgcn_s_memrealtime());
+    }
 }
 
 }  // namespace hipclaw

@@ -1,5 +1,6 @@
 // How a launch of the strip kernel (hipclaw_strips.h) lays the patches of its
-// work list on waves of 64 lanes.  Host code, without HIP.
+// work list on waves of 64 lanes, and which launches the tile kernel takes instead.
+// Host code, without HIP.
 #pragma once
 
 namespace hipclaw {
@@ -87,6 +88,45 @@ inline void strip_rows(int my, int nwork, int simds, bool pairs, bool whole, Str
         if (nsy == 1 || cost < best) { best = cost; sh.nsy = nsy; }
     }
     sh.H = (my + sh.nsy - 1) / sh.nsy;
+}
+
+// Whether a launch takes less time on the tile kernel, whose waves share a tile's
+// rows: a strip's wave, alone on its SIMD, issues one instruction per four cycles
+// and leads in with five row steps, so strips win once their waves fill the SIMDs.
+// Kernel times in us, tiles and strips:
+//   T = 8   shallow water FP64 24 x 20 (9 tiles each), 16 patches 7.9 / 14.6, 133
+//           15.7 / 18.4, 266 29.1 / 22.0; FP32-bulk 16 5.6 / 7.5, 66 8.1 / 8.2, 133
+//           10.6 / 9.5; advection FP64 16 4.5 / 5.8, 66 6.6 / 6.1
+//   T = 16  shallow water FP64 16 x 16, 15 patches 12.4 / 14.6, 500 18.4 / 22.1, 1000
+//           39.7 / 32.2; Euler FP64 250 16.8 / 24.5, 1000 43.3 / 44.2; lighter solvers
+//           and the FP32-bulk form 0.7 to 1.0 times as long with strips
+//   T = 32  shallow water FP64 32 x 32, 1 patch 29.5 / 14.6, 700 85 / 62
+// and with time-sync registers, which the tiles store at the end of a tile,
+//   T = 8   shallow water FP64 24 x 24, strips 1.24 times as long with 88 patches and
+//           0.8 with 333; FP32-bulk 1.07 with 28, 0.91 with 44
+// Tiles that overlap (a patch the tile does not divide) compute cells twice, and
+// count as much more.
+// In place a patch is one strip of all its rows, a serial chain: tiles until the
+// strips' waves fill three quarters of the SIMDs (half of them for a solver of few
+// wave components).  Shallow water FP64 8 x 8, 1 patch 6.6 / 30.7, 2000 17.1 / 32.9,
+// 4000 29.1 / 33.9, 8000 52.8 / 51.7; 16 x 16, 1 patch 11.6 / 52.6, 2000 53.6 / 56.8,
+// 3000 76 / 64; 32 x 32 (T = 32) 28.5 / 96, 700 80 / 101; advection FP64 8 x 8, 1000
+// 6.9 / 9.4, 2000 9.9 / 9.7.
+// wave_bytes: of one interface's waves (meqn x mwaves values).
+inline bool tiles_pay(int wave_bytes, int tile, int mx, int my, int nwork, int tiles_per_patch, int simds, bool regs,
+                      bool inplace) {
+    const long long cus = simds / 4;
+    if (inplace) {
+        const int across = StripShape::LANES / (mx + StripShape::HALO);
+        const int per_wave = across < 1 ? 1 : across < StripShape::SEGS ? across : StripShape::SEGS;
+        return 4LL * nwork <= (wave_bytes >= 24 ? 3LL : 2LL) * simds * per_wave;
+    }
+    const bool heavy = wave_bytes >= 72;
+    double most;                 // tiles per CU
+    if (tile == 8) most = regs ? (heavy ? 4 : 1) : heavy ? 8 : wave_bytes < 9 ? 1 : wave_bytes / 9.0;
+    else most = tile == 16 && heavy ? 2 : 0;
+    const double ntiles = (double) nwork * tiles_per_patch, twice = (double) tiles_per_patch * tile * tile / ((double) mx * my);
+    return ntiles * twice <= most * cus;
 }
 
 }  // namespace hipclaw

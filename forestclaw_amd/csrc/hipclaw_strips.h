@@ -28,60 +28,6 @@
 
 namespace hipclaw {
 
-// Limiter and second-order correction of one interface (clawpack46_inlinelimiter.f,
-// clawpack46_flux2.f:139-153).  dotl, dotr: the waves' products with those of
-// the interface before and after.  FP64 limits the waves and sums them in the
-// reference's order; FP32 puts the limiter into the sum's coefficients, and a
-// wave whose norm is below the smallest normal number has the limiter of a
-// slightly larger one (its terms are below 1e-19 either way).
-template <class RP, typename R, int IXY, bool STD>
-__device__ __forceinline__ void limited_correction(const StepArgs& a, const R wave[RP::MWAVES][RP::MEQN],
-                                                   const R s[RP::MWAVES], const R dotl[RP::MWAVES],
-                                                   const R dotr[RP::MWAVES], R dtd, R cqxx[RP::MEQN]) {
-#pragma clang fp contract(off)
-    constexpr int MEQN = RP::MEQN, MW = RP::MWAVES;
-    using WZ = wave_zeros<RP, IXY>;
-    R phi[MW];
-#pragma unroll
-    for (int mw = 0; mw < MW; mw++) {
-        phi[mw] = R(1);
-        const int mth = STD ? 4 : a.mthlim[mw];
-        if (mth == 0) continue;
-        R wn = R(0);
-        bool first = true;
-#pragma unroll
-        for (int m = 0; m < MEQN; m++)
-            if (!WZ::at(mw, m)) sum_term(wn, wave[mw][m], wave[mw][m], first);
-        const R d = pick(s[mw] > R(0), dotl[mw], dotr[mw]);
-        if constexpr (sizeof(R) == 4) {
-            const float r = d * __builtin_amdgcn_rcpf(rmax(wn, 1.17549435e-38f));
-            phi[mw] = STD ? rmax(0.0f, rmin(rmin(mad(0.5f, r, 0.5f), 2.0f), 2.0f * r)) : philim<float>(mth, r);
-        } else {
-            const R rr = dv(d, wn);
-            phi[mw] = pick(wave_nonzero(wn), philim<R, true>(mth, rr), R(1));
-        }
-    }
-    R c[MW];
-#pragma unroll
-    for (int mw = 0; mw < MW; mw++) {
-        const R as = fabs(s[mw]);
-        if constexpr (sizeof(R) == 4) c[mw] = mad(-(as * dtd), as, as) * phi[mw];
-        else c[mw] = as * (R(1) - as * dtd);
-    }
-#pragma unroll
-    for (int m = 0; m < MEQN; m++) {
-        R sum = R(0);
-        bool first = true;
-#pragma unroll
-        for (int mw = 0; mw < MW; mw++) {
-            if (WZ::at(mw, m)) continue;
-            if constexpr (sizeof(R) == 4) sum_term(sum, c[mw], wave[mw][m], first);
-            else sum_term(sum, c[mw], phi[mw] * wave[mw][m], first);
-        }
-        cqxx[m] = sum;
-    }
-}
-
 // Any value: what a skipped stage leaves behind is not read, and must not keep
 // the registers it stands in alive.
 template <typename V, int N>
@@ -106,9 +52,6 @@ __device__ __forceinline__ void reg_put(double* r, int stride, double el, const 
         for (int m = 0; m < N; m++) r[m * stride] = 0.0 + el * (double) v[m];
     }
 }
-
-// a b + c in one rounding: the FP32-bulk form's FP64 state update
-__device__ __forceinline__ double fmad64(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
 // x, computed where it stands: an address used in a rare branch of the row loop
 // must not be hoisted out of it into registers that live through every row.
@@ -399,7 +342,7 @@ step_strips(StepArgs a, StripShape sh) {
                         dotl[mw] = d;
                         dotr[mw] = next_lane(d);
                     }
-                    limited_correction<RP, R, 1, STD>(a, w, s, dotl, dotr, dtdx, cq);
+                    limited_correction<RP, R, 1, STD, true>(a, w, s, dotl, dotr, dtdx, cq);
                 }
 #pragma unroll
                 for (int m = 0; m < MEQN; m++) {
@@ -509,7 +452,7 @@ step_strips(StepArgs a, StripShape sh) {
                 R cq[MEQN];
 #pragma unroll
                 for (int m = 0; m < MEQN; m++) cq[m] = R(0);
-                if (STD || a.order2) limited_correction<RP, R, 2, STD>(a, wv[O], so, dlo, dl[P], dtdy, cq);
+                if (STD || a.order2) limited_correction<RP, R, 2, STD, true>(a, wv[O], so, dlo, dl[P], dtdy, cq);
 #pragma unroll
                 for (int m = 0; m < MEQN; m++) {
                     gm[m] = gt[m] + mad(R(0.5), cq[m], zadd(am[O][m]));
