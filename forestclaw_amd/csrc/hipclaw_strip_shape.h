@@ -74,16 +74,18 @@ inline bool strip_pattern(int mx, bool whole, StripShape& sh) {
 // the kernel's registers leave room for it).  Kernel times, us: shallow water
 // FP64, 700 patches of 32 x 32 (420 waves of columns), H = 4, 8, 16, 32: 71, 62,
 // 66, 110; 256 of 16 x 16 (86), H = 1, 2, 4, 8, 16: 23, 20, 25, 36, 59; Euler
-// FP32-bulk, 2800 of 16 x 16 (934), H = 4, 8, 16: 50, 42, 45.
+// FP32-bulk, 2800 of 16 x 16 (934), H = 4, 8, 16: 50, 42, 45.  The waves of a last
+// pattern with fewer patches are started all the same and count: 134 of 61 x 61, 153
+// waves of columns in 20 patterns of 8, are three rounds at H = 5 (2,080 waves, 63 us)
+// and one at H = 11 (49).
 inline void strip_rows(int my, int nwork, int simds, bool pairs, bool whole, StripShape& sh) {
-    const double cols = (double) nwork * sh.waves / sh.patches;
+    const long long cols = ((long long) nwork + sh.patches - 1) / sh.patches * sh.waves;
     double best = 0.0;
     sh.nsy = 1;
     for (int nsy = 1; nsy <= (whole ? 1 : my); nsy++) {
         const int H = (my + nsy - 1) / nsy;
         if ((my + H - 1) / H != nsy) continue;   // (the same H as fewer strips)
-        const double load = cols * nsy / simds;
-        const long long rounds = load > 1.0 ? (long long) (load + 0.999) : 1;
+        const long long rounds = (cols * nsy + simds - 1) / simds;
         const double cost = (double) rounds * (H + 3) * (pairs && rounds == 1 ? 1.2 : 1.0);
         if (nsy == 1 || cost < best) { best = cost; sh.nsy = nsy; }
     }
