@@ -116,7 +116,8 @@ inline int launch_step_shape(const StepArgs& a, const StepLaunch& st) {
 inline bool launches_tiles(const StepArgs& a, int tile, int wave_bytes, int simds) {
     const bool inplace = a.qsrc == a.qdst;
     if (inplace && a.ntx * a.nty != 1) return false;
-    return tiles_pay(wave_bytes, tile, a.mx, a.my, a.nwork, a.ntx * a.nty, simds, a.reg != nullptr, inplace);
+    return tiles_pay(wave_bytes, tile, a.mx, a.my, a.nwork, a.ntx * a.nty, simds,
+                     !a.reg ? TILES_PLAIN : a.reg_accumulate ? TILES_ACCUMULATE : TILES_REGISTERS, inplace);
 }
 
 inline int device_simds() {
@@ -184,7 +185,7 @@ inline int launch_step_strips(int nw, const StepArgs& a, const StepLaunch& st) {
 // and one and wait at the barrier; FP64 tiles need the latency hiding of four).
 // hipclaw_set_waves and the autotuner choose 2, 3 or 4.
 constexpr int STRIP_WAVES = 4;
-inline int default_waves(bool strips, bool fp64, int tile) {
+constexpr int default_waves(bool strips, bool fp64, int tile) {
     return tile != 16 ? 0 : strips ? STRIP_WAVES : fp64 ? 4 : 2;   // (0: one choice)
 }
 
@@ -199,15 +200,22 @@ constexpr bool has_tile(int tile, bool regs) {
                               (regs ? step_fits<RP, R, 32, FF, true>() : step_fits<RP, R, 32, FF, false>());
 }
 
+// The small launches of a solver that uses strips have one shape per tile and
+// precision: the choice of 2, 3 or 4 waves is the strips' (and each further kernel
+// makes the code larger that every launch is fetched from: with all of them a call of
+// two small kernels took 0.5 to 1 us more).
 template <class RP, typename R, bool WITH_REGS, bool WITH32>
 inline int launch_step_tiles(int tile, int waves, const StepArgs& a, const StepLaunch& st) {
     if (waves == 0) waves = default_waves(false, sizeof(R) == 8, tile);
     switch (tile) {
     case 8: return launch_step_shape<RP, R, 8, 2, WITH_REGS>(a, st);
     case 16:
-        return waves == 2 ? launch_step_shape<RP, R, 16, 2, WITH_REGS>(a, st)
-             : waves == 3 ? launch_step_shape<RP, R, 16, 3, WITH_REGS>(a, st)
-                          : launch_step_shape<RP, R, 16, 4, WITH_REGS>(a, st);
+        if constexpr (uses_strips<RP>())
+            return launch_step_shape<RP, R, 16, default_waves(false, sizeof(R) == 8, 16), WITH_REGS>(a, st);
+        else
+            return waves == 2 ? launch_step_shape<RP, R, 16, 2, WITH_REGS>(a, st)
+                 : waves == 3 ? launch_step_shape<RP, R, 16, 3, WITH_REGS>(a, st)
+                              : launch_step_shape<RP, R, 16, 4, WITH_REGS>(a, st);
     case 32:
         if constexpr (WITH32) return launch_step_shape<RP, R, 32, 16, WITH_REGS>(a, st);
         return (int) hipErrorInvalidValue;
@@ -215,11 +223,12 @@ inline int launch_step_tiles(int tile, int waves, const StepArgs& a, const StepL
     }
 }
 
-// waves = 0: the default; 2, 3 or 4 select the variant.
+// waves = 0: the default; 2, 3 or 4 select the variant (of the strips, which then take
+// small launches too, unless in place).
 template <class RP, typename R, bool WITH_REGS, bool WITH32 = false>
 inline int launch_step_tile(int tile, int waves, const StepArgs& a, const StepLaunch& st) {
     if constexpr (uses_strips<RP>()) {
-        if (!has_tile<RP, R, WITH_REGS, WITH32>(tile, a.reg != nullptr) ||
+        if ((waves > 0 && a.qsrc != a.qdst) || !has_tile<RP, R, WITH_REGS, WITH32>(tile, a.reg != nullptr) ||
             !launches_tiles(a, tile, RP::MEQN * RP::MWAVES * (int) sizeof(R), device_simds()))
             return launch_step_strips<RP, R, WITH_REGS>(waves > 0 ? waves : STRIP_WAVES, a, st);
     }

@@ -56,7 +56,6 @@ struct StepArgs {
     unsigned long long* cfl;
     long long pstride;         // doubles per patch in q
     long long astride;         // doubles per patch in aux
-    int clock;
     int nwork;
     int mx, my, mbc;
     int ntx, nty;              // tiles per patch in x and y
@@ -74,6 +73,7 @@ struct StepArgs {
     double* reg;
     long long rstride;
     int reg_accumulate;   // add to the registers (subcycling) instead of overwriting them
+    int clock;
     const double* dtscale;  // per-slot factor on dt (an ensemble of runs), or null
     // Deferred conservation fix-up (null: none pending).  qcorr[slot][face][m][pos]
     // holds the time-sync increment of interior edge cell pos of `face` for the

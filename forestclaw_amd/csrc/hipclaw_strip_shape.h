@@ -106,6 +106,10 @@ inline void strip_rows(int my, int nwork, int simds, bool pairs, bool whole, Str
 // and with time-sync registers, which the tiles store at the end of a tile,
 //   T = 8   shallow water FP64 24 x 24, strips 1.24 times as long with 88 patches and
 //           0.8 with 333; FP32-bulk 1.07 with 28, 0.91 with 44
+// and where these add up over substeps, which the strips leave to the L2 (one level's
+// copy, step, ghost fill and synchronisation),
+//   T = 8   shallow water FP64 12 x 12, 100 patches 23.7 / 25.6, 256 27.7 / 26.5
+//   T = 16  16 x 16, 256 patches 28.1 / 30.8, 288 32.7 / 31.4
 // Tiles that overlap (a patch the tile does not divide) compute cells twice, and
 // count as much more.
 // In place a patch is one strip of all its rows, a serial chain: tiles until the
@@ -115,7 +119,8 @@ inline void strip_rows(int my, int nwork, int simds, bool pairs, bool whole, Str
 // 3000 76 / 64; 32 x 32 (T = 32) 28.5 / 96, 700 80 / 101; advection FP64 8 x 8, 1000
 // 6.9 / 9.4, 2000 9.9 / 9.7.
 // wave_bytes: of one interface's waves (meqn x mwaves values).
-inline bool tiles_pay(int wave_bytes, int tile, int mx, int my, int nwork, int tiles_per_patch, int simds, bool regs,
+enum { TILES_PLAIN = 0, TILES_REGISTERS = 1, TILES_ACCUMULATE = 2 };
+inline bool tiles_pay(int wave_bytes, int tile, int mx, int my, int nwork, int tiles_per_patch, int simds, int regs,
                       bool inplace) {
     const long long cus = simds / 4;
     if (inplace) {
@@ -125,8 +130,8 @@ inline bool tiles_pay(int wave_bytes, int tile, int mx, int my, int nwork, int t
     }
     const bool heavy = wave_bytes >= 72;
     double most;                 // tiles per CU
-    if (tile == 8) most = regs ? (heavy ? 4 : 1) : heavy ? 8 : wave_bytes < 9 ? 1 : wave_bytes / 9.0;
-    else most = tile == 16 && heavy ? 2 : 0;
+    if (tile == 8) most = regs ? (!heavy ? 1 : regs == TILES_ACCUMULATE ? 2 : 4) : heavy ? 8 : wave_bytes < 9 ? 1 : wave_bytes / 9.0;
+    else most = tile == 16 && heavy ? (regs == TILES_ACCUMULATE ? 1 : 2) : 0;
     const double ntiles = (double) nwork * tiles_per_patch, twice = (double) tiles_per_patch * tile * tile / ((double) mx * my);
     return ntiles * twice <= most * cus;
 }

@@ -17,7 +17,7 @@ int main() {
     for (int tile = 8; tile <= 32; tile *= 2)
         for (int w = 0; w < 6; w++)
             for (int mx = tile; mx <= 200; mx += 7)
-                for (int regs = 0; regs < 2; regs++)
+                for (int regs = 0; regs < 3; regs++)
                     for (int here = 0; here < (mx == tile ? 2 : 1); here++) {
                         const int across = (mx + tile - 1) / tile;
                         std::printf("[%d, %d, %d, %d, %d, %d, [", tile, waves[w], mx, regs, here, across * across);
@@ -52,20 +52,20 @@ def test_in_place_steps_of_few_patches_take_tiles(routes):
         if here:
             seen += 1
             assert all(tiles[:9])            # up to 256 patches, a quarter of the SIMDs
-    assert seen == 36
+    assert seen == 54
 
 
 def test_small_launches_take_tiles(routes):
     """8 x 8 tiles: one per CU for any solver, four for shallow water FP32-bulk, eight
-    for FP64 (four with time-sync registers); 16 x 16 tiles two per CU, only where an
-    interface has 72 bytes of waves; 32 x 32 tiles in place only.  Tiles that overlap
-    count by the cells they compute."""
+    for FP64 (four with time-sync registers, two where they add up); 16 x 16 tiles two
+    per CU (one), only where an interface has 72 bytes of waves; 32 x 32 tiles in
+    place only.  Tiles that overlap count by the cells they compute."""
     cus = SIMDS // 4
     for tile, wave_bytes, mx, regs, here, per, tiles in routes:
         if here:
             continue
         heavy = wave_bytes >= 72
-        limit = {8: ((4 if heavy else 1) if regs else 8 if heavy else max(1, wave_bytes / 9)) * cus,
-                 16: 2 * cus if heavy else 0, 32: 0}[tile]
+        limit = {8: (((8, 4, 2) if heavy else (max(1, wave_bytes / 9), 1, 1))[regs]) * cus,
+                 16: (2, 2, 1)[regs] * cus if heavy else 0, 32: 0}[tile]
         load = per * per * tile * tile / (mx * mx)
         assert [bool(t) for t in tiles] == [2 ** k * load <= limit for k in range(len(tiles))], (tile, wave_bytes, mx, regs)
