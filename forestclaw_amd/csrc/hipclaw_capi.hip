@@ -12,9 +12,7 @@
 #include <cstdio>
 #include <cstring>
 #include <cmath>
-#include <memory>
 #include <mutex>
-#include <new>
 #include <unordered_map>
 #include <vector>
 
@@ -197,12 +195,15 @@ struct hipclaw_state {
 };
 
 // ---------------------------------------------------------------- allocation-free step
-// Device scratch of hipclaw_step_batch_noalloc: the CFL word, then the staged
+// Device scratch of hipclaw_step_batch_noalloc: the CFL words, then the staged
 // slot list.  Every GPU holds its own copy of this array for the life of the
 // process; its device address is looked up once per device (scratch_ptr) and
 // only that address is passed to kernels, copies and fills.
 namespace {
 constexpr size_t NOALLOC_CFL_BYTES = CFL_BYTES;
+// So many slots go up in one copy with the cleared words, from the stack (16 KiB of
+// it); a longer list goes up as it is and a launch clears the words.
+constexpr int NOALLOC_STACK_SLOTS = 3072;
 constexpr size_t NOALLOC_SCRATCH_BYTES =
     NOALLOC_CFL_BYTES + sizeof(int) * (size_t) HIPCLAW_NOALLOC_MAX_SLOTS;
 constexpr int NOALLOC_MAX_DEVICES = 64;
@@ -1861,13 +1862,21 @@ int hipclaw_step_batch_noalloc(const hipclaw_config_t* cfg, int npatch, const do
     unsigned long long* dcfl = reinterpret_cast<unsigned long long*>(base);
     int* dslots = reinterpret_cast<int*>(base + NOALLOC_CFL_BYTES);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    // the cleared CFL words and the slot list behind them in one copy
-    const size_t nupload = NOALLOC_CFL_BYTES + sizeof(int) * (size_t) nslots;
-    std::unique_ptr<unsigned char[]> upload(new (std::nothrow) unsigned char[nupload]);
-    if (!upload) return fail(HIPCLAW_ENOMEM, "hipclaw_step_batch_noalloc: host allocation failed%s");
-    std::memset(upload.get(), 0, NOALLOC_CFL_BYTES);
-    std::memcpy(upload.get() + NOALLOC_CFL_BYTES, slots, sizeof(int) * (size_t) nslots);
-    HIP_TRY(hipMemcpyAsync(base, upload.get(), nupload, hipMemcpyHostToDevice, st));
+    // (whole 64 bytes: the odd tail of a copy goes up by itself, 3 us)
+    struct { unsigned long long words[hipclaw::CFL_BLOCK]; int slots[NOALLOC_STACK_SLOTS]; } up;
+    auto done = [&](int result) { (void) hipStreamSynchronize(st); return result; };   // (the copies may still read)
+    hipError_t e;
+    if (nslots <= NOALLOC_STACK_SLOTS) {
+        const int padded = (nslots + 15) / 16 * 16;
+        std::memset(up.words, 0, sizeof(up.words));
+        std::memcpy(up.slots, slots, sizeof(int) * (size_t) nslots);
+        std::memset(up.slots + nslots, 0, sizeof(int) * (size_t) (padded - nslots));
+        e = hipMemcpyAsync(base, &up, NOALLOC_CFL_BYTES + sizeof(int) * (size_t) padded, hipMemcpyHostToDevice, st);
+    } else {
+        e = hipMemcpyAsync(dslots, slots, sizeof(int) * (size_t) nslots, hipMemcpyHostToDevice, st);
+        if (e == hipSuccess) e = (hipError_t) hipclaw::launch_reset_cfl(dcfl, 1, nullptr, st);
+    }
+    if (e != hipSuccess) return done(hipfail(e, "hipclaw_step_batch_noalloc upload"));
     hipclaw::StepArgs a;
     a.qsrc = q_in;
     a.qdst = q_out;
@@ -1890,15 +1899,13 @@ int hipclaw_step_batch_noalloc(const hipclaw_config_t* cfg, int npatch, const do
     a.reg_accumulate = 0;
     a.dtscale = nullptr;
     const hipclaw::StepLaunch L(st);
-    if (int e = launch_solver_step(cfg->solver, cfg->precision, tile, 0, a, L)) {
-        (void) hipStreamSynchronize(st);   // (the copy may still read `upload`)
-        return hipfail((hipError_t) e, "step launch");
-    }
-    unsigned long long words[CFL_BYTES / sizeof(unsigned long long)];
-    HIP_TRY(hipMemcpyAsync(words, dcfl, CFL_BYTES, hipMemcpyDeviceToHost, st));
+    e = (hipError_t) launch_solver_step(cfg->solver, cfg->precision, tile, 0, a, L);
+    if (e != hipSuccess) return done(hipfail(e, "step launch"));
+    e = hipMemcpyAsync(up.words, dcfl, CFL_BYTES, hipMemcpyDeviceToHost, st);
+    if (e != hipSuccess) return done(hipfail(e, "hipMemcpyAsync"));
     HIP_TRY(hipStreamSynchronize(st));
     unsigned long long bits = 0;
-    for (int k = 0; k < hipclaw::CFL_WORDS; k++) bits = std::max(bits, words[k * hipclaw::CFL_STRIDE]);
+    for (int k = 0; k < hipclaw::CFL_WORDS; k++) bits = std::max(bits, up.words[k * hipclaw::CFL_STRIDE]);
     if (maxcfl) *maxcfl = as_double(bits);
     return HIPCLAW_OK;
 }

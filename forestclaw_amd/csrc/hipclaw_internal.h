@@ -125,7 +125,7 @@ int launch_apply_qcorr(double* q, const double* qcorr, const int* cmask, const i
                        hipStream_t st);
 int launch_step_fp64(int solver, int tile, int waves, const StepArgs& a, const StepLaunch& st);
 int launch_step_fp32(int solver, int tile, int waves, const StepArgs& a, const StepLaunch& st);
-// `blocks` blocks of CFL and clock words (StepArgs::cfl) and the sums to zero.
+// `blocks` blocks of CFL and clock words (StepArgs::cfl) and the sums (or null) to zero.
 int launch_reset_cfl(unsigned long long* p, int blocks, unsigned long long* sum, hipStream_t st);
 // What an advance's steps left in the first `blocks` blocks (at most
 // STEP_BLOCKS) added to sum, and the blocks cleared.  With out (host memory),

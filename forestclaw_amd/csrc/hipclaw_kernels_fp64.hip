@@ -683,7 +683,7 @@ int launch_apply_qcorr(double* q, const double* qcorr, const int* cmask, const i
 __global__ void reset_cfl(unsigned long long* p, unsigned long long* sum) {
     unsigned long long* w = p + (long long) blockIdx.x * CFL_BLOCK + threadIdx.x * CFL_STRIDE;
     w[0] = w[1] = w[2] = 0ull;
-    if (blockIdx.x == 0 && threadIdx.x < STEP_SUMS) sum[threadIdx.x] = 0ull;
+    if (sum && blockIdx.x == 0 && threadIdx.x < STEP_SUMS) sum[threadIdx.x] = 0ull;
 }
 
 // The end of an advance, in one launch: its Courant number and the steps'

@@ -146,7 +146,8 @@ int hipclaw_step_batch(hipclaw_state_t *s, const int *slots, int nslots, double 
 #define HIPCLAW_NOALLOC_MAX_SLOTS 65536
 
 /* The batched update of hipclaw_step_batch on caller-owned device memory,
- * allocating nothing: no hipMalloc, hipFree or allocating library call, so
+ * allocating nothing: no hipMalloc, hipFree or allocating library call, no host
+ * allocation (some 16 KiB of the caller's stack), so
  * callers that cannot allocate (code under graph capture, tight serving loops,
  * harnesses that forbid it) can drive it.  No counterpart in the reference.
  *   q_in, q_out : device, npatch slabs in the layout above; the interior cells
@@ -159,8 +160,8 @@ int hipclaw_step_batch(hipclaw_state_t *s, const int *slots, int nslots, double 
  *   stream      : the hipStream_t to run on (NULL: the default stream); the
  *                 call returns after the stream has finished its work.
  *   maxcfl      : the largest Courant number of the batch (may be NULL).
- * The slot list and the CFL word are staged in one fixed device scratch array
- * of the library (about 256 KiB per GPU, held until the process ends), cleared
+ * The slot list and the CFL words are staged in one fixed device scratch array
+ * of the library (260 KiB per GPU, held until the process ends), cleared
  * by every call: calls that overlap on one GPU race on it.  No time-sync
  * registers and no per-slot dt scale.  Make the device current first (the
  * scratch address is looked up once per device, at hipclaw_initialize_device
