@@ -455,7 +455,7 @@ class Solver:
         _check(lib().hipclaw_restore_step(self._h), "hipclaw_restore_step")
 
     def autotune(self, dt, nsteps=8):
-        """Time every allowed tile (16 x 16 with 2 and 4 waves) in every
+        """Time every allowed tile (16 x 16 with 2, 3 and 4 waves) in every
         ghost-fill layout over nsteps steps of dt (the state is put back
         after each) and keep the fastest; returns
         {(tile, waves, layout): ms per step}."""
@@ -476,7 +476,7 @@ class Solver:
         return lib().hipclaw_waves(self._h)
 
     def set_waves(self, waves):
-        """Waves per workgroup of 16 x 16 tiles: 2, 4 or 0 (the default)."""
+        """Waves per workgroup of the update: 2, 3, 4 or 0 (the default)."""
         _check(lib().hipclaw_set_waves(self._h, waves), "hipclaw_set_waves")
 
     @property

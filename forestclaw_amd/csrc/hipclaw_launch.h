@@ -133,11 +133,10 @@ inline int device_simds() {
     return n;
 }
 
-// pairs: two waves of the kernel fit a SIMD.  lds: its bytes per wave (one wave per
-// workgroup then).  nw: waves per workgroup.
+// pairs: two waves of the kernel fit a SIMD.  lds: its bytes per wave.  nw: waves per
+// workgroup.
 template <typename K>
 inline int launch_strips(K kernel, bool pairs, int lds, int nw, const StepArgs& a, const StepLaunch& L) {
-    if (lds > 0) nw = 1;
     if (a.nwork <= 0) return 0;
     const bool inplace = a.qsrc == a.qdst;
     const int simds = device_simds();
@@ -148,9 +147,9 @@ inline int launch_strips(K kernel, bool pairs, int lds, int nw, const StepArgs& 
     const long long blocks = ((waves + nw - 1) / nw + 7) / 8 * 8;   // a multiple of the 8 XCDs
     if (waves * 64 > 0x7fffffffLL) return (int) hipErrorInvalidConfiguration;
     if (L.start || L.stop)
-        hipExtLaunchKernelGGL(kernel, dim3((unsigned) blocks), dim3(64 * nw), lds, L.st, L.start, L.stop, 0, a, sh);
+        hipExtLaunchKernelGGL(kernel, dim3((unsigned) blocks), dim3(64 * nw), lds * nw, L.st, L.start, L.stop, 0, a, sh);
     else
-        hipLaunchKernelGGL(kernel, dim3((unsigned) blocks), dim3(64 * nw), lds, L.st, a, sh);
+        hipLaunchKernelGGL(kernel, dim3((unsigned) blocks), dim3(64 * nw), lds * nw, L.st, a, sh);
     return (int) hipGetLastError();
 }
 
@@ -179,15 +178,16 @@ inline int launch_step_strips(int nw, const StepArgs& a, const StepLaunch& st) {
 // Waves per workgroup by default.  Strips: four, which share nothing but lie on the
 // four SIMDs of one CU, beside each other in its cache (one and four, subcycled dam
 // break FP64 9.80 and 9.62 ms, dam break FP64 22.53 and 22.46, shock-bubble FP32
-// 5.20 and 5.16, advection 567 and 565 us; three leave a SIMD of every CU idle).
+// 5.20 and 5.16, advection 567 and 565 us; three leave a SIMD of every CU idle); one
+// for the kernels that keep values in LDS, which a workgroup holds until its last wave
+// ends.
 // 16 x 16 tiles: four for FP64, two for the FP32-bulk form (a sweep's 18 rows, three
 // per wave, are three groups for each of two waves, where four take two, two, one
 // and one and wait at the barrier; FP64 tiles need the latency hiding of four).
 // hipclaw_set_waves and the autotuner choose 2, 3 or 4.
-constexpr int STRIP_WAVES = 4;
-constexpr int default_waves(bool strips, bool fp64, int tile) {
-    return tile != 16 ? 0 : strips ? STRIP_WAVES : fp64 ? 4 : 2;   // (0: one choice)
-}
+template <class RP, typename R>
+constexpr int strip_waves() { return strip_carry<RP, R>() ? 1 : 4; }
+constexpr int default_tile_waves(bool fp64, int tile) { return tile != 16 ? 0 : fp64 ? 4 : 2; }   // (0: one choice)
 
 // Whether the tile kernel is instantiated for a tile (T = 32 only WITH32).
 template <class RP, typename R, bool WITH_REGS, bool WITH32>
@@ -206,12 +206,12 @@ constexpr bool has_tile(int tile, bool regs) {
 // two small kernels took 0.5 to 1 us more).
 template <class RP, typename R, bool WITH_REGS, bool WITH32>
 inline int launch_step_tiles(int tile, int waves, const StepArgs& a, const StepLaunch& st) {
-    if (waves == 0) waves = default_waves(false, sizeof(R) == 8, tile);
+    if (waves == 0) waves = default_tile_waves(sizeof(R) == 8, tile);
     switch (tile) {
     case 8: return launch_step_shape<RP, R, 8, 2, WITH_REGS>(a, st);
     case 16:
         if constexpr (uses_strips<RP>())
-            return launch_step_shape<RP, R, 16, default_waves(false, sizeof(R) == 8, 16), WITH_REGS>(a, st);
+            return launch_step_shape<RP, R, 16, default_tile_waves(sizeof(R) == 8, 16), WITH_REGS>(a, st);
         else
             return waves == 2 ? launch_step_shape<RP, R, 16, 2, WITH_REGS>(a, st)
                  : waves == 3 ? launch_step_shape<RP, R, 16, 3, WITH_REGS>(a, st)
@@ -230,7 +230,7 @@ inline int launch_step_tile(int tile, int waves, const StepArgs& a, const StepLa
     if constexpr (uses_strips<RP>()) {
         if ((waves > 0 && a.qsrc != a.qdst) || !has_tile<RP, R, WITH_REGS, WITH32>(tile, a.reg != nullptr) ||
             !launches_tiles(a, tile, RP::MEQN * RP::MWAVES * (int) sizeof(R), device_simds()))
-            return launch_step_strips<RP, R, WITH_REGS>(waves > 0 ? waves : STRIP_WAVES, a, st);
+            return launch_step_strips<RP, R, WITH_REGS>(waves > 0 ? waves : strip_waves<RP, R>(), a, st);
     }
     return launch_step_tiles<RP, R, WITH_REGS, WITH32>(tile, waves, a, st);
 }
