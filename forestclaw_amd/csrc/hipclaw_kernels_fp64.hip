@@ -857,27 +857,30 @@ regrid_remap(const double* __restrict__ qold, double* __restrict__ qnew,
     }
 }
 
-// One workgroup per patch, then four zeroed registers (slot, face) per workgroup:
-// both only move memory, and a launch of its own for either lasts 5 us at least
-// (a subcycled dam break's 1,480 fine patches of 16 x 16: copy 9.6 and reset 8.0 us
-// apart, 10.8 us together).
+// A workgroup per COPY_CHUNK values of a patch, then four zeroed registers (slot, face)
+// per workgroup: both only move memory, and a launch of its own for either lasts 5 us
+// at least (a subcycled dam break's 1,480 fine patches of 16 x 16: copy 9.6 and reset
+// 8.0 us apart, 10.8 us together).  Not one workgroup per patch, which copies a large
+// one alone (hipclaw_step_batch of a subcycling state, one patch of 256 x 256: 143 us,
+// 37 in chunks; 64 x 64 42 and 36, 16 x 16, which is one chunk, 31).
+constexpr int COPY_CHUNK = 1024;
 template <typename V>
 __global__ void __launch_bounds__(256)
-copy_patches(const V* __restrict__ src, V* __restrict__ dst, const int* __restrict__ slots, int n, int pstride,
+copy_patches(const V* __restrict__ src, V* __restrict__ dst, const int* __restrict__ slots, int n, int chunks, int pstride,
              double* __restrict__ reg, const int* __restrict__ resets, int nresets, long long rstride, int per_face) {
-    if ((int) blockIdx.x < n) {
-        const long long base = (long long) slots[blockIdx.x] * pstride;
-        for (int e = threadIdx.x; e < pstride; e += 1024) {
-            V v[4];
+    const int b = blockIdx.x;
+    if (b < n * chunks) {
+        const int w = b / chunks, e0 = (b - w * chunks) * COPY_CHUNK + threadIdx.x;
+        const long long base = (long long) slots[w] * pstride;
+        V v[COPY_CHUNK / 256];
 #pragma unroll
-            for (int u = 0; u < 4; u++) v[u] = src[base + min(e + 256 * u, pstride - 1)];
+        for (int u = 0; u < COPY_CHUNK / 256; u++) v[u] = src[base + min(e0 + 256 * u, pstride - 1)];
 #pragma unroll
-            for (int u = 0; u < 4; u++)
-                if (e + 256 * u < pstride) dst[base + e + 256 * u] = v[u];
-        }
+        for (int u = 0; u < COPY_CHUNK / 256; u++)
+            if (e0 + 256 * u < pstride) dst[base + e0 + 256 * u] = v[u];
         return;
     }
-    const int r = ((int) blockIdx.x - n) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = (b - n * chunks) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (r >= nresets) return;
     double* p = reg + (long long) resets[2 * r] * rstride + (long long) resets[2 * r + 1] * per_face;
     for (int e = threadIdx.x & 63; e < per_face; e += 64) p[e] = 0.0;
@@ -1029,14 +1032,17 @@ int launch_ghost_physbc(const GhostArgs& g, hipStream_t st) {
 
 int launch_copy_patches(const double* src, double* dst, const int* slots, int n, long long pstride, const Resets& z,
                         hipStream_t st) {
-    const int blocks = n + (z.n + 3) / 4;
+    const bool pairs = pstride % 2 == 0;
+    const int values = (int) (pairs ? pstride / 2 : pstride), chunks = (values + COPY_CHUNK - 1) / COPY_CHUNK;
+    const long long blocks = (long long) n * chunks + (z.n + 3) / 4;
     if (blocks <= 0) return 0;
-    if (pstride % 2 == 0)
-        hipLaunchKernelGGL(copy_patches<double2>, dim3(blocks), dim3(256), 0, st, (const double2*) src, (double2*) dst,
-                           slots, n, (int) (pstride / 2), z.reg, z.list, z.n, z.rstride, z.per_face);
+    if (blocks > 0x7fffffffLL) return (int) hipErrorInvalidConfiguration;
+    if (pairs)
+        hipLaunchKernelGGL(copy_patches<double2>, dim3((unsigned) blocks), dim3(256), 0, st, (const double2*) src,
+                           (double2*) dst, slots, n, chunks, values, z.reg, z.list, z.n, z.rstride, z.per_face);
     else
-        hipLaunchKernelGGL(copy_patches<double>, dim3(blocks), dim3(256), 0, st, src, dst, slots, n, (int) pstride, z.reg,
-                           z.list, z.n, z.rstride, z.per_face);
+        hipLaunchKernelGGL(copy_patches<double>, dim3((unsigned) blocks), dim3(256), 0, st, src, dst, slots, n, chunks,
+                           values, z.reg, z.list, z.n, z.rstride, z.per_face);
     return (int) hipGetLastError();
 }
 
