@@ -331,12 +331,44 @@ static int upload_array(hipclaw_state_t* s, T*& dev, int& cap, const T* host, in
     return HIPCLAW_OK;
 }
 
+// A captured graph holds its launches' arguments: op counts, table and
+// buffer addresses, patch counts.  Whatever changes those drops the graph
+// (replaying it is then an error until the next capture).
+static void drop_graph(hipclaw_state_t* s) {
+    if (s->gexec) { hipGraphExecDestroy(s->gexec); s->gexec = nullptr; }
+    if (s->graph) { hipGraphDestroy(s->graph); s->graph = nullptr; }
+    s->graph_steps = 0;
+}
+
+// Gives the second slab of a state whose tile covers a patch back, so that its memory
+// can serve an allocation that failed; the state steps in place from then on.  Not
+// while the other slab holds the saved state.
+static bool give_back_slab(hipclaw_state_t* s) {
+    if (!s->covers || !s->q[1] || (s->save_lazy && s->save_slab != s->cur)) return false;
+    if (hipStreamSynchronize(s->st) != hipSuccess) return false;
+    drop_graph(s);
+    hipFree(s->q[1 - s->cur]);
+    s->q[0] = s->q[s->cur];
+    s->q[1] = nullptr;
+    s->cur = s->save_slab = 0;
+    s->inplace = true;
+    return true;
+}
+
 // Copy slab `from` into qsave (allocated on first use).
 static int copy_to_save(hipclaw_state_t* s, int from) {
     const size_t bytes = sizeof(double) * (size_t) s->pstride * (size_t) s->npatch;
     if (!s->qsave) {
-        if (hipMalloc((void**) &s->qsave, sizeof(double) * (size_t) s->pstride * (size_t) s->max_patches) != hipSuccess)
+        const size_t room = sizeof(double) * (size_t) s->pstride * (size_t) s->max_patches;
+        hipError_t e = hipMalloc((void**) &s->qsave, room);
+        if (e != hipSuccess && from == s->cur && give_back_slab(s)) {
+            from = s->cur;
+            e = hipMalloc((void**) &s->qsave, room);
+        }
+        if (e != hipSuccess) {
+            s->qsave = nullptr;
             return fail(HIPCLAW_ENOMEM, "hipMalloc of the saved state failed%s");
+        }
     }
     if (bytes > 0) HIP_TRY(hipMemcpyAsync(s->qsave, s->q[from], bytes, hipMemcpyDeviceToDevice, s->st));
     return HIPCLAW_OK;
@@ -348,18 +380,9 @@ static int copy_to_save(hipclaw_state_t* s, int from) {
 // fix-up), so it leaves the saved state in place.
 static int guard_save(hipclaw_state_t* s, bool one_step_advance = false) {
     if (!s->save_lazy) return HIPCLAW_OK;
-    if (one_step_advance && s->cur == s->save_slab) return HIPCLAW_OK;
+    if (one_step_advance && !s->inplace && s->cur == s->save_slab) return HIPCLAW_OK;
     s->save_lazy = false;
     return copy_to_save(s, s->save_slab);
-}
-
-// A captured graph holds its launches' arguments: op counts, table and
-// buffer addresses, patch counts.  Whatever changes those drops the graph
-// (replaying it is then an error until the next capture).
-static void drop_graph(hipclaw_state_t* s) {
-    if (s->gexec) { hipGraphExecDestroy(s->gexec); s->gexec = nullptr; }
-    if (s->graph) { hipGraphDestroy(s->graph); s->graph = nullptr; }
-    s->graph_steps = 0;
 }
 
 extern "C" {
@@ -2285,6 +2308,7 @@ int hipclaw_replay_graph(hipclaw_state_t* s) {
         return fail(HIPCLAW_EINVAL, "the captured graph starts from the other slab (an odd number of "
                                     "steps or a restored step since the capture)%s");
     if (int rc = guard_save(s)) return rc;
+    if (!s->gexec) return fail(HIPCLAW_ENOMEM, "no memory for the saved state beside the captured graph%s");
     if (s->cur != s->graph_cur) {   // (any number of steps where a tile covers a patch)
         if (int e = hipclaw::launch_copy_patches(s->q[s->cur], s->q[s->graph_cur], s->all_slots, s->npatch,
                                                  s->pstride, hipclaw::Resets{}, s->st))
@@ -2440,7 +2464,9 @@ int hipclaw_regrid(hipclaw_state_t* s, int npatch_new, const int* kind, const in
         for (int g = 0; g < 4; g++) op[2 + g] = sp[g];
     }
     // destination slab: the spare ping-pong slab when the new patches fit,
-    // otherwise a larger allocation (with room to grow) replacing both slabs
+    // otherwise a larger allocation (with room to grow) replacing both slabs; the
+    // second slab of a state whose tile covers a patch goes first, so that the old
+    // and the new state need no more memory than with one slab
     const bool reuse = !s->inplace && npatch_new <= s->max_patches;
     const int cap = reuse ? s->max_patches
                           : std::max(npatch_new, std::max(s->max_patches, npatch_new + npatch_new / 4));
@@ -2448,6 +2474,7 @@ int hipclaw_regrid(hipclaw_state_t* s, int npatch_new, const int* kind, const in
     if (int rc = ensure_iwork(s, ops.size())) return rc;
     int* dops = s->iwork;
     HIP_TRY(hipStreamSynchronize(s->st));
+    if (!reuse) give_back_slab(s);
     if (reuse) qnew = s->q[1 - s->cur];
     else if (hipMalloc((void**) &qnew, sizeof(double) * s->pstride * (size_t) cap) != hipSuccess)
         return fail(HIPCLAW_ENOMEM, "hipclaw_regrid: device allocation failed%s");
@@ -2469,17 +2496,10 @@ int hipclaw_regrid(hipclaw_state_t* s, int npatch_new, const int* kind, const in
         s->q[0] = qnew;
         s->q[1] = nullptr;
         s->cur = 0;
-        if (s->covers) {
-            const int old = s->max_patches;
-            s->max_patches = cap;
-            second_slab(s);
-            s->max_patches = old;
-        } else if (hipMalloc((void**) &s->q[1], sizeof(double) * s->pstride * (size_t) cap) != hipSuccess) {
+        s->inplace = s->covers;
+        if (!s->covers && hipMalloc((void**) &s->q[1], sizeof(double) * s->pstride * (size_t) cap) != hipSuccess) {
             s->q[1] = nullptr;
             return fail(HIPCLAW_ENOMEM, "hipclaw_regrid: device allocation failed%s");
-        }
-        if (s->q[1]) {
-            HIP_TRY(hipMemset(s->q[1], 0, sizeof(double) * s->pstride * (size_t) cap));
         }
     }
     // a saved state names old slots (and is sized for the old capacity)
@@ -2491,6 +2511,10 @@ int hipclaw_regrid(hipclaw_state_t* s, int npatch_new, const int* kind, const in
         if (int rc = grow_patch_buffers(s, cap)) return rc;
     } else if (s->reg) {
         HIP_TRY(hipMemset(s->reg, 0, sizeof(double) * s->rstride * (size_t) s->max_patches));
+    }
+    if (!reuse) {   // the second slab from what the grown buffers leave
+        if (s->covers) second_slab(s);
+        if (s->q[1]) HIP_TRY(hipMemset(s->q[1], 0, sizeof(double) * s->pstride * (size_t) s->max_patches));
     }
     // every program and the dt scale name old slots; the graph names old buffers
     hipFree(s->dtscale);

@@ -92,6 +92,11 @@ int hipclaw_initialize_device(int device, char *name, size_t name_len);
 
 /* Create a solver state with room for max_patches patches.  One allocation per
  * slab (q, its ping-pong partner, aux, geometry); no per-patch allocation.
+ * Where one tile covers a patch the partner is not needed, and is taken only if
+ * as much memory again stays free (not by a subcycling state); a program that
+ * needs that memory for something else allocates it before.  hipclaw_regrid and
+ * a kept state that has to be copied give the partner back if their own
+ * allocation needs the room; the state then steps in place, with the same bits.
  * Replaces fc2d_cudaclaw_allocate_buffers and the per-patch
  * cudaclaw_allocate_fluxes pool
  * (src/solvers/fc2d_cudaclaw/cuda_source/cudaclaw_allocate.cu:21-132) and
