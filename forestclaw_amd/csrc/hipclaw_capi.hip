@@ -467,19 +467,6 @@ static bool solver_tile_ok(int solver, int precision, int tile) {
     return precision == HIPCLAW_FP64 ? d->launch_fp64 != nullptr : d->launch_fp32 != nullptr;
 }
 
-// Waves per workgroup of a solver's strips by default (a registered solver's keep
-// nothing in LDS).
-static int solver_strip_waves(int solver, int precision) {
-    using namespace hipclaw;
-    const bool fp64 = precision == HIPCLAW_FP64;
-    switch (solver) {
-    case 0: return fp64 ? strip_waves<RPAdvection<double>, double>() : strip_waves<RPAdvection<float>, float>();
-    case 1: return fp64 ? strip_waves<RPShallow<double>, double>() : strip_waves<RPShallow<float>, float>();
-    case 2: return fp64 ? strip_waves<RPEuler<double>, double>() : strip_waves<RPEuler<float>, float>();
-    default: return 4;
-    }
-}
-
 static int launch_solver_step(int solver, int precision, int tile, int waves,
                               const hipclaw::StepArgs& a, const hipclaw::StepLaunch& L) {
     if (solver >= 0 && solver <= 2)
@@ -1642,7 +1629,7 @@ static int effective_waves(const hipclaw_state_t* s) {
     if (s->waves) return s->waves;
     if (s->tile != 16) return 0;
     return steps_by_tiles(s, s->npatch) ? hipclaw::default_tile_waves(s->cfg.precision == HIPCLAW_FP64, 16)
-                                        : solver_strip_waves(s->cfg.solver, s->cfg.precision);
+                                        : hipclaw::STRIP_WAVES;
 }
 
 int hipclaw_set_waves(hipclaw_state_t* s, int waves) {
@@ -1701,7 +1688,7 @@ int hipclaw_autotune(hipclaw_state_t* s, double dt, int nsteps, int* tiles, int*
             for (int l = 0; l <= s->lmax - s->lmin; l++) tiles = tiles || steps_by_tiles(s, s->loff[l + 1] - s->loff[l]);
         else
             tiles = s->inplace || steps_by_tiles(s, s->npatch);
-        return tiles ? 0 : s->waves ? s->waves : solver_strip_waves(s->cfg.solver, s->cfg.precision);
+        return tiles ? 0 : s->waves ? s->waves : hipclaw::STRIP_WAVES;
     };
     for (int t : candidates) {
         if (!tile_allowed(s, t)) continue;

@@ -178,15 +178,15 @@ inline int launch_step_strips(int nw, const StepArgs& a, const StepLaunch& st) {
 // Waves per workgroup by default.  Strips: four, which share nothing but lie on the
 // four SIMDs of one CU, beside each other in its cache (one and four, subcycled dam
 // break FP64 9.80 and 9.62 ms, dam break FP64 22.53 and 22.46, shock-bubble FP32
-// 5.20 and 5.16, advection 567 and 565 us; three leave a SIMD of every CU idle); one
-// for the kernels that keep values in LDS, which a workgroup holds until its last wave
-// ends.
+// 5.20 and 5.16, advection 567 and 565 us; three leave a SIMD of every CU idle).  Single
+// waves may also come two to a SIMD beside an idle one when a launch meets an idle
+// device: Euler FP64 on 134 patches of 61 x 61, 960 waves, 97 us alone and 71 among
+// other steps with one wave, 68 and 71 with four.
 // 16 x 16 tiles: four for FP64, two for the FP32-bulk form (a sweep's 18 rows, three
 // per wave, are three groups for each of two waves, where four take two, two, one
 // and one and wait at the barrier; FP64 tiles need the latency hiding of four).
 // hipclaw_set_waves and the autotuner choose 2, 3 or 4.
-template <class RP, typename R>
-constexpr int strip_waves() { return strip_carry<RP, R>() ? 1 : 4; }
+constexpr int STRIP_WAVES = 4;
 constexpr int default_tile_waves(bool fp64, int tile) { return tile != 16 ? 0 : fp64 ? 4 : 2; }   // (0: one choice)
 
 // Whether the tile kernel is instantiated for a tile (T = 32 only WITH32).
@@ -230,7 +230,7 @@ inline int launch_step_tile(int tile, int waves, const StepArgs& a, const StepLa
     if constexpr (uses_strips<RP>()) {
         if ((waves > 0 && a.qsrc != a.qdst) || !has_tile<RP, R, WITH_REGS, WITH32>(tile, a.reg != nullptr) ||
             !launches_tiles(a, tile, RP::MEQN * RP::MWAVES * (int) sizeof(R), device_simds()))
-            return launch_step_strips<RP, R, WITH_REGS>(waves > 0 ? waves : strip_waves<RP, R>(), a, st);
+            return launch_step_strips<RP, R, WITH_REGS>(waves > 0 ? waves : STRIP_WAVES, a, st);
     }
     return launch_step_tiles<RP, R, WITH_REGS, WITH32>(tile, waves, a, st);
 }

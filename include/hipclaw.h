@@ -302,8 +302,7 @@ int hipclaw_set_ghost_layout(hipclaw_state_t *s, int layout);
 int hipclaw_ghost_layout(const hipclaw_state_t *s);
 
 /* Waves per workgroup of the update, for the 16 x 16 tile: 2, 3 or 4 (0 = the
- * default).  Strips take 4 by default, or 1 where they keep values in LDS
- * (shallow water FP32-bulk, Euler FP64); tiles 4, or 2 in the FP32-bulk form.
+ * default).  Strips take 4 by default; tiles 4, or 2 in the FP32-bulk form.
  * Small launches of the solvers that use strips go to the tile kernel by default;
  * a choice of waves keeps them in strips, except those in place.
  * hipclaw_waves returns the waves the next update of all patches uses (0 for tiles without

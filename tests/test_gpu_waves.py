@@ -10,8 +10,7 @@ from helpers import setup_problem
 
 pytestmark = pytest.mark.gpu
 
-# by solver and form: strips' waves (1 where they keep values in LDS)
-STRIPS = {("swe", fa.FP64): 4, ("swe", fa.FP32_BULK): 1, ("euler", fa.FP64): 1, ("euler", fa.FP32_BULK): 4}
+STRIPS = 4     # strips' waves by default
 
 
 def _setup(name, precision, minlevel, **kw):
@@ -25,7 +24,7 @@ def _setup(name, precision, minlevel, **kw):
 def test_waves_by_default_and_by_choice(gpu, name, precision):
     prob, (forest, q0, _, sv) = _setup(name, precision, 5)
     assert forest.npatch == 1024
-    assert sv.waves == STRIPS[name, precision]
+    assert sv.waves == STRIPS
     dt = 0.5 * P.stable_dt(prob, forest, q0)
     sv.advance(dt, 4)
     want = sv.get_q()
@@ -37,10 +36,10 @@ def test_waves_by_default_and_by_choice(gpu, name, precision):
         sv.advance(dt, 4)
         np.testing.assert_array_equal(sv.get_q(), want)
     sv.set_waves(0)
-    assert sv.waves == STRIPS[name, precision]
-    # a small launch: FP64 takes 16 x 16 tiles with four waves
+    assert sv.waves == STRIPS
+    # a small launch: FP64 takes 16 x 16 tiles with four waves, FP32-bulk stays in strips
     _, (_, _, _, small) = _setup(name, precision, 2)
-    assert small.waves == (4 if precision == fa.FP64 else STRIPS[name, precision])
+    assert small.waves == 4
 
 
 @pytest.mark.parametrize("name,precision", [("swe", fa.FP64), ("swe", fa.FP32_BULK)])
@@ -49,7 +48,7 @@ def test_autotune_times_the_same_launches_once(gpu, name, precision):
     timings = sv.autotune(0.5 * P.stable_dt(prob, forest, q0), 2)
     assert set(timings) == {(t, w, l) for t, w in ((8, 0), (16, 2), (16, 3), (16, 4)) for l in (0, 1, 2)}
     assert (sv.tile, sv.waves, sv.ghost_layout) == min(timings, key=timings.get)
-    if STRIPS[name, precision] == 4:     # an 8 x 8 tile's strips are those of the 16 x 16 tile with four waves
-        for layout in (0, 1, 2):
-            assert timings[8, 0, layout] == timings[16, 4, layout]
-        assert sv.tile == 16
+    # an 8 x 8 tile's strips are those of the 16 x 16 tile with four waves
+    for layout in (0, 1, 2):
+        assert timings[8, 0, layout] == timings[16, 4, layout]
+    assert sv.tile == 16
