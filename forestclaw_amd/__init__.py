@@ -457,8 +457,8 @@ class Solver:
     def autotune(self, dt, nsteps=8):
         """Time every allowed tile (16 x 16 with 2, 3 and 4 waves) in every
         ghost-fill layout over nsteps steps of dt (the state is put back
-        after each) and keep the fastest; returns
-        {(tile, waves, layout): ms per step}."""
+        after each; trials with the same launches share one timing) and keep
+        the fastest; returns {(tile, waves, layout): ms per step}."""
         tiles = np.zeros(AUTOTUNE_MAX_TRIALS, np.int32)
         waves = np.zeros(AUTOTUNE_MAX_TRIALS, np.int32)
         layouts = np.zeros(AUTOTUNE_MAX_TRIALS, np.int32)

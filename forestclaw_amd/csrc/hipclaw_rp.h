@@ -156,7 +156,8 @@ __device__ __forceinline__ void quotients(const double (&n)[N], double b, bool f
 }
 // The correctly rounded square root of a number between 2^-900 and 2^900
 // (Goldschmidt's iteration from the hardware estimate, then two corrections by
-// the exact residual): 26 ns where the general one takes 39.
+// the exact residual; P. Markstein, "Software division and square root using
+// Goldschmidt's algorithms", RNC6, 2004): 26 ns where the general one takes 39.
 __device__ __forceinline__ double fast_root(double x) {
     const double y = __builtin_amdgcn_rsq(x);
     double g = x * y, h = 0.5 * y;

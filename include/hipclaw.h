@@ -61,8 +61,8 @@ typedef struct hipclaw_config {
                         default.  Solvers with meqn x mwaves > 16 are updated tile by
                         tile (a tile that does not divide the patch overlaps its last
                         tile with the one before), the others in strips laid out by
-                        the patch size; for them the tile only says whether one
-                        covers a patch */
+                        the patch size; for them the tile says whether one covers
+                        a patch, and what small launches are updated in */
     int time_sync;   /* keep flux registers for the conservation fix-up
                         (fclaw_options time-sync, src/fclaw_options.c:110); needs mx == my */
     int subcycle;    /* keep the state before each update and time-interpolated
@@ -276,11 +276,12 @@ int hipclaw_set_dt_scale(hipclaw_state_t *s, const double *scale);
  * for all patches at once, as save_time_step / restore_time_step of the run
  * loop use them to reject a step whose Courant number exceeds max_cfl
  * (src/fclaw2d_run.c:47-80).  Restoring without a saved state, or after a
- * regrid (the slots changed), is an error.  With two slabs the saved state stays in its slab without a copy while
- * only a one-step advance runs (it writes the other slab); any other call
- * that may write that slab copies it first.  A restore may so make the
- * other slab current: a graph captured before then refuses to replay, or, where
- * a tile covers a patch, first copies the state to the slab it starts from. */
+ * regrid (the slots changed), is an error.  With two slabs the saved state stays
+ * in its slab without a copy while only a one-step advance runs (it writes the
+ * other slab); any other call that may write that slab copies it first.  A
+ * restore may so make the other slab current: a graph captured before then
+ * refuses to replay, or, where a tile covers a patch, first copies the state to
+ * the slab it starts from. */
 int hipclaw_save_step(hipclaw_state_t *s);
 int hipclaw_restore_step(hipclaw_state_t *s);
 
@@ -305,8 +306,9 @@ int hipclaw_ghost_layout(const hipclaw_state_t *s);
  * default).  Strips take 4 by default; tiles 4, or 2 in the FP32-bulk form.
  * Small launches of the solvers that use strips go to the tile kernel by default;
  * a choice of waves keeps them in strips, except those in place.
- * hipclaw_waves returns the waves the next update of all patches uses (0 for tiles without
- * a choice).  No counterpart in the reference (128 threads per patch). */
+ * hipclaw_waves returns the waves the next update of all patches uses (0 for
+ * tiles without a choice).  No counterpart in the reference (128 threads per
+ * patch). */
 int hipclaw_set_waves(hipclaw_state_t *s, int waves);
 int hipclaw_waves(const hipclaw_state_t *s);
 
@@ -318,7 +320,8 @@ int hipclaw_waves(const hipclaw_state_t *s);
  * patch size allow, with 2, 3 and 4 waves per workgroup for 16 x 16 tiles, in
  * every ghost-fill layout the program allows, each trial from the state saved
  * at entry and restored after it (the saved state of hipclaw_save_step is
- * overwritten), and keep the fastest.  tiles[k], waves[k], layouts[k], ms[k]
+ * overwritten), and keep the fastest.  Trials that launch the same kernels the
+ * same way are timed once and share the time.  tiles[k], waves[k], layouts[k], ms[k]
  * (room for HIPCLAW_AUTOTUNE_MAX_TRIALS)
  * receive each trial and its mean step time, *ntrials their count.  A
  * subcycling state (levels set) is timed on subcycled coarse steps.  No
@@ -355,10 +358,12 @@ int hipclaw_sync(hipclaw_state_t *s);
 
 /* Capture nsteps of hipclaw_advance_async in a HIP graph (replaces any graph
  * captured before) and replay it.  The graph starts from the slab current at
- * its capture; a replay when the other slab is current (after an odd number
- * of steps, or a restore) is refused with HIPCLAW_EINVAL.  Installing a ghost
- * or sync program, the levels, or geometry for another number of patches
- * drops the graph (its launches hold the old tables and counts). */
+ * its capture and ends in it: with two slabs nsteps is even, or a tile covers a
+ * patch.  A replay when the other slab is current (after an odd number of steps,
+ * or a restore) is refused with HIPCLAW_EINVAL, or, where a tile covers a patch,
+ * copies the state over first.  Installing a ghost or sync program, the levels,
+ * or geometry for another number of patches drops the graph (its launches hold
+ * the old tables and counts). */
 int hipclaw_capture_graph(hipclaw_state_t *s, double dt, int nsteps);
 int hipclaw_replay_graph(hipclaw_state_t *s);
 
