@@ -1626,10 +1626,10 @@ static bool steps_by_tiles(const hipclaw_state_t* s, int n) {
 }
 
 static int effective_waves(const hipclaw_state_t* s) {
-    if (s->waves) return s->waves;
+    if (!steps_by_tiles(s, s->npatch)) return s->waves ? s->waves : s->tile == 16 ? hipclaw::STRIP_WAVES : 0;
     if (s->tile != 16) return 0;
-    return steps_by_tiles(s, s->npatch) ? hipclaw::default_tile_waves(s->cfg.precision == HIPCLAW_FP64, 16)
-                                        : hipclaw::STRIP_WAVES;
+    const bool choice = s->cfg.meqn * s->cfg.mwaves > 16;   // (one shape where strips are the larger launches' kernel)
+    return choice && s->waves ? s->waves : hipclaw::default_tile_waves(s->cfg.precision == HIPCLAW_FP64, 16);
 }
 
 int hipclaw_set_waves(hipclaw_state_t* s, int waves) {
@@ -1694,9 +1694,17 @@ int hipclaw_autotune(hipclaw_state_t* s, double dt, int nsteps, int* tiles, int*
         if (!tile_allowed(s, t)) continue;
         const int nlay = s->fused_ok ? 3 : 2;
         for (int trial = 0; trial < (t == 16 ? 3 * nlay : nlay) && !rc; trial++) {
-            const int lay = trial % nlay, w = t == 16 ? 2 + trial / nlay : 0;
+            // Two, three and four waves for 16 x 16 tiles.  The strips' four are the
+            // default, which leaves small launches to the tile kernel: a chosen four
+            // would keep them out of the trials (Euler FP64, 250 patches of 16 x 16,
+            // tiles 16.8 us, strips 24.5).
+            int w = t == 16 ? 2 + trial / nlay : 0;
+            const int lay = trial % nlay;
+            const bool by_strips = s->cfg.meqn * s->cfg.mwaves <= 16;
+            if (w == 4 && by_strips) w = 0;
             if ((rc = set_tile(s, t)) || (rc = hipclaw_set_ghost_layout(s, lay)) || (rc = hipclaw_set_waves(s, w)))
                 break;
+            if (w && by_strips && steps_by_tiles(s, s->npatch)) continue;   // (in place: the tiles have one shape)
             const int sw = strips();
             const auto known = std::find_if(timed.begin(), timed.end(),
                                             [&](const Timed& k) { return sw && k.strip_waves == sw && k.layout == lay; });

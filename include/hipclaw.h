@@ -317,7 +317,8 @@ int hipclaw_waves(const hipclaw_state_t *s);
 
 /* Autotuner: time nsteps full steps (update, ghost fill, time sync) of dt on
  * the current patches for every tile size the state's solver, precision and
- * patch size allow, with 2, 3 and 4 waves per workgroup for 16 x 16 tiles, in
+ * patch size allow, with 2, 3 and 4 waves per workgroup for 16 x 16 tiles (of
+ * strips the four are the default, small launches in tiles included), in
  * every ghost-fill layout the program allows, each trial from the state saved
  * at entry and restored after it (the saved state of hipclaw_save_step is
  * overwritten), and keep the fastest.  Trials that launch the same kernels the

@@ -52,3 +52,16 @@ def test_autotune_times_the_same_launches_once(gpu, name, precision):
     for layout in (0, 1, 2):
         assert timings[8, 0, layout] == timings[16, 4, layout]
     assert sv.tile == 16
+
+
+@pytest.mark.parametrize("name", ["swe", "euler"])
+def test_autotune_tries_the_tile_kernel_for_small_launches(gpu, name):
+    """The trial of a 16 x 16 tile with four waves, the default, is the tile kernel where
+    the default takes it; chosen waves are strips.  A step of tiles takes 0.83 (shallow
+    water) and 0.78 (Euler) of the time of one of strips with three waves, strips with
+    four 0.99."""
+    prob, (forest, q0, _, sv) = _setup(name, fa.FP64, 4)
+    assert forest.npatch == 256
+    timings = sv.autotune(0.5 * P.stable_dt(prob, forest, q0), 16)
+    print(name, timings, "tile", sv.tile, "waves", sv.waves, "layout", sv.ghost_layout, flush=True)
+    assert timings[16, 4, 2] <= 0.92 * timings[16, 3, 2]
